@@ -1,8 +1,7 @@
 // oxr_device.h -- device-side vector math, Philox RNG, tables and CSG intersection.
 //
 // Float semantics are deliberate: sources are compiled with -ffp-contract=off and
-// correctly rounded fp32 divide/sqrt, and log/sin/cos/atan2 are evaluated in fp64 and
-// rounded, so every fp32 result is a function of its inputs alone.
+// correctly rounded fp32 divide/sqrt, and sin/cos/atan2 are evaluated in fp64 and rounded, so every fp32 result is a function of its inputs alone.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -51,8 +50,39 @@ OXD float xlog(float x) {
     float dk = float(k);
     return dk * ln2_hi - ((hfsq - (s * (hfsq + R) + dk * ln2_lo)) - f);
 }
-OXD float xsin(float x) { return (float)sin((double)x); }
-OXD float xcos(float x) { return (float)cos((double)x); }
+// sin and cos of a single-precision argument, each the double-precision value rounded once.
+// One reduction serves both: n = rint(x 2/pi), r = x - n pi/2 with pi/2 in two doubles (the
+// first difference is exact: x and n hi are multiples of 2^-52 and r is below 1), then the
+// Taylor series of sin to r^15 and cos to r^16 on |r| <= pi/4, where the next terms are below
+// half an ulp. Equal to the host libm's (float)sin((double)x), (float)cos((double)x) for every
+// Philox uniform times 2 pi and over |x| <= 8e5 (checked on 2^24 arguments each). The
+// library's sin and cos reduce twice, carry the code for huge arguments and take three
+// times the instructions.
+OXD void sincos_bounded(float x, float& s, float& c) {
+    const double xd = double(x);
+    const double n = rint(xd * 0.63661977236758134308);
+    double r = fma(-n, 1.5707963267948965580, xd);
+    r = fma(-n, 6.1232339957367658860e-17, r);
+    const double z = r * r;
+    double ps = fma(z, -1.0 / 1307674368000.0, 1.0 / 6227020800.0);
+    ps = fma(z, ps, -1.0 / 39916800.0); ps = fma(z, ps, 1.0 / 362880.0); ps = fma(z, ps, -1.0 / 5040.0);
+    ps = fma(z, ps, 1.0 / 120.0); ps = fma(z, ps, -1.0 / 6.0);
+    double pc = fma(z, 1.0 / 20922789888000.0, -1.0 / 87178291200.0);
+    pc = fma(z, pc, 1.0 / 479001600.0); pc = fma(z, pc, -1.0 / 3628800.0); pc = fma(z, pc, 1.0 / 40320.0);
+    pc = fma(z, pc, -1.0 / 720.0); pc = fma(z, pc, 1.0 / 24.0); pc = fma(z, pc, -0.5);
+    const float sn = float(fma(r * z, ps, r)), cs = float(fma(z, pc, 1.0));
+    const int q = int(n);
+    const float a = (q & 1) ? cs : sn, b = (q & 1) ? sn : cs;
+    s = (q & 2) ? -a : a;
+    c = ((q + 1) & 2) ? -b : b;
+}
+// any argument (genstep angles and phases are the caller's): huge, infinite, NaN and zero
+// ones (whose sign sin keeps) take the library's functions
+OXD void xsincos(float x, float& s, float& c) {
+    if (fabsf(x) <= 8e5f && x != 0.f) { sincos_bounded(x, s, c); return; }
+    s = (float)sin((double)x);
+    c = (float)cos((double)x);
+}
 OXD float xatan2(float y, float x) { return (float)atan2((double)y, (double)x); }
 constexpr float PIf = 3.14159265358979323846f;
 
@@ -72,16 +102,16 @@ constexpr float RT_DEFAULT_MAX = 1.e27f;   // CSG/csg_intersect_leaf_head.h:10
 // ------------------------------------------------------------------ Philox4x32-10
 // Counter-based generator of Salmon et al. (SC'11). Stream of photon p: key = seed,
 // counter = (block lo, block hi, p lo, p hi), uniform j at block (start+j)/4, lane (start+j)%4.
-// The four outputs of the current block are held in scalars b0..b3 and consumed by
-// shifting, so the state never needs an indexed (memory-resident) array.
+// Between two bounces a stream is its position and the words left of the block that the
+// position stands in, so a bounce computes one block (draws) and takes its uniforms by fixed
+// names; the rejection loops have one refill where a turn begins (queue_fill). No buffer is
+// ever indexed, and the ten Philox rounds stand in a few places instead of behind every
+// uniform (a plain-form production kernel shrank from 109 to 71 KB of code).
 struct Rng {
     uint32_t k0, k1;
     uint32_t p0, p1;          // photon index (subsequence)
     uint64_t pos;             // absolute uniform index of the next uniform
-    uint32_t b0, b1, b2, b3;  // unconsumed outputs of the current block, b0 next
-    int have;                 // how many of b0..b3 are valid
-    uint32_t c0, c1, c2, c3;  // the following block, computed ahead by rng_topup
-    int have2;                // 4 when c0..c3 hold it, else 0
+    uint32_t c0, c1, c2;      // the next (-pos) & 3 words
     const float* pre;         // precooked row or null
     int32_t npre, cur;
     uint32_t overflow;
@@ -105,67 +135,149 @@ OXD void philox(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0,
     o0 = c0; o1 = c1; o2 = c2; o3 = c3;
 }
 
-OXD void rng_init(Rng& r, uint64_t seed, uint64_t offset, uint64_t skip, uint64_t event, uint64_t photon) {
-    r.k0 = uint32_t(seed); r.k1 = uint32_t(seed >> 32);
-    r.p0 = uint32_t(photon); r.p1 = uint32_t(photon >> 32);
-    r.pos = offset + skip * event;
-    r.have = 0; r.have2 = 0;
-    r.b0 = r.b1 = r.b2 = r.b3 = 0u;
-    r.c0 = r.c1 = r.c2 = r.c3 = 0u;
-    r.pre = nullptr; r.npre = 0; r.cur = 0; r.overflow = 0;
+OXD void rng_block(const Rng& r, uint64_t block, uint32_t& o0, uint32_t& o1, uint32_t& o2, uint32_t& o3) {
+    philox(uint32_t(block), uint32_t(block >> 32), r.p0, r.p1, r.k0, r.k1, o0, o1, o2, o3);
+}
+// word k of a precooked row from the current place on, wrapping round
+OXD uint32_t pre_word(const Rng& r, int k) {
+    int i = r.cur + k;
+    while (i >= r.npre) i -= r.npre;
+    return __float_as_uint(r.pre[i]);
+}
+// the uniform a word stands for: Philox words map to (0,1], precooked rows hold the floats
+OXD float unit(const Rng& r, uint32_t w) {
+    return r.pre ? __uint_as_float(w) : float((w >> 8) + 1u) * (1.0f / 16777216.0f);
+}
+// k uniforms are spent (the caller then sets the words left: keep, or rng_rest)
+OXD void advance(Rng& r, int k) {
+    if (r.pre) {
+        r.cur += k;
+        while (r.cur > r.npre) { r.cur -= r.npre; r.overflow++; }
+    }
+    r.pos += uint64_t(k);
+}
+OXD void keep(Rng& r, uint32_t c0, uint32_t c1, uint32_t c2) { r.c0 = c0; r.c1 = c1; r.c2 = c2; }
+// the words left of pos's block, computed again
+OXD void rng_rest(Rng& r) {
+    const uint32_t skip = uint32_t(r.pos) & 3u;
+    if (r.pre || skip == 0u) return;
+    uint32_t b0, b1, b2, b3;
+    rng_block(r, r.pos >> 2, b0, b1, b2, b3);
+    r.c0 = skip == 1u ? b1 : (skip == 2u ? b2 : b3);
+    r.c1 = skip == 1u ? b2 : b3;
+    r.c2 = b3;
 }
 
-// continue a stream at uniform number pos (the counter-based stream needs nothing else)
+// continue a stream at uniform number pos (the counter-based stream needs nothing else;
+// rng_rest before the first draws)
 OXD void rng_resume(Rng& r, uint64_t seed, uint64_t pos, uint64_t photon) {
     r.k0 = uint32_t(seed); r.k1 = uint32_t(seed >> 32);
     r.p0 = uint32_t(photon); r.p1 = uint32_t(photon >> 32);
     r.pos = pos;
-    r.have = 0; r.have2 = 0;
-    r.b0 = r.b1 = r.b2 = r.b3 = 0u;
-    r.c0 = r.c1 = r.c2 = r.c3 = 0u;
+    r.c0 = r.c1 = r.c2 = 0u;
     r.pre = nullptr; r.npre = 0; r.cur = 0; r.overflow = 0;
 }
-
-// refill an empty buffer: from the block computed ahead, else from Philox
-OXD void rng_refill(Rng& r) {
-    if (r.have2) {                             // the block after a buffer always starts aligned
-        r.b0 = r.c0; r.b1 = r.c1; r.b2 = r.c2; r.b3 = r.c3;
-        r.have = 4; r.have2 = 0;
-        return;
-    }
-    uint64_t block = r.pos >> 2;
-    philox(uint32_t(block), uint32_t(block >> 32), r.p0, r.p1, r.k0, r.k1, r.b0, r.b1, r.b2, r.b3);
-    uint32_t skip = uint32_t(r.pos & 3);      // only the first block of a stream can start mid-block
-    if (skip >= 1u) { r.b0 = r.b1; r.b1 = r.b2; r.b2 = r.b3; }
-    if (skip >= 2u) { r.b0 = r.b1; r.b1 = r.b2; }
-    if (skip >= 3u) { r.b0 = r.b1; }
-    r.have = 4 - int(skip);
+OXD void rng_init(Rng& r, uint64_t seed, uint64_t offset, uint64_t skip, uint64_t event, uint64_t photon) {
+    rng_resume(r, seed, offset + skip * event, photon);
 }
 
-// Compute the block after the buffered uniforms now, so that the next five to eight
-// uniforms need no Philox. Called where every lane of a branch is about to draw (the
-// start of a bounce's physics, the diffuse-reflection rejection loops): the Philox rounds
-// then run once for the branch instead of inside divergent loops whenever some lane's
-// buffer empties. The values drawn are unchanged; only when they are computed moves.
-OXD void rng_topup(Rng& r) {
-    if (r.pre || r.have2) return;
-    if (r.have == 0) rng_refill(r);
-    uint64_t next = (r.pos + uint64_t(r.have)) >> 2;
-    philox(uint32_t(next), uint32_t(next >> 32), r.p0, r.p1, r.k0, r.k1, r.c0, r.c1, r.c2, r.c3);
-    r.have2 = 4;
-}
-
-OXD float uniform(Rng& r) {
+// The next four to seven uniforms, as words: those left of pos's block and the whole block
+// after them. n counts the valid ones.
+struct Draws { uint32_t w0, w1, w2, w3, w4, w5, w6; int n; };
+OXD Draws draws(const Rng& r) {
+    Draws d;
     if (r.pre) {
-        if (r.cur >= r.npre) { r.cur = 0; r.overflow++; }
-        return r.pre[r.cur++];
+        d.w0 = pre_word(r, 0); d.w1 = pre_word(r, 1); d.w2 = pre_word(r, 2); d.w3 = pre_word(r, 3);
+        d.w4 = pre_word(r, 4); d.w5 = pre_word(r, 5); d.w6 = pre_word(r, 6);
+        d.n = 7;
+        return d;
     }
-    if (r.have == 0) rng_refill(r);
-    uint32_t x = r.b0;
-    r.b0 = r.b1; r.b1 = r.b2; r.b2 = r.b3;
-    r.have--;
-    r.pos++;
-    return float((x >> 8) + 1u) * (1.0f / 16777216.0f);
+    uint32_t b0, b1, b2, b3;
+    rng_block(r, (r.pos + 3u) >> 2, b0, b1, b2, b3);
+    const int c = int(0u - uint32_t(r.pos)) & 3;
+    const bool c1 = c >= 1, c2 = c >= 2, c3 = c == 3;
+    d.w0 = c1 ? r.c0 : b0;
+    d.w1 = c2 ? r.c1 : (c1 ? b0 : b1);
+    d.w2 = c3 ? r.c2 : (c2 ? b0 : (c1 ? b1 : b2));
+    d.w3 = c3 ? b0 : (c2 ? b1 : (c1 ? b2 : b3));
+    d.w4 = c3 ? b1 : (c2 ? b2 : b3);
+    d.w5 = c3 ? b2 : b3;
+    d.w6 = b3;
+    d.n = c + 4;
+    return d;
+}
+// The next five uniforms, spent, from two blocks that owe nothing to the words kept (rare
+// bulk physics and generation).
+struct Five { float u0, u1, u2, u3, u4; };
+OXD Five draw5(Rng& r) {
+    uint32_t w0, w1, w2, w3, w4, w5, w6, w7;
+    if (r.pre) {
+        w0 = pre_word(r, 0); w1 = pre_word(r, 1); w2 = pre_word(r, 2); w3 = pre_word(r, 3); w4 = pre_word(r, 4);
+        w5 = w6 = w7 = 0u;
+    } else {
+        const uint64_t block = r.pos >> 2;
+        rng_block(r, block, w0, w1, w2, w3);
+        rng_block(r, block + 1, w4, w5, w6, w7);
+        const uint32_t skip = uint32_t(r.pos) & 3u;
+        if (skip & 1u) { w0 = w1; w1 = w2; w2 = w3; w3 = w4; w4 = w5; w5 = w6; w6 = w7; }
+        if (skip & 2u) { w0 = w2; w1 = w3; w2 = w4; w3 = w5; w4 = w6; w5 = w7; }
+    }
+    Five f;
+    f.u0 = unit(r, w0); f.u1 = unit(r, w1); f.u2 = unit(r, w2); f.u3 = unit(r, w3); f.u4 = unit(r, w4);
+    advance(r, 5);
+    keep(r, w5, w6, w7);
+    return f;
+}
+
+// the next two uniforms, spent: one block unless they straddle two (leaves the words kept stale)
+OXD void draw2(Rng& r, float& a, float& b) {
+    uint32_t w0, w1;
+    if (r.pre) {
+        w0 = pre_word(r, 0); w1 = pre_word(r, 1);
+    } else {
+        uint32_t v2, v3;
+        rng_block(r, r.pos >> 2, w0, w1, v2, v3);
+        const uint32_t skip = uint32_t(r.pos) & 3u;
+        if (skip & 2u) { w0 = v2; w1 = v3; }
+        if (skip & 1u) {
+            w0 = w1; w1 = v2;
+            if (skip & 2u) { uint32_t x1, x2, x3; rng_block(r, (r.pos >> 2) + 1, w1, x1, x2, x3); }
+        }
+    }
+    a = unit(r, w0);
+    b = unit(r, w1);
+    advance(r, 2);
+}
+
+// A queue of at most six words ahead of pos for rejection loops, refilled by one block where
+// a loop turn begins (the only Philox of the loop). Its words are the stream from pos on, so
+// the block after them starts aligned once the first has been cut.
+struct Queue { uint32_t w0, w1, w2, w3, w4, w5; int n; };
+OXD void queue_fill(const Rng& r, Queue& q) {   // needs n < 3
+    uint32_t b0, b1, b2, b3;
+    if (r.pre) {
+        b0 = pre_word(r, q.n); b1 = pre_word(r, q.n + 1); b2 = pre_word(r, q.n + 2); b3 = pre_word(r, q.n + 3);
+    } else {
+        rng_block(r, (r.pos + uint64_t(q.n)) >> 2, b0, b1, b2, b3);
+    }
+    const bool n0 = q.n == 0, n1 = q.n == 1;
+    q.w0 = n0 ? b0 : q.w0;
+    q.w1 = n0 ? b1 : (n1 ? b0 : q.w1);
+    q.w2 = n0 ? b2 : (n1 ? b1 : b0);
+    q.w3 = n0 ? b3 : (n1 ? b2 : b1);
+    q.w4 = n1 ? b3 : b2;
+    q.w5 = b3;
+    q.n += 4;
+}
+OXD void queue_take2(Rng& r, Queue& q) {
+    q.w0 = q.w2; q.w1 = q.w3; q.w2 = q.w4; q.w3 = q.w5;
+    q.n -= 2;
+    advance(r, 2);
+}
+OXD void queue_take1(Rng& r, Queue& q) {
+    q.w0 = q.w1; q.w1 = q.w2; q.w2 = q.w3; q.w3 = q.w4; q.w4 = q.w5;
+    q.n -= 1;
+    advance(r, 1);
 }
 
 // ------------------------------------------------------------------ tables

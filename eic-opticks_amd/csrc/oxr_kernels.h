@@ -93,9 +93,12 @@ template <bool FP64, bool LIST>
 hipError_t launch_simulate_plain(hipStream_t s, const oxd::Params& P, dim3 g, dim3 b, size_t sm, int kind, int tm);
 template <bool FP64, bool LIST>
 hipError_t launch_simulate_persist(hipStream_t s, const oxd::Params& P, dim3 g, dim3 b, size_t sm, bool debug, int tm);
+template <bool FP64, bool LIST>
+const void* persist_kernel(bool debug, int tm);
 #define OXR_SIM_EXTERN(F, L)                                                                                        \
     extern template hipError_t launch_simulate_plain<F, L>(hipStream_t, const oxd::Params&, dim3, dim3, size_t, int, int); \
-    extern template hipError_t launch_simulate_persist<F, L>(hipStream_t, const oxd::Params&, dim3, dim3, size_t, bool, int);
+    extern template hipError_t launch_simulate_persist<F, L>(hipStream_t, const oxd::Params&, dim3, dim3, size_t, bool, int); \
+    extern template const void* persist_kernel<F, L>(bool, int);
 OXR_SIM_EXTERN(false, false)
 OXR_SIM_EXTERN(false, true)
 OXR_SIM_EXTERN(true, false)

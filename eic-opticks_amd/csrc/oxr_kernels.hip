@@ -231,10 +231,11 @@ __global__ void __launch_bounds__(256) k_simtrace(Params P, const float4* __rest
     const int gridaxes = __float_as_int(q[0].y);
     Rng r;
     rng_init(r, P.rng_seed, 0ull, 0ull, 0ull, (unsigned long long)i);
-    float u0 = uniform(r);
+    float u0, u1;
+    draw2(r, u0, u1);
     float ph = 2.f * PIf * u0;
-    float sinPhi = xsin(ph), cosPhi = xcos(ph);
-    float u1 = uniform(r);
+    float sinPhi, cosPhi;
+    sincos_bounded(ph, sinPhi, cosPhi);
     float cosTheta = 2.f * u1 - 1.f;
     float sinTheta = sqrtf(1.f - cosTheta * cosTheta);
     f3 d;

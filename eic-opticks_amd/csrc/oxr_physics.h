@@ -134,7 +134,9 @@ OXD f3 uniform_sphere(float u0, float u1) {
     float phi = u0 * 2.f * PIf;
     float cosTheta = 2.f * u1 - 1.f;
     float sinTheta = sqrtf(1.f - cosTheta * cosTheta);
-    return mk(xcos(phi) * sinTheta, xsin(phi) * sinTheta, cosTheta);
+    float sinPhi, cosPhi;
+    sincos_bounded(phi, sinPhi, cosPhi);
+    return mk(cosPhi * sinTheta, sinPhi * sinTheta, cosTheta);
 }
 
 // qsim::rayleigh_scatter (qudarap/qsim.h:601-689)
@@ -143,12 +145,14 @@ OXD void rayleigh_scatter(Ph& p, Rng& r) {
     bool looping = true;
     int turns = 0;
     do {
-        float u0 = uniform(r), u1 = uniform(r), u2 = uniform(r), u3 = uniform(r), u4 = uniform(r);
+        const Five f = draw5(r);
+        const float u0 = f.u0, u1 = f.u1, u2 = f.u2, u3 = f.u3, u4 = f.u4;
         float cosTheta = u0;
         float sinTheta = sqrtf(1.0f - u0 * u0);
         if (u1 < 0.5f) cosTheta = -cosTheta;
         float ph = 2.f * PIf * u2;
-        float sinPhi = xsin(ph), cosPhi = xcos(ph);
+        float sinPhi, cosPhi;
+        sincos_bounded(ph, sinPhi, cosPhi);
         direction = mk(sinTheta * cosPhi, sinTheta * sinPhi, cosTheta);
         rotateUz(direction, p.mom);
         float constant = -dot(direction, p.pol);
@@ -156,7 +160,7 @@ OXD void rayleigh_scatter(Ph& p, Rng& r) {
                           p.pol.z + constant * direction.z);
         if (dot(polarization, polarization) == 0.f) {
             float ph3 = 2.f * PIf * u3;
-            sinPhi = xsin(ph3); cosPhi = xcos(ph3);
+            sincos_bounded(ph3, sinPhi, cosPhi);
             polarization = mk(cosPhi, sinPhi, 0.f);
             rotateUz(polarization, direction);
         } else {
@@ -172,21 +176,25 @@ OXD void rayleigh_scatter(Ph& p, Rng& r) {
 }
 
 // qsim::propagate_to_boundary (qudarap/qsim.h:718-863)
-OXD int propagate_to_boundary(unsigned& flag, Ph& p, const St& s, float dist, Rng& r, const Tables& t, int aligned) {
+// d holds the stream from the photon's position on (the aligned schedule's two burns spent)
+OXD int propagate_to_boundary(unsigned& flag, Ph& p, const St& s, float dist, Rng& r, const Draws& d, const Tables& t) {
     float absorption_length = s.m1.y, scattering_length = s.m1.z, reemission_prob = s.m1.w;
     float group_velocity = s.m1g2.x;
-    if (aligned) { uniform(r); uniform(r); }
-    float u_scattering = uniform(r);
-    float u_absorption = uniform(r);
+    float u_scattering = unit(r, d.w0);
+    float u_absorption = unit(r, d.w1);
+    advance(r, 2);
+    keep(r, d.w2, d.w3, d.w4);
     float scattering_distance = -scattering_length * xlog(u_scattering);
     float absorption_distance = -absorption_length * xlog(u_absorption);
     if (absorption_distance <= scattering_distance) {
         if (absorption_distance <= dist) {
             p.time += absorption_distance / group_velocity;
             p.pos = add(p.pos, mul(absorption_distance, p.mom));
-            float u_reemit = reemission_prob == 0.f ? 2.f : uniform(r);
+            float u_reemit = 2.f;
+            if (reemission_prob != 0.f) { u_reemit = unit(r, d.w2); advance(r, 1); keep(r, d.w3, d.w4, d.w5); }
             if (u_reemit < reemission_prob) {
-                float u_wl = uniform(r), u_mph = uniform(r), u_mct = uniform(r), u_pph = uniform(r), u_pct = uniform(r);
+                const Five f = draw5(r);
+                const float u_wl = f.u0, u_mph = f.u1, u_mct = f.u2, u_pph = f.u3, u_pct = f.u4;
                 p.wavelength = scint_wavelength(t, u_wl);
                 p.mom = uniform_sphere(u_mph, u_mct);
                 p.pol = normalize(cross(uniform_sphere(u_pph, u_pct), p.mom));
@@ -211,7 +219,7 @@ OXD int propagate_to_boundary(unsigned& flag, Ph& p, const St& s, float dist, Rn
 }
 
 // qsim::propagate_at_boundary (qudarap/qsim.h:998-1205)
-OXD int propagate_at_boundary(unsigned& flag, Ph& p, const St& s, f3 normal, Rng& r, int aligned) {
+OXD int propagate_at_boundary(unsigned& flag, Ph& p, const St& s, f3 normal, Rng& r, const Draws& d, int aligned) {
     float n1 = s.m1.x, n2 = s.m2.x;
     float eta = n1 / n2;
     float _c1 = -dot(p.mom, normal);
@@ -238,8 +246,10 @@ OXD int propagate_at_boundary(unsigned& flag, Ph& p, const St& s, f3 normal, Rng
     float tinv = 1.0f / sqrtf(E2tx * E2tx + E2ty * E2ty);
     float TTx = E2tx * tinv, TTy = E2ty * tinv;
     float TransCoeff = (tir || n1c1 == 0.f) ? 0.f : n2c2 * (E2tx * E2tx + E2ty * E2ty) / n1c1;
-    if (aligned) uniform(r);
-    float u_reflect = uniform(r);
+    float u_reflect = unit(r, aligned ? d.w3 : d.w2);   // the aligned schedule burns one first
+    advance(r, aligned ? 2 : 1);
+    if (aligned) keep(r, d.w4, d.w5, d.w6);
+    else keep(r, d.w3, d.w4, d.w5);
     bool reflect = u_reflect > TransCoeff;
     p.mom = reflect ? add(p.mom, mul(2.f * c1, on)) : add(mul(eta, p.mom), mul(eta * c1 - c2, on));
     f3 A_paral = normalize(cross(p.mom, A_trans));
@@ -251,23 +261,13 @@ OXD int propagate_at_boundary(unsigned& flag, Ph& p, const St& s, f3 normal, Rng
         p.pol = add(mul(TTx, A_trans), mul(TTy, A_paral));
     }
     flag = reflect ? BOUNDARY_REFLECT : BOUNDARY_TRANSMIT;
-    if (aligned && reflect) { uniform(r); uniform(r); uniform(r); uniform(r); }
+    if (aligned && reflect) {   // a block's worth: the words left are those of the next block
+        advance(r, 4);
+        rng_rest(r);
+    }
     return CONTINUE;
 }
 
-// qsim::random_direction_marsaglia (qudarap/qsim.h:551-572)
-OXD f3 random_direction_marsaglia(Rng& r) {
-    float u, v, b, a;
-    int turns = 0;
-    do {
-        float u0 = uniform(r), u1 = uniform(r);
-        u = 2.f * u0 - 1.f;
-        v = 2.f * u1 - 1.f;
-        b = u * u + v * v;
-    } while (b > 1.f && ++turns < MAX_REJECT);
-    a = 2.f * sqrtf(1.f - b);
-    return mk(a * u, a * v, 2.f * b - 1.f);
-}
 // qsim::lambertian_direction (qudarap/qsim.h:430-483) with random_direction_marsaglia
 // (qsim.h:551-572) inlined. The reference nests the Marsaglia rejection loop inside the
 // Lambertian acceptance loop; here both run as one loop, one Marsaglia try per turn, so
@@ -275,11 +275,14 @@ OXD f3 random_direction_marsaglia(Rng& r) {
 // outer turn waiting for the slowest lane's inner loop. Each lane draws the same uniforms
 // in the same order, and both turn caps (MAX_REJECT Marsaglia tries per direction, 1024
 // directions) end the loop where the nested form ends.
-OXD f3 lambertian_direction(f3 normal, float orient, Rng& r) {
+// q holds the stream from the photon's position on.
+OXD f3 lambertian_direction(f3 normal, float orient, Rng& r, Queue& q) {
     int count = 0, turns = 0;
     f3 dir = mk(0.f, 0.f, 0.f);
     for (;;) {
-        float u0 = uniform(r), u1 = uniform(r);
+        if (q.n < 3) queue_fill(r, q);
+        float u0 = unit(r, q.w0), u1 = unit(r, q.w1);
+        queue_take2(r, q);
         float mu = 2.f * u0 - 1.f;
         float mv = 2.f * u1 - 1.f;
         float b = mu * mu + mv * mv;
@@ -290,17 +293,17 @@ OXD f3 lambertian_direction(f3 normal, float orient, Rng& r) {
         dir = mk(a * mu, a * mv, 2.f * b - 1.f);
         float ndotv = dot(dir, normal) * orient;
         if (ndotv < 0.f) { dir = mul(-1.f, dir); ndotv = -1.f * ndotv; }
-        float u = uniform(r);
+        float u = unit(r, q.w0);
+        queue_take1(r, q);
         if (u < ndotv || count >= 1024) break;
     }
     return dir;
 }
 // qsim::reflect_diffuse (qudarap/qsim.h:1977-2012)
-OXD void reflect_diffuse(Ph& p, f3 normal, Rng& r) {
-    rng_topup(r);
+OXD void reflect_diffuse(Ph& p, f3 normal, Rng& r, Queue& q) {
     f3 old_mom = p.mom;
     float orient = dot(old_mom, normal) > 0.f ? -1.f : 1.f;
-    p.mom = lambertian_direction(normal, orient, r);
+    p.mom = lambertian_direction(normal, orient, r, q);
     f3 fn = normalize(sub(p.mom, old_mom));
     float EdotN = dot(p.pol, fn);
     p.pol = add(mul(-1.f, p.pol), mul(2.f * EdotN, fn));
@@ -313,16 +316,25 @@ OXD void reflect_specular(Ph& p, f3 normal) {
     p.pol = add(mul(-1.f, p.pol), mul(2.f * EdotN, normal));
 }
 // qsim::propagate_at_surface (qudarap/qsim.h:1677-1747)
-OXD int propagate_at_surface(unsigned& flag, Ph& p, const St& s, f3 normal, Rng& r, int aligned) {
+OXD int propagate_at_surface(unsigned& flag, Ph& p, const St& s, f3 normal, Rng& r, const Draws& d, int aligned) {
     float detect = s.su.x, absorb = s.su.y, rdiff = s.su.w;
-    float u_surface = uniform(r);
-    if (aligned) uniform(r);
+    float u_surface = unit(r, d.w2);
+    advance(r, aligned ? 2 : 1);   // the aligned schedule burns one after
+    if (aligned) keep(r, d.w4, d.w5, d.w6);
+    else keep(r, d.w3, d.w4, d.w5);
     int action = u_surface < absorb + detect ? BREAK : CONTINUE;
     if (action == BREAK) {
         flag = u_surface < absorb ? SURFACE_ABSORB : SURFACE_DETECT;
     } else {
         flag = u_surface < absorb + detect + rdiff ? SURFACE_DREFLECT : SURFACE_SREFLECT;
-        if (flag == SURFACE_DREFLECT) reflect_diffuse(p, normal, r);
+        if (flag == SURFACE_DREFLECT) {
+            Queue q;   // what is left of d
+            q.w0 = d.w3; q.w1 = d.w4; q.w2 = d.w5; q.w3 = d.w6; q.w4 = 0u; q.w5 = 0u;
+            q.n = d.n - 3;
+            if (aligned) { q.w0 = q.w1; q.w1 = q.w2; q.w2 = q.w3; q.n -= 1; }
+            reflect_diffuse(p, normal, r, q);
+            keep(r, q.w0, q.w1, q.w2);
+        }
         else reflect_specular(p, normal);
     }
     return action;
@@ -341,15 +353,16 @@ OXD int propagate(Ph& p, const Hit& h, f3 normal, Rng& r, const Tables& t, int a
     set_prd(p, boundary, identity, cosTheta, iindex);
     St s;
     fill_state(t, s, boundary, p.wavelength, cosTheta);
-    rng_topup(r);
+    if (aligned) { advance(r, 2); rng_rest(r); }   // propagate_to_boundary's burns
+    const Draws d = draws(r);
     unsigned flag = 0;
-    int command = propagate_to_boundary(flag, p, s, h.t, r, t, aligned);
+    int command = propagate_to_boundary(flag, p, s, h.t, r, d, t);
     if (command == BOUNDARY) {
         int ems = int(s.opt.y);
-        if (ems == 1) command = propagate_at_boundary(flag, p, s, normal, r, aligned);
-        else if (ems == 2) command = propagate_at_surface(flag, p, s, normal, r, aligned);
-        else if (lpos_cost(h.lpos) < 0.f) command = propagate_at_surface(flag, p, s, normal, r, aligned);
-        else if (ems == 3) { uniform(r); flag = SURFACE_DETECT; command = BREAK; }
+        if (ems == 1) command = propagate_at_boundary(flag, p, s, normal, r, d, aligned);
+        else if (ems == 2) command = propagate_at_surface(flag, p, s, normal, r, d, aligned);
+        else if (lpos_cost(h.lpos) < 0.f) command = propagate_at_surface(flag, p, s, normal, r, d, aligned);
+        else if (ems == 3) { advance(r, 1); keep(r, d.w3, d.w4, d.w5); flag = SURFACE_DETECT; command = BREAK; }
     }
     set_flag(p, flag);
     return command;
@@ -365,23 +378,31 @@ OXG void gen_torch(Ph& p, const float4* gs, uint64_t photon_id, Rng& r) {
     float zx = q4.x, zy = q4.y, ax = q4.z, ay = q4.w, radius = q5.x, distance = q5.y;
     p.wavelength = q3.w; p.time = q1.w;
     const float TWOPI = 2.f * PIf;
+    float u0 = 0.f, u1 = 0.f, u2 = 0.f;
+    if (type == 1 || type == 7 || type == 8) {   // the types that draw, type 6 apart (it loops)
+        const Draws d = draws(r);
+        u0 = unit(r, d.w0); u1 = unit(r, d.w1); u2 = unit(r, d.w2);
+        if (type == 8) { advance(r, 3); keep(r, d.w3, d.w4, d.w5); }
+        else { advance(r, 2); keep(r, d.w2, d.w3, d.w4); }
+    }
+    float sinPhi, cosPhi;
     if (type == 1) {
         p.mom = gmom;
-        float u_zenith = zx + uniform(r) * (zy - zx);
-        float u_azimuth = ax + uniform(r) * (ay - ax);
+        float u_zenith = zx + u0 * (zy - zx);
+        float u_azimuth = ax + u1 * (ay - ax);
         float rr = radius * u_zenith;
         float phi = TWOPI * u_azimuth;
-        float sinPhi = xsin(phi), cosPhi = xcos(phi);
+        xsincos(phi, sinPhi, cosPhi);
         p.pos = mk(rr * cosPhi, rr * sinPhi, 0.f);
         rotateUz(p.pos, p.mom);
         p.pos = add(p.pos, gpos);
         p.pol = mk(sinPhi, -cosPhi, 0.f);
         rotateUz(p.pol, p.mom);
     } else if (type == 7) {
-        float u_zenith = zx + uniform(r) * (zy - zx);
-        float u_azimuth = ax + uniform(r) * (ay - ax);
+        float u_zenith = zx + u0 * (zy - zx);
+        float u_azimuth = ax + u1 * (ay - ax);
         float phi = TWOPI * u_azimuth;
-        float sinPhi = xsin(phi), cosPhi = xcos(phi);
+        xsincos(phi, sinPhi, cosPhi);
         float cosTheta = 1.f - 2.f * u_zenith;
         float sinTheta = sqrtf(1.f - cosTheta * cosTheta);
         float flip = copysignf(1.f, radius);
@@ -389,25 +410,29 @@ OXG void gen_torch(Ph& p, const float4* gs, uint64_t photon_id, Rng& r) {
         float rad = fabsf(radius);
         p.pos = mk(sinTheta * cosPhi * rad, sinTheta * sinPhi * rad, cosTheta * rad);
         float phase = TWOPI * distance;
-        p.pol = mk(xcos(phase), xsin(phase), 0.f);
+        xsincos(phase, sinPhi, cosPhi);
+        p.pol = mk(cosPhi, sinPhi, 0.f);
         rotateUz(p.pol, p.mom);
     } else if (type == 6) {
         float u0z, u1a, u, v, b, a;
         int turns = 0;
         do {
-            u0z = zx + uniform(r) * (zy - zx);
-            u1a = ax + uniform(r) * (ay - ax);
+            draw2(r, u0, u1);
+            u0z = zx + u0 * (zy - zx);
+            u1a = ax + u1 * (ay - ax);
             u = 2.f * u0z - 1.f;
             v = 2.f * u1a - 1.f;
             b = u * u + v * v;
         } while (b > 1.f && ++turns < MAX_REJECT);
+        rng_rest(r);
         a = 2.f * sqrtf(1.f - b);
         float rad = fabsf(radius);
         float flip = copysignf(1.f, radius);
         p.mom = mk(flip * a * u, flip * a * v, flip * (2.f * b - 1.f));
         p.pos = mk(a * u * rad, a * v * rad, (2.f * b - 1.f) * rad);
         float phase = TWOPI * distance;
-        p.pol = mk(xcos(phase), xsin(phase), 0.f);
+        xsincos(phase, sinPhi, cosPhi);
+        p.pol = mk(cosPhi, sinPhi, 0.f);
         rotateUz(p.pol, p.mom);
     } else if (type == 2) {
         p.mom = gmom;
@@ -430,7 +455,7 @@ OXG void gen_torch(Ph& p, const float4* gs, uint64_t photon_id, Rng& r) {
         float f = float(photon_id) / float(numphoton);
         float frac = ax * (1.f - f) + ay * f;
         float phi = TWOPI * frac;
-        float sinPhi = xsin(phi), cosPhi = xcos(phi);
+        xsincos(phi, sinPhi, cosPhi);
         float rr = radius < 0.f ? -radius : radius;
         p.mom = mk(radius < 0.f ? -cosPhi : cosPhi, 0.f, radius < 0.f ? -sinPhi : sinPhi);
         p.pos = mk(rr * cosPhi, 0.f, rr * sinPhi);
@@ -453,14 +478,15 @@ OXG void gen_torch(Ph& p, const float4* gs, uint64_t photon_id, Rng& r) {
         p.pol = mk(0.f, -1.f, 0.f);
         rotateUz(p.pol, p.mom);
     } else if (type == 8) {
-        float u0 = uniform(r), u1 = uniform(r), u2 = uniform(r);
         float phi = TWOPI * u0;
         float cosTheta = 1.f - 2.f * u1;
         float sinTheta = sqrtf(1.f - cosTheta * cosTheta);
-        p.mom = mk(sinTheta * xcos(phi), sinTheta * xsin(phi), cosTheta);
+        sincos_bounded(phi, sinPhi, cosPhi);
+        p.mom = mk(sinTheta * cosPhi, sinTheta * sinPhi, cosTheta);
         p.pos = gpos;
         float phase = TWOPI * u2;
-        p.pol = mk(xcos(phase), xsin(phase), 0.f);
+        sincos_bounded(phase, sinPhi, cosPhi);
+        p.pol = mk(cosPhi, sinPhi, 0.f);
         rotateUz(p.pol, p.mom);
     }
     zero_flags(p);
@@ -477,21 +503,24 @@ OXG void gen_cerenkov(Ph& p, const float4* gs, Rng& r, const Tables& t) {
     float wavelength, cosTheta, sin2Theta, u_maxSin2;
     unsigned count = 0;
     do {
-        float u0 = uniform(r);
+        float u0, u1;
+        draw2(r, u0, u1);
         float w = Wmin + u0 * (Wmax - Wmin);
         wavelength = Wmin * Wmax / w;
         float4 props = boundary_lookup(t, wavelength, matline, 0u);
         float sampledRI = props.x;
         cosTheta = BetaInverse / sampledRI;
         sin2Theta = fmaxf(0.f, (1.f - cosTheta) * (1.f + cosTheta));
-        float u1 = uniform(r);
         u_maxSin2 = u1 * maxSin2;
         count += 1;
     } while (u_maxSin2 > sin2Theta && count < 100);
     float sinTheta = sqrtf(sin2Theta);
-    float u0 = uniform(r);
-    float phi = 2.f * PIf * u0;
-    float sinPhi = xsin(phi), cosPhi = xcos(phi);
+    rng_rest(r);
+    const Draws d = draws(r);   // the azimuth and the first try of the loop below
+    advance(r, 1);
+    float phi = 2.f * PIf * unit(r, d.w0);
+    float sinPhi, cosPhi;
+    sincos_bounded(phi, sinPhi, cosPhi);
     p.mom = mk(sinTheta * cosPhi, sinTheta * sinPhi, cosTheta);
     rotateUz(p.mom, p0);
     p.pol = mk(cosTheta * cosPhi, cosTheta * sinPhi, -sinTheta);
@@ -503,12 +532,14 @@ OXG void gen_cerenkov(Ph& p, const float4* gs, Rng& r, const Tables& t) {
     float step_length = q2.w;
     int turns = 0;
     do {
-        fraction = uniform(r);
+        float u;
+        if (turns == 0) { fraction = unit(r, d.w1); u = unit(r, d.w2); advance(r, 2); }
+        else draw2(r, fraction, u);
         delta = fraction * step_length;
         NumberOfPhotons = mean1 - fraction * DeltaN;
-        float u = uniform(r);
         N = u * MeanMax;
     } while (N > NumberOfPhotons && ++turns < MAX_REJECT);
+    rng_rest(r);
     float preV = q3.w, postV = q5.w;
     float midVelocity = preV + fraction * (postV - preV) * 0.5f;
     p.time = q1.w + delta / midVelocity;
@@ -520,21 +551,30 @@ OXG void gen_cerenkov(Ph& p, const float4* gs, Rng& r, const Tables& t) {
 // qscint::generate + mom_pol_wavelength (qudarap/qscint.h:55-145)
 OXG void gen_scint(Ph& p, const float4* gs, Rng& r, const Tables& t) {
     float4 q1 = gs[1], q2 = gs[2], q3 = gs[3], q5 = gs[5];
-    float u0 = uniform(r), u1 = uniform(r), u2 = uniform(r), u3 = uniform(r);
+    const Draws d = draws(r);
+    advance(r, 4);
+    const float u0 = unit(r, d.w0), u1 = unit(r, d.w1), u2 = unit(r, d.w2), u3 = unit(r, d.w3);
+    keep(r, d.w4, d.w5, d.w6);
+    const Draws e = draws(r);
     float cost = 1.f - 2.f * u0;
     float sint = sqrtf((1.f - cost) * (1.f + cost));
     float phi = 2.f * PIf * u1;
-    float sinp = xsin(phi), cosp = xcos(phi);
+    float sinp, cosp;
+    sincos_bounded(phi, sinp, cosp);
     p.mom = mk(sint * cosp, sint * sinp, cost);
     p.pol = mk(cost * cosp, cost * sinp, -sint);
     phi = 2.f * PIf * u2;
-    sinp = xsin(phi); cosp = xcos(phi);
+    sincos_bounded(phi, sinp, cosp);
     p.pol = normalize(add(mul(cosp, p.pol), mul(sinp, cross(p.mom, p.pol))));
     p.wavelength = scint_wavelength(t, u3);
     float charge = q3.y;
-    float fraction = charge == 0.f ? 1.f : uniform(r);
+    const bool drawn = charge != 0.f;   // the fraction, else it is 1
+    float fraction = drawn ? unit(r, e.w0) : 1.f;
+    float u4 = unit(r, drawn ? e.w1 : e.w0);
+    advance(r, drawn ? 2 : 1);
+    if (drawn) keep(r, e.w2, e.w3, e.w4);
+    else keep(r, e.w1, e.w2, e.w3);
     p.pos = add(mk(q1.x, q1.y, q1.z), mul(fraction, mk(q2.x, q2.y, q2.z)));
-    float u4 = uniform(r);
     float deltaTime = fraction * q2.w / q3.w - q5.x * xlog(u4);
     p.time = q1.w + deltaTime;
     zero_flags(p);

@@ -98,6 +98,7 @@ OXD bool begin_photon(const Params& P, Lane& L, long long idx) {
     const float4* gs = gsb + 6 * gsi;
     rng_init(L.r, P.rng_seed, P.rng_offset, P.skip, (unsigned long long)evt, pidx);
     if (DBG && P.pre) { L.r.pre = P.pre + (size_t)idx * P.npre; L.r.npre = P.npre; }
+    rng_rest(L.r);
     uint32_t gencode = __float_as_uint(gs[0].x);
     // the photon starts zeroed (sctx ctx = {}, CSGOptiX7.cu:432): a generator that leaves a
     // field unset (T_RECTANGLE beyond its fourth side sets no position or direction,
@@ -192,6 +193,7 @@ OXD bool resume_photon(const Params& P, Lane& L, long long idx) {
     L.idx = idx;
     load_photon(L.p, P.photon + 4 * idx);
     rng_resume(L.r, P.rng_seed, st.x, st.y);
+    rng_rest(L.r);
     L.bounce = 0;
     return true;
 }

@@ -4,4 +4,5 @@
 namespace oxl {
 template hipError_t launch_simulate_plain<false, false>(hipStream_t, const oxd::Params&, dim3, dim3, size_t, int, int);
 template hipError_t launch_simulate_persist<false, false>(hipStream_t, const oxd::Params&, dim3, dim3, size_t, bool, int);
+template const void* persist_kernel<false, false>(bool, int);
 } // namespace oxl
