@@ -349,17 +349,22 @@ OXD float scint_wavelength(const Tables& t, float u0) {
 // ------------------------------------------------------------------ CSG
 struct Is { float x, y, z, w; };
 
-// CSGNode as four float4: q0 params, q1 (z1, z2, boundary, index), q2/q3 aabb, q3.z typecode,
-// q3.w gtransformIdx|complement (CSG/CSGNode.h:67-98)
-struct NodeV { float4 q0, q1, q3; };
+// A CSGNode (CSG/CSGNode.h:67-98) on the device is two float4, the words a test reads: q0 the
+// parameters, q1 = (z1, z2, typecode | next << 8, gtransformIdx|complement). The box and the
+// index stay on the host, so a node is two loads and 32 B.
+// next is a tree node's successor in postorder that is not CSG_ZERO (0: the end), so the walk
+// neither computes it nor visits the zero nodes that fill a tree up.
+struct NodeV { float4 q0, q1; };
 OXD NodeV load_node(const float4* node, int i) {
     NodeV n;
-    n.q0 = node[4 * i + 0];
-    n.q1 = node[4 * i + 1];
-    n.q3 = node[4 * i + 3];
+    n.q0 = node[2 * i + 0];
+    n.q1 = node[2 * i + 1];
     return n;
 }
-OXD unsigned typecode(const NodeV& n) { return __float_as_uint(n.q3.z); }
+OXD unsigned node_link(const float4* node, int i) { return __float_as_uint(node[2 * i + 1].z); }
+OXD unsigned node_type(const float4* node, int i) { return node_link(node, i) & 0xffu; }
+OXD unsigned node_word0(const float4* node, int i) { return __float_as_uint(node[2 * i].x); }   // tree and list nodes: subNum
+OXD unsigned node_word1(const float4* node, int i) { return __float_as_uint(node[2 * i].y); }   // list nodes: subOffset
 
 // csg_robust_quadratic_roots.h:95-134
 OXD void rq_roots(float& t1, float& t2, float& sdisc, float d, float b, float c) {
@@ -731,21 +736,23 @@ OXD bool intersect_leaf(Is& is, const float4* node, int ni, const float4* plan, 
                         float t_min, f3 ro, f3 rd) {
     NodeV n = load_node(node, ni);
     is.x = 0.f; is.y = 0.f; is.z = 0.f; is.w = 0.f;
-    unsigned tc = typecode(n);
-    unsigned gtc = __float_as_uint(n.q3.w);
+    unsigned tc = __float_as_uint(n.q1.z) & 0xffu;
+    unsigned gtc = __float_as_uint(n.q1.w);
     unsigned gt = gtc & 0x7fffffffu;
     bool complement = (gtc & 0x80000000u) != 0;
     f3 o = ro, d = rd;
-    float4 q0, q1, q2, q3;
+    // the inverse transform's rows, element k of row j being itra[gt-1][k][j]: what the last
+    // column holds is never read
+    float4 r0, r1, r2;
     if (gt > 0) {
-        const float4* q = itra + 4 * (gt - 1);
-        q0 = q[0]; q1 = q[1]; q2 = q[2]; q3 = q[3];
-        o = mk(q0.x * ro.x + q1.x * ro.y + q2.x * ro.z + q3.x * 1.f,
-               q0.y * ro.x + q1.y * ro.y + q2.y * ro.z + q3.y * 1.f,
-               q0.z * ro.x + q1.z * ro.y + q2.z * ro.z + q3.z * 1.f);
-        d = mk(q0.x * rd.x + q1.x * rd.y + q2.x * rd.z + q3.x * 0.f,
-               q0.y * rd.x + q1.y * rd.y + q2.y * rd.z + q3.y * 0.f,
-               q0.z * rd.x + q1.z * rd.y + q2.z * rd.z + q3.z * 0.f);
+        const float4* q = itra + 3 * (gt - 1);
+        r0 = q[0]; r1 = q[1]; r2 = q[2];
+        o = mk(r0.x * ro.x + r0.y * ro.y + r0.z * ro.z + r0.w * 1.f,
+               r1.x * ro.x + r1.y * ro.y + r1.z * ro.z + r1.w * 1.f,
+               r2.x * ro.x + r2.y * ro.y + r2.z * ro.z + r2.w * 1.f);
+        d = mk(r0.x * rd.x + r0.y * rd.y + r0.z * rd.z + r0.w * 0.f,
+               r1.x * rd.x + r1.y * rd.y + r1.z * rd.z + r1.w * 0.f,
+               r2.x * rd.x + r2.y * rd.y + r2.z * rd.z + r2.w * 0.f);
     }
     bool valid = false;
     if constexpr (SIMPLE) {
@@ -769,9 +776,9 @@ OXD bool intersect_leaf(Is& is, const float4* node, int ni, const float4* plan, 
         default: break;
     }
     if (valid && gt > 0) {
-        float x = q0.x * is.x + q0.y * is.y + q0.z * is.z;
-        float y = q1.x * is.x + q1.y * is.y + q1.z * is.z;
-        float z = q2.x * is.x + q2.y * is.y + q2.z * is.z;
+        float x = r0.x * is.x + r1.x * is.y + r2.x * is.z;
+        float y = r0.y * is.x + r1.y * is.y + r2.y * is.z;
+        float z = r0.z * is.x + r1.z * is.y + r2.z * is.z;
         is.x = x; is.y = y; is.z = z;
     }
     if (complement) {
@@ -806,7 +813,7 @@ constexpr int CONTIGUOUS_MAX_SUB = 8;   // enter/aux/idx arrays of csg_intersect
 template <bool FP64>
 OXD bool intersect_node_discontiguous(Is& is, const float4* node, int ni, int root, const float4* plan,
                                       const float4* itra, float t_min, f3 ro, f3 rd) {
-    const unsigned num_sub = __float_as_uint(node[4 * ni].x), offset_sub = __float_as_uint(node[4 * ni].y);
+    const unsigned num_sub = node_word0(node, ni), offset_sub = node_word1(node, ni);
     Is closest; closest.x = 0.f; closest.y = 0.f; closest.z = 0.f; closest.w = RT_DEFAULT_MAX;
     Is s; s.x = 0.f; s.y = 0.f; s.z = 0.f; s.w = 0.f;   // one per call: a leaf reporting valid without writing keeps the last values
     for (unsigned isub = 0; isub < num_sub; isub++) {
@@ -826,7 +833,7 @@ OXD bool intersect_node_discontiguous(Is& is, const float4* node, int ni, int ro
 template <bool FP64>
 OXD bool intersect_node_contiguous(Is& is, const float4* node, int ni, int root, const float4* plan,
                                    const float4* itra, float t_min, f3 ro, f3 rd) {
-    const int num_sub = int(__float_as_uint(node[4 * ni].x)), offset_sub = int(__float_as_uint(node[4 * ni].y));
+    const int num_sub = int(node_word0(node, ni)), offset_sub = int(node_word1(node, ni));
     Is nearest_enter; nearest_enter.x = 0.f; nearest_enter.y = 0.f; nearest_enter.z = 0.f; nearest_enter.w = RT_DEFAULT_MAX;
     Is farthest_exit; farthest_exit.x = 0.f; farthest_exit.y = 0.f; farthest_exit.z = 0.f; farthest_exit.w = t_min;
     int exit_count = 0;
@@ -887,7 +894,7 @@ OXD bool intersect_node_contiguous(Is& is, const float4* node, int ni, int root,
 template <bool FP64>
 OXD bool intersect_node_overlap(Is& is, const float4* node, int ni, int root, const float4* plan,
                                 const float4* itra, float t_min, f3 ro, f3 rd) {
-    const unsigned num_sub = __float_as_uint(node[4 * ni].x), offset_sub = __float_as_uint(node[4 * ni].y);
+    const unsigned num_sub = node_word0(node, ni), offset_sub = node_word1(node, ni);
     Is farthest_enter; farthest_enter.x = 0.f; farthest_enter.y = 0.f; farthest_enter.z = 0.f; farthest_enter.w = t_min;
     Is nearest_exit; nearest_exit.x = 0.f; nearest_exit.y = 0.f; nearest_exit.z = 0.f; nearest_exit.w = RT_DEFAULT_MAX;
     const float propagate_epsilon = 0.0001f;
@@ -926,11 +933,24 @@ template <bool FP64, bool LIST, bool SIMPLE = false>
 OXD bool intersect_node(Is& is, const float4* node, int ni, int root, const float4* plan, const float4* itra,
                         float t_min, f3 ro, f3 rd) {
     if (!LIST) return intersect_leaf<FP64, SIMPLE>(is, node, ni, plan, itra, t_min, ro, rd);
-    const unsigned tc = __float_as_uint(node[4 * ni + 3].z);
+    const unsigned tc = node_type(node, ni);
     if (tc == CSG_CONTIGUOUS) { is.x = 0.f; is.y = 0.f; is.z = 0.f; is.w = 0.f; return intersect_node_contiguous<FP64>(is, node, ni, root, plan, itra, t_min, ro, rd); }
     if (tc == CSG_DISCONTIGUOUS) { is.x = 0.f; is.y = 0.f; is.z = 0.f; is.w = 0.f; return intersect_node_discontiguous<FP64>(is, node, ni, root, plan, itra, t_min, ro, rd); }
     if (tc == CSG_OVERLAP) { is.x = 0.f; is.y = 0.f; is.z = 0.f; is.w = 0.f; return intersect_node_overlap<FP64>(is, node, ni, root, plan, itra, t_min, ro, rd); }
     return intersect_leaf<FP64>(is, node, ni, plan, itra, t_min, ro, rd);
+}
+
+// What an operator makes of its two operands (CSG/csg_intersect_tree.h:430-560): the decision
+// for this pair of states, and whose sign bits promote a miss to an exit at infinity.
+OXD int csg_decide(unsigned op, const Is& L, const Is& R, f3 rd, float tmin) {
+    int l_state = classify(L, rd, tmin);
+    int r_state = classify(R, rd, tmin);
+    bool leftIsCloser = fabsf(L.w) <= fabsf(R.w);
+    bool l_promote = l_state == 2 && (signbit(L.x) || signbit(L.y));
+    bool r_promote = r_state == 2 && (signbit(R.x) || signbit(R.y));
+    if (r_promote) { r_state = 1; leftIsCloser = true; }
+    if (l_promote) { l_state = 1; leftIsCloser = false; }
+    return csg_lut(op, l_state, r_state, leftIsCloser);
 }
 
 // intersect_tree (CSG/csg_intersect_tree.h:277-672): postorder evaluation with a tranche
@@ -945,7 +965,7 @@ OXD bool intersect_node(Is& is, const float4* node, int ni, int root, const floa
 template <bool FP64, bool LIST, bool SHALLOW = false, bool SIMPLE = false>
 OXD bool intersect_tree(Is& out, const float4* node, int root, const float4* plan, const float4* itra,
                         float t_min, f3 ro, f3 rd) {
-    const unsigned numNode = __float_as_uint(node[4 * root].x);
+    const unsigned numNode = node_word0(node, root);
     const unsigned height = unsigned(__ffs(int(numNode + 1)) - 2);
     const float propagate_epsilon = 0.0001f;
     constexpr int NS = SHALLOW ? 3 : 15, NT = SHALLOW ? 3 : 4;
@@ -997,7 +1017,12 @@ OXD bool intersect_tree(Is& out, const float4* node, int root, const float4* pla
     int tr = -1;
     int sp = -1;
     int ierr = 0;
-    tr++; push_tr(tr, ((1u << height) & 0xffu) << 16, t_min);
+    // a tree node, or the next one that is not zero
+    auto skip_zero = [&](unsigned i) __attribute__((always_inline)) -> unsigned {
+        const unsigned w = node_link(node, root + int(i) - 1);
+        return (w & 0xffu) == CSG_ZERO ? w >> 8 : i;
+    };
+    tr++; push_tr(tr, skip_zero(1u << height) << 16, t_min);
     while (tr > -1) {
         unsigned slice;
         float tmin;
@@ -1011,14 +1036,8 @@ OXD bool intersect_tree(Is& out, const float4* node, int root, const float4* pla
         tr--;
         unsigned nodeIdx = (slice >> 16) & 0xff, endIdx = (slice >> 24) & 0xff;
         while (nodeIdx != endIdx) {
-            unsigned depth = 31u - unsigned(__clz(int(nodeIdx)));
-            unsigned elevation = height - depth;
             int ni = root + int(nodeIdx) - 1;
-            unsigned tc = __float_as_uint(node[4 * ni + 3].z);
-            if (tc == CSG_ZERO) {
-                nodeIdx = (nodeIdx & 1u) ? nodeIdx >> 1 : (nodeIdx << elevation) + (1u << elevation);
-                continue;
-            }
+            const unsigned link = node_link(node, ni), tc = link & 0xffu;
             if (tc >= CSG_NODE) {
                 Is ni_is; ni_is.x = 0.f; ni_is.y = 0.f; ni_is.z = 0.f; ni_is.w = 0.f;
                 intersect_node<FP64, LIST, SIMPLE>(ni_is, node, ni, root, plan, itra, tmin, ro, rd);
@@ -1032,15 +1051,7 @@ OXD bool intersect_tree(Is& out, const float4* node, int root, const float4* pla
                 bool secondLeft = signbit(top1.w);
                 if (!(firstLeft ^ secondLeft)) { ierr = 1; break; }
                 const Is L = pick(firstLeft, top0, top1), R = pick(firstLeft, top1, top0);
-                int l_state = classify(L, rd, tmin);
-                int r_state = classify(R, rd, tmin);
-                float t_left = fabsf(L.w), t_right = fabsf(R.w);
-                bool leftIsCloser = t_left <= t_right;
-                bool l_promote = l_state == 2 && (signbit(L.x) || signbit(L.y));
-                bool r_promote = r_state == 2 && (signbit(R.x) || signbit(R.y));
-                if (r_promote) { r_state = 1; leftIsCloser = true; }
-                if (l_promote) { l_state = 1; leftIsCloser = false; }
-                int ctrl = csg_lut(tc, l_state, r_state, leftIsCloser);
+                const int ctrl = csg_decide(tc, L, R, rd, tmin);
                 if (ctrl < 4) {
                     Is result = pick(ctrl == 1, L, R);
                     if (ctrl == 0) { result.x = 0.f; result.y = 0.f; result.z = 0.f; result.w = 0.f; }
@@ -1050,15 +1061,16 @@ OXD bool intersect_tree(Is& out, const float4* node, int root, const float4* pla
                     put(++sp, result);
                 } else {
                     bool loopA = ctrl == 4;
+                    const unsigned elevation = height - (31u - unsigned(__clz(int(nodeIdx))));
                     const Is other = pick(loopA, R, L);
                     unsigned leftIdx = 2 * nodeIdx, rightIdx = leftIdx + 1;
                     float tminAdvanced = fabsf(loopA ? L.w : R.w) + propagate_epsilon;
                     sp -= 2;
                     put(++sp, other);
-                    unsigned endTree = ((nodeIdx & 0xffu) << 16) | ((endIdx & 0xffu) << 24);
-                    unsigned leftTree = (((leftIdx << (elevation - 1)) & 0xffu) << 16) | (((rightIdx << (elevation - 1)) & 0xffu) << 24);
-                    unsigned rightTree = (((rightIdx << (elevation - 1)) & 0xffu) << 16) | ((nodeIdx & 0xffu) << 24);
-                    unsigned loopTree = loopA ? leftTree : rightTree;
+                    const unsigned rightFirst = skip_zero(rightIdx << (elevation - 1));   // where the right operand begins
+                    unsigned endTree = (nodeIdx << 16) | (endIdx << 24);
+                    unsigned loopTree = loopA ? (skip_zero(leftIdx << (elevation - 1)) << 16) | (rightFirst << 24)
+                                              : (rightFirst << 16) | (nodeIdx << 24);
                     if (tr >= NT - 1) { ierr = 1; break; }
                     tr++; push_tr(tr, endTree, tmin);
                     if (tr >= NT - 1) { ierr = 1; break; }
@@ -1066,7 +1078,7 @@ OXD bool intersect_tree(Is& out, const float4* node, int root, const float4* pla
                     break;
                 }
             }
-            nodeIdx = (nodeIdx & 1u) ? nodeIdx >> 1 : (nodeIdx << elevation) + (1u << elevation);
+            nodeIdx = link >> 8;
         }
         if (ierr) break;
     }
@@ -1075,17 +1087,49 @@ OXD bool intersect_tree(Is& out, const float4* node, int root, const float4* pla
     return out.w > 0.f;
 }
 
-// intersect_prim (CSG/csg_intersect_tree.h:684-719)
+// intersect_prim (CSG/csg_intersect_tree.h:684-719): a leaf, a list node, or a tree. A tree
+// of one operator over two leaves - most booleans of real detectors: 99 of pfRICH's 103
+// prims - takes none of the tree walk's stacks: it takes its left and right leaf and then
+// whichever the decision asks for again, from beyond its last hit, until the operator
+// decides. That is the walk's own sequence for height 1 (its tranches hold one leaf each and
+// return to the operator with the first tmin), with the two operands in named registers.
+// Leaf and pair share one call of intersect_leaf.
 template <bool FP64, bool LIST, bool SHALLOW = false, bool SIMPLE = false>
 OXD bool intersect_prim(Is& is, const float4* node, int root, const float4* plan, const float4* itra,
                         float t_min, f3 ro, f3 rd) {
     is.x = 0.f; is.y = 0.f; is.z = 0.f; is.w = 0.f;   // zeroed isect of CSGOptiX7.cu:894-898
-    unsigned tc = __float_as_uint(node[4 * root + 3].z);
-    if (tc >= CSG_LEAF) return intersect_leaf<FP64, SIMPLE>(is, node, root, plan, itra, t_min, ro, rd);
-    if (tc < CSG_NODE) return intersect_tree<FP64, LIST, SHALLOW, SIMPLE>(is, node, root, plan, itra, t_min, ro, rd);
-    if (LIST) return intersect_node<FP64, LIST>(is, node, root, root, plan, itra, t_min, ro, rd);
-    is.x = 0.f; is.y = 0.f; is.z = 0.f; is.w = 0.f;
-    return false;
+    const unsigned tc = node_type(node, root);
+    const bool leaf = tc >= CSG_LEAF;
+    const bool list = LIST && !leaf && tc >= CSG_NODE;
+    if (!leaf && !list && (node_word0(node, root) != 3u || node_type(node, root + 1) < CSG_NODE || node_type(node, root + 2) < CSG_NODE))
+        return intersect_tree<FP64, LIST, SHALLOW, SIMPLE>(is, node, root, plan, itra, t_min, ro, rd);
+    const float propagate_epsilon = 0.0001f;
+    Is L = is, R = is;
+    int which = 0;            // the operand to take: 0 left, 1 right
+    bool both = false;        // R has been taken
+    float tmin = t_min;
+    for (;;) {
+        Is v; v.x = 0.f; v.y = 0.f; v.z = 0.f; v.w = 0.f;
+        const bool valid = intersect_node<FP64, LIST, SIMPLE>(v, node, leaf || list ? root : root + 1 + which, root, plan, itra, tmin, ro, rd);
+        if (leaf || list) { is = v; return valid; }
+        if (which == 0) L = v; else R = v;
+        if (!both) {
+            both = which == 1;
+            which = 1;
+            if (!both) continue;
+        }
+        const int ctrl = csg_decide(tc, L, R, rd, t_min);
+        if (ctrl < 4) {
+            if (ctrl == 0) return false;
+            const bool left = ctrl == 1;
+            is.x = left ? L.x : R.x; is.y = left ? L.y : R.y; is.z = left ? L.z : R.z;
+            if (ctrl == 3) { is.x = -is.x; is.y = -is.y; is.z = -is.z; }
+            is.w = fabsf(left ? L.w : R.w);
+            return is.w > 0.f;
+        }
+        which = ctrl == 4 ? 0 : 1;
+        tmin = fabsf(which == 0 ? L.w : R.w) + propagate_epsilon;
+    }
 }
 
 } // namespace oxd

@@ -35,11 +35,11 @@ oxd::Geom Engine::geom() const {
     oxd::Geom g;
     g.node = node.p; g.plan = plan.p; g.itra = itra.p; g.prim = prim.p;
     const bool f = use_flat();
-    g.tlas = f ? tlas_f.p : tlas.p; g.blas = blas.p; g.inst = inst.p;
+    g.tlas = f ? tlas_f.p : tlas.p; g.inst = inst.p;
     g.flat = f ? flat.p : nullptr;
     g.tlas_root = f ? tlas_root_f : tlas_root; g.num_inst = num_inst;
     g.vizmask = cfg.vizmask;
-    g.rad_top = f ? rad_flat.p : rad_tlas.p; g.rad_blas = rad_blas.p;
+    g.rad = f ? rad_flat.p : rad_tlas.p;
     return g;
 }
 
@@ -72,7 +72,7 @@ bool Engine::tn_stack_for(const oxr_tuning& t, int block) const {
 // per CU at the kernels' 4 waves per SIMD. A copy that cost a resident block would cost
 // more in latency hiding than its LDS reads save.
 bool Engine::csg_copy_for(size_t smem, int block) const {
-    const size_t bytes = size_t(num_node + num_itra) * 64 + size_t(num_prim) * 8;
+    const size_t bytes = size_t(dev_nodes) * 32 + size_t(num_itra) * 48 + size_t(num_prim) * 8;
     if (bytes > 16 * 1024 || smem + bytes > 64 * 1024 || block < 64) return false;
     const size_t waves = size_t(16 / (block / 64));
     auto resident = [&](size_t sm) { return std::min(waves, size_t(160 * 1024) / std::max<size_t>(sm, 1)); };
@@ -127,8 +127,8 @@ oxd::Params Engine::params(EventBuffers& b, int64_t n, int64_t slot_off, int32_t
     P.simple_leaves = simple_leaves && !has_list ? 1 : 0;
     P.csg_node4 = P.csg_itra4 = P.csg_prim = 0;
     if (P.simple_leaves && csg_copy_for(oxl::simulate_smem(P, block), block)) {
-        P.csg_node4 = num_node * 4;
-        P.csg_itra4 = num_itra * 4;
+        P.csg_node4 = dev_nodes * 2;
+        P.csg_itra4 = num_itra * 3;
         P.csg_prim = num_prim;
     }
     P.gen_inplace = tune.generate_inplace == 1 ? 1 : 0;
@@ -383,6 +383,58 @@ static int validate_and_prims(Engine& e, const oxr_geometry* g, const oxr_physic
     return OXR_OK;
 }
 
+// The device's nodes (oxr_device.h, load_node): two float4 per CSGNode with the words the
+// tests read, and in each tree node's type word its successor in postorder that is not
+// CSG_ZERO. A link belongs to one tree: a prim whose nodes another tree has linked already
+// gets a copy of its own, behind the others.
+static std::vector<float4> device_nodes(const oxr_geometry* g, std::vector<int2>& primtab) {
+    std::vector<float4> out(size_t(g->num_node) * 2);
+    auto word = [&](int64_t n) -> uint32_t { return fbits(out[size_t(2 * n + 1)].z); };
+    for (int64_t i = 0; i < g->num_node; i++) {
+        const float* q = g->node + 16 * i;
+        out[size_t(2 * i)] = make_float4(q[0], q[1], q[2], q[3]);
+        out[size_t(2 * i + 1)] = make_float4(q[4], q[5], q[14], q[15]);
+    }
+    std::vector<int64_t> tree_of(size_t(g->num_node), -1);
+    for (int64_t p = 0; p < g->num_prim; p++) {
+        int64_t root = primtab[size_t(p)].x;
+        if (!is_op(fbits(g->node[16 * root + 14]))) continue;
+        const uint32_t num = fbits(g->node[16 * root]);   // 2^k - 1 tree nodes (validate_and_prims)
+        bool linked = false, mine = true;
+        for (uint32_t i = 0; i < num; i++) {
+            linked = linked || tree_of[size_t(root + i)] >= 0;
+            mine = mine && tree_of[size_t(root + i)] == root;
+        }
+        if (mine) continue;   // a prim of the same nodes came before
+        if (linked) {
+            int32_t numNode;
+            std::memcpy(&numNode, g->prim + 16 * p, 4);
+            const int64_t copy = int64_t(out.size() / 2);
+            for (int64_t i = 0; i < numNode; i++) {
+                const float* q = g->node + 16 * (root + i);
+                out.push_back(make_float4(q[0], q[1], q[2], q[3]));
+                out.push_back(make_float4(q[4], q[5], q[14], q[15]));
+            }
+            root = copy;
+            primtab[size_t(p)].x = int(copy);
+        } else {
+            for (uint32_t i = 0; i < num; i++) tree_of[size_t(root + i)] = root;
+        }
+        const uint32_t height = 30u - uint32_t(__builtin_clz(num + 1u));
+        auto successor = [&](uint32_t i) -> uint32_t {
+            const uint32_t elevation = height - (31u - uint32_t(__builtin_clz(i)));
+            return (i & 1u) ? i >> 1 : (i << elevation) + (1u << elevation);
+        };
+        for (uint32_t i = 1; i <= num; i++) {
+            uint32_t next = successor(i);
+            while (next != 0u && (word(root + next - 1) & 0xffu) == 0u) next = successor(next);
+            const uint32_t w = (word(root + i - 1) & 0xffu) | (next << 8);
+            std::memcpy(&out[size_t(2 * (root + i - 1) + 1)].z, &w, 4);
+        }
+    }
+    return out;
+}
+
 } // namespace oxh
 
 using namespace oxh;
@@ -494,13 +546,15 @@ int oxr_engine_create(const oxr_geometry* g, const oxr_physics* ph, const oxr_co
     std::vector<int2> primtab;
     int rc = validate_and_prims(*e, g, ph, primtab);
     if (rc) return bail(rc);
-    e->num_prim = int(g->num_prim); e->num_node = int(g->num_node); e->num_solid = int(g->num_solid);
+    const std::vector<float4> nodes = device_nodes(g, primtab);
+    e->num_prim = int(g->num_prim); e->num_node = int(g->num_node); e->dev_nodes = int(nodes.size() / 2); e->num_solid = int(g->num_solid);
     e->num_itra = int(g->num_itra);
     e->num_inst = int(g->num_inst);
     e->num_bnd = ph->num_bnd;
 
     // ---- per-solid BLAS over prim AABBs
     std::vector<oxh::NodeOut> blas_all;
+    std::vector<int32_t> solid_nodes(size_t(g->num_solid) + 1, 0);   // each solid's first node in blas_all
     std::vector<oxh::RadOut> rad_blas;
     int max_blas_depth = 0;
     e->solid_prim_offset.resize(size_t(g->num_solid));
@@ -573,6 +627,7 @@ int oxr_engine_create(const oxr_geometry* g, const oxr_physics* ph, const oxr_co
         e->solid_blas_root[size_t(s)] = bv.root_ref;
         max_blas_depth = std::max(max_blas_depth, bv.depth);
         blas_all.insert(blas_all.end(), bv.nodes.begin(), bv.nodes.end());
+        solid_nodes[size_t(s) + 1] = int32_t(blas_all.size());
         rad_blas.insert(rad_blas.end(), bv.rad.begin(), bv.rad.end());
     }
     // ---- instances and TLAS
@@ -628,7 +683,7 @@ int oxr_engine_create(const oxr_geometry* g, const oxr_physics* ph, const oxr_co
     }
     e->has_flat = placed <= kFlatMax;
     oxh::Bvh tl, tf;
-    std::vector<int2> flat_items;
+    std::vector<int4> flat_items;   // {instance, prim's place, its node offset, InstD flags}
     if (e->has_flat) {
         std::vector<oxh::Box> leaf_box;
         std::vector<oxh::RadItem> leaf_rad;
@@ -647,7 +702,8 @@ int oxr_engine_create(const oxr_geometry* g, const oxr_physics* ph, const oxr_co
                     wb.grow_point(w);
                 }
                 leaf_box.push_back(wb);
-                flat_items.push_back(make_int2(int(i), int(p)));
+                const int place = e->solid_prim_offset[size_t(gas)] + int(p);
+                flat_items.push_back(make_int4(int(i), place, primtab[size_t(place)].x, insts[size_t(i)].info.z));
                 // world-frame sphere only for an instance with the identity transform
                 oxh::RadItem ri = prim_rad[size_t(gas)][p];
                 const bool ident = q[0] == 1.f && q[1] == 0.f && q[2] == 0.f && q[4] == 0.f && q[5] == 1.f && q[6] == 0.f &&
@@ -665,9 +721,30 @@ int oxr_engine_create(const oxr_geometry* g, const oxr_physics* ph, const oxr_co
     for (auto& r : inst_rad) r.sphere = false;
     tl = oxh::build_bvh(inst_box, 0, slack_world, &inst_rad);
     e->stack_need = tl.depth + 1 + max_blas_depth;
-    e->tlas_root = tl.root_ref;
     e->tlas_nodes = int64_t(tl.nodes.size());
     e->blas_nodes = int64_t(blas_all.size());
+    // The device's refs (oxr_trace.h): instance leaves as INST_LEAVES + instance, prim leaves
+    // as ~(place in the prim table), and the solids' trees behind the instance tree in one array.
+    if (g->num_inst >= (int64_t(1) << 30) - 16 || g->num_prim > (int64_t(1) << 30) || e->tlas_nodes + e->blas_nodes >= (int64_t(1) << 31))
+        return bail(fail(OXR_EINVAL, "geometry too large for the BVH's references"));
+    auto inst_ref = [](int32_t r) { return r >= 0 ? r : int32_t(oxd::INST_LEAVES + uint32_t(~r)); };
+    for (auto& n : tl.nodes) { n.ch[0] = inst_ref(n.ch[0]); n.ch[1] = inst_ref(n.ch[1]); }
+    e->tlas_root = inst_ref(tl.root_ref);
+    for (int64_t s = 0; s < g->num_solid; s++) {
+        const int32_t offset = e->solid_prim_offset[size_t(s)];
+        auto prim_ref = [&](int32_t r) { return r >= 0 ? r + int32_t(e->tlas_nodes) : ~(~r + offset); };
+        for (int32_t k = solid_nodes[size_t(s)]; k < solid_nodes[size_t(s) + 1]; k++) {
+            blas_all[size_t(k)].ch[0] = prim_ref(blas_all[size_t(k)].ch[0]);
+            blas_all[size_t(k)].ch[1] = prim_ref(blas_all[size_t(k)].ch[1]);
+        }
+        e->solid_blas_root[size_t(s)] = prim_ref(e->solid_blas_root[size_t(s)]);
+    }
+    for (int64_t i = 0; i < g->num_inst; i++) {
+        int32_t gas; std::memcpy(&gas, g->inst + 16 * i + 7, 4);
+        insts[size_t(i)].info.w = e->solid_blas_root[size_t(gas)];
+    }
+    tl.nodes.insert(tl.nodes.end(), blas_all.begin(), blas_all.end());
+    tl.rad.insert(tl.rad.end(), rad_blas.begin(), rad_blas.end());
     if (e->stack_cap() > 96) return bail(fail(OXR_EINVAL, "BVH too deep for the traversal stack"));
 
     // ---- uploads
@@ -682,17 +759,20 @@ int oxr_engine_create(const oxr_geometry* g, const oxr_physics* ph, const oxr_co
         e->geometry_bytes += int64_t(nn * elem);
         return OXR_OK;
     };
-    if ((rc = up(e->node, g->node, size_t(g->num_node) * 4, 16))) return bail(rc);
+    std::vector<float4> rows(size_t(g->num_itra) * 3);   // the three rows of each transform
+    for (int64_t i = 0; i < g->num_itra; i++) {
+        const float* q = g->itra + 16 * i;
+        for (int j = 0; j < 3; j++) rows[size_t(3 * i + j)] = make_float4(q[j], q[4 + j], q[8 + j], q[12 + j]);
+    }
+    if ((rc = up(e->node, nodes.data(), nodes.size(), 16))) return bail(rc);
     if ((rc = up(e->plan, g->plan, size_t(g->num_plan), 16))) return bail(rc);
-    if ((rc = up(e->itra, g->itra, size_t(g->num_itra) * 4, 16))) return bail(rc);
+    if ((rc = up(e->itra, rows.data(), rows.size(), 16))) return bail(rc);
     if ((rc = up(e->prim, primtab.data(), primtab.size(), 8))) return bail(rc);
     if ((rc = up(e->tlas, tl.nodes.data(), tl.nodes.size(), 64))) return bail(rc);
-    if ((rc = up(e->blas, blas_all.data(), blas_all.size(), 64))) return bail(rc);
-    if ((rc = up(e->flat, flat_items.data(), flat_items.size(), 8))) return bail(rc);
+    if ((rc = up(e->flat, flat_items.data(), flat_items.size(), 16))) return bail(rc);
     if ((rc = up(e->tlas_f, tf.nodes.data(), tf.nodes.size(), 64))) return bail(rc);
     if ((rc = up(e->inst, insts.data(), insts.size(), 64))) return bail(rc);
     if ((rc = up(e->rad_tlas, tl.rad.data(), tl.rad.size() * 2, 16))) return bail(rc);
-    if ((rc = up(e->rad_blas, rad_blas.data(), rad_blas.size() * 2, 16))) return bail(rc);
     if ((rc = up(e->rad_flat, tf.rad.data(), tf.rad.size() * 2, 16))) return bail(rc);
     size_t bnd_f4 = size_t(ph->num_bnd) * 4 * 2 * size_t(ph->num_wl);
     if ((rc = up(e->bnd, ph->bnd, bnd_f4, 16))) return bail(rc);
@@ -718,8 +798,8 @@ void oxr_engine_destroy(oxr_engine* eh) {
     if (e->stream) (void)hipStreamSynchronize(e->stream);
     e->ev.release_all();
     e->node.release(); e->plan.release(); e->itra.release(); e->bnd.release(); e->prim.release();
-    e->tlas.release(); e->blas.release(); e->inst.release(); e->flat.release(); e->tlas_f.release();
-    e->rad_tlas.release(); e->rad_blas.release(); e->rad_flat.release(); e->optical.release(); e->icdf.release();
+    e->tlas.release(); e->inst.release(); e->flat.release(); e->tlas_f.release();
+    e->rad_tlas.release(); e->rad_flat.release(); e->optical.release(); e->icdf.release();
     if (e->e0) (void)hipEventDestroy(e->e0);
     if (e->e1) (void)hipEventDestroy(e->e1);
     if (e->e2) (void)hipEventDestroy(e->e2);

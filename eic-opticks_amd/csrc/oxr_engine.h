@@ -72,11 +72,11 @@ struct Engine {
     // geometry
     DBuf<float4> node, plan, itra, bnd;
     DBuf<int2> prim;
-    DBuf<oxd::BNode> tlas, blas;
+    DBuf<oxd::BNode> tlas;       // the instance tree, then every solid's tree
     DBuf<oxd::InstD> inst;
-    DBuf<int2> flat;             // (instance, local prim) per leaf of the flattened BVH
+    DBuf<int4> flat;             // {instance, prim's place, node offset, flags} per leaf of the flattened BVH
     DBuf<oxd::BNode> tlas_f;     // the flattened BVH (built when the placed prims are few enough)
-    DBuf<float4> rad_tlas, rad_blas, rad_flat;   // radial bounds, two float4 per node of each tree
+    DBuf<float4> rad_tlas, rad_flat;   // radial bounds, two float4 per node of tlas and tlas_f
     bool has_flat = false;
     int tlas_root_f = 0;
     int64_t tlas_nodes_f = 0;
@@ -89,6 +89,7 @@ struct Engine {
     DBuf<float> icdf;
     int tlas_root = 0;
     int num_inst = 0, num_solid = 0, num_prim = 0, num_node = 0, num_itra = 0;
+    int dev_nodes = 0;       // nodes on the device: num_node and the copies of shared trees (device_nodes)
     int64_t tlas_nodes = 0, blas_nodes = 0;
     int stack_need = 0;
     std::vector<int> solid_prim_offset, solid_num_prim, solid_blas_root;

@@ -198,9 +198,8 @@ __global__ void __launch_bounds__(256) k_trace_rays(Params P, const float4* __re
     if (i >= n) return;
     float4 a = rays[2 * i], b = rays[2 * i + 1];
     Hit h;
-    uint32_t v = 0, t = 0, err = 0, cb = 0, iv = 0;
-    bool found = trace<FP64, false, LIST, false, FLAT>(P.g, mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), a.w, b.w, h, stk, blockDim.x,
-                                    P.stack_cap, top, P.ntop, v, t, err, cb, iv);
+    bool found = trace<FP64, LIST, FLAT>(P.g, mk(a.x, a.y, a.z), mk(b.x, b.y, b.z), a.w, b.w, h, stk, blockDim.x, P.stack_cap,
+                                         top, P.ntop);
     float lc = 0.f, lf = 0.f;
     if (found) {
         lc = h.lpos.z / sqrtf(dot(h.lpos, h.lpos));
@@ -254,9 +253,13 @@ __global__ void __launch_bounds__(256) k_simtrace(Params P, const float4* __rest
                   m0.y * d.x + m1.y * d.y + m2.y * d.z + m3.y * 0.f,
                   m0.z * d.x + m1.z * d.y + m2.z * d.z + m3.z * 0.f);
     Hit h;
-    uint32_t nv = 0, nt = 0, err = 0, cb = 0, iv = 0;
-    const bool found = trace_refined<FP64, false, LIST, false, FLAT, false, false>(P, o, v, P.tmin, h, stk, blockDim.x, top, P.ntop,
-                                                                            nv, nt, err, cb, iv);
+    float t_approx = NOT_REFINED;
+    bool found;
+    do {
+        found = trace<FP64, LIST, FLAT>(P.g, ray_origin(o, v, t_approx), v, P.tmin, P.tmax, h, stk, blockDim.x, P.stack_cap, top, P.ntop);
+        if (!found) h.t = 1.f;
+    } while (refine_again(P, h, t_approx));
+    if (t_approx != NOT_REFINED) h.t = h.t + t_approx;
     // a miss carries the miss program's q0: the mid-grey background as normal, distance 1
     // (CSGOptiX7.cu:655-682 with SBT::updateMiss, SBT.cc:180-192)
     if (!found) h.n = mk(0.6f, 0.6f, 0.6f);

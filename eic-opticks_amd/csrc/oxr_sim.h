@@ -117,50 +117,47 @@ OXD bool begin_photon(const Params& P, Lane& L, long long idx) {
     return true;
 }
 
-// trace<refine> (CSGOptiX7.cu:110-216): with PropagateRefine, when 0.99 of the distance
-// found lies beyond the refine distance, the ray is traced again from that point and the
-// 0.99 part added back, so a far surface is intersected from close by. A miss reports
-// distance 1, as the miss program writes it (CSGOptiX7.cu:666-670), so h.t is the
-// reference's prd distance in every case. One trace call site serves both passes.
-// CSGL: the node and itra arrays and the prim table are read from the LDS copy stage_csg made.
-template <bool FP64, bool COUNT, bool LIST, bool TN, bool FLAT, bool SHALLOW, bool RADIAL, bool SIMPLE = false,
-          bool CSGL = false>
-OXD bool trace_refined(const Params& P, f3 pos, f3 mom, float tmin, Hit& h, int* stk, int stride,
-                       const BNode* top, int ntop, uint32_t& visits, uint32_t& tests, uint32_t& err,
-                       uint32_t& csgb, uint32_t& ivis) {
+// the geometry as the kernel reads it: with CSGL the node and itra arrays and the prim table
+// come from the LDS copy stage_csg made
+template <bool CSGL>
+OXD Geom geom_of(const Params& P) {
     Geom g = P.g;
     if constexpr (CSGL) {
         g.node = csg_copy(P);
         g.itra = g.node + P.csg_node4;
         g.prim = reinterpret_cast<const int2*>(g.itra + P.csg_itra4);
     }
-    f3 o = pos;
-    float t_approx = 0.f;
-    bool refined = false, found;
-    for (;;) {
-        found = trace<FP64, COUNT, LIST, TN, FLAT, SHALLOW, RADIAL, SIMPLE>(g, o, mom, tmin, P.tmax, h, stk, stride, P.stack_cap,
-                                                                   top, ntop, visits, tests, err, csgb, ivis);
-        if (!found) h.t = 1.f;
-        if (!P.refine || refined) break;
-        t_approx = 0.99f * h.t;
-        if (!(t_approx > P.refine_distance)) break;
-        o = mk(pos.x + t_approx * mom.x, pos.y + t_approx * mom.y, pos.z + t_approx * mom.z);
-        refined = true;
-    }
-    if (refined) h.t = h.t + t_approx;
-    return found;
+    return g;
 }
 
-// one loop iteration of CSGOptiX7.cu:450-482; returns false when the photon is done
-template <bool FP64, bool COUNT, bool DBG, bool LIST, int TM>
-OXD bool step_photon(const Params& P, Lane& L, int* stk, int stride, const BNode* top, int ntop,
-                     uint32_t& visits, uint32_t& tests, uint32_t& err, uint32_t& csgb, uint32_t& ivis) {
-    if (!(L.bounce < P.max_bounce && L.p.time < P.max_time)) return false;
-    float tmin = (L.p.obf & P.eps0_mask) ? P.tmin0 : P.tmin;
-    Hit h;
-    bool found = trace_refined<FP64, COUNT, LIST, (TM & 1) != 0, (TM & 2) != 0, (TM & 4) != 0, (TM & 8) != 0, (TM & 16) != 0,
-                               (TM & 32) != 0>(
-        P, L.p.pos, L.p.mom, tmin, h, stk, stride, top, ntop, visits, tests, err, csgb, ivis);
+// trace<refine> (CSGOptiX7.cu:110-216): with PropagateRefine, when 0.99 of the distance
+// found lies beyond the refine distance, the ray is traced again from that point and the
+// 0.99 part added back, so a far surface is intersected from close by. A miss reports
+// distance 1, as the miss program writes it (CSGOptiX7.cu:666-670), so h.t is the
+// reference's prd distance in every case. t_approx holds the part already covered,
+// NOT_REFINED before the second trace.
+constexpr float NOT_REFINED = -1e38f;
+OXD f3 ray_origin(f3 pos, f3 mom, float t_approx) {
+    if (t_approx == NOT_REFINED) return pos;
+    return mk(pos.x + t_approx * mom.x, pos.y + t_approx * mom.y, pos.z + t_approx * mom.z);
+}
+// true when the ended trace (distance h.t) has to run again from t_approx, which is set
+OXD bool refine_again(const Params& P, const Hit& h, float& t_approx) {
+    if (!P.refine || t_approx != NOT_REFINED) return false;
+    const float ta = 0.99f * h.t;
+    if (!(ta > P.refine_distance)) return false;
+    t_approx = ta;
+    return true;
+}
+
+// the photon goes on to another trace (loop condition of CSGOptiX7.cu:450-482)
+OXD bool goes_on(const Params& P, const Lane& L) { return L.bounce < P.max_bounce && L.p.time < P.max_time; }
+OXD float photon_tmin(const Params& P, const Lane& L) { return (L.p.obf & P.eps0_mask) ? P.tmin0 : P.tmin; }
+
+// what one loop iteration of CSGOptiX7.cu:450-482 does with its trace; returns false when the
+// photon is done
+template <bool DBG>
+OXD bool shade(const Params& P, Lane& L, const Hit& h, bool found) {
     if (!found) {
         if (DBG) { L.lc = 0.f; L.lf = 0.f; }   // __miss__ms sets lposcost = lposfphi = 0
         return false;
@@ -260,7 +257,132 @@ OXD void flush_counters(const Params& P, unsigned long long steps, unsigned long
 }
 
 
+// ------------------------------------------------------------------ the wave's loop
+// A wave holds up to 64 photons, each at its own place: at a BVH node, at a prim to test, or
+// at the end of its trace with a bounce to compute. A turn of the loop runs one of the three
+// for the lanes that wait for it. The loop is bound by vector issue under divergence: when a
+// bounce waited for every lane's trace and a prim was tested as soon as one lane reached it,
+// 18-37% of the lanes of an issued instruction were active.
+//   * Nodes run while NODE_LEAST/64 of the wave's photons are at one: a visit costs a tenth to
+//     a fiftieth of a prim test or a bounce and brings lanes on to those. 3 and 10 of 64 cost the
+//     instanced-CSG event 3% more, 12 gained 2% on thin shells and lost 5% there.
+//   * Prims are tested before bounces are computed unless LEAF_WEIGHT times as many lanes wait
+//     for a bounce, the dearer step. With 2 instead of 16 the instanced-CSG event takes 8.5 ms
+//     and thin shells 17.5; 32 is the same as 16; choosing by the steps' measured clocks was
+//     slower on every event but the calorimeter.
+// Kernel times on MI355X, bounce-by-bounce loop -> this one: instanced CSG (10M photons)
+// 9.5 -> 7.8 ms, thin shells (500k) 20.9 -> 16.1 ms, with FP64 roots (150k) 11.8 -> 9.5 ms,
+// pfRICH (300k) 6.5 -> 6.1 ms, calorimeter (2.07M) 2.9 -> 2.4 ms (claims by the chunk, below).
+constexpr int NODE_LEAST = 6, LEAF_WEIGHT = 16;
+
+template <bool FP64, bool COUNT, bool DBG, bool LIST, int TM, bool REFILL>
+OXD void run_wave(const Params& P, int* stk, int stride, const BNode* top) {
+    constexpr bool TN = (TM & 1) != 0, FLAT = (TM & 2) != 0, SHALLOW = (TM & 4) != 0, RADIAL = (TM & 8) != 0,
+                   SIMPLE = (TM & 16) != 0, CSGL = (TM & 32) != 0;
+    const Geom g = geom_of<CSGL>(P);
+    const int lane = threadIdx.x & 63;
+    Lane L;
+    Trav v;
+    float t_approx = NOT_REFINED;
+    uint32_t steps = 0;
+    uint32_t err = 0;
+    TraceCount cnt = {0, 0, 0, 0};
+    v.cur = TRAV_IDLE;
+    bool first = true, drained = false;
+    unsigned long long pool = 0;   // photons the wave has claimed and not yet started: [pool, pool + pooled)
+    int pooled = 0;
+    for (;;) {
+        int nnode = __popcll(__ballot(at_node(v)));
+        const int nleaf = __popcll(__ballot(at_leaf(v)));
+        const int nend = __popcll(__ballot(v.cur == TRAV_DONE));
+        const int least = max(1, ((nnode + nleaf + nend) * NODE_LEAST) >> 6);   // lanes that keep the nodes running
+        if (nnode >= least) {
+            RayF r;
+            const f3 org = P.refine ? ray_origin(L.p.pos, L.p.mom, t_approx) : L.p.pos;
+            if (at_node(v)) ray_of<FLAT, RADIAL>(r, g, v, org, L.p.mom);
+            do {
+                if (at_node(v)) trav_node<COUNT, TN, FLAT, RADIAL>(v, g, r, org, L.p.mom, stk, stride, P.stack_cap, top, P.ntop, err, cnt);
+                nnode = __popcll(__ballot(at_node(v)));
+            } while (nnode >= least);
+            continue;
+        }
+        if (nleaf > 0 && nleaf * LEAF_WEIGHT >= nend) {
+            if (at_leaf(v))
+                trav_leaf<FP64, COUNT, LIST, TN, FLAT, SHALLOW, SIMPLE>(v, g, P.refine ? ray_origin(L.p.pos, L.p.mom, t_approx) : L.p.pos,
+                                                                       L.p.mom, photon_tmin(P, L), stk, stride, P.stack_cap, cnt);
+            continue;
+        }
+        if (nend > 0 && v.cur == TRAV_DONE) {
+            Hit h;
+            const bool found = trav_hit<FLAT>(v, g, ray_origin(L.p.pos, L.p.mom, t_approx), L.p.mom, h);
+            if (!found) h.t = 1.f;
+            if (refine_again(P, h, t_approx)) {
+                trav_begin(v, g, P.tmax, stk, stride, P.stack_cap, TN);
+            } else {
+                if (t_approx != NOT_REFINED) h.t = h.t + t_approx;
+                t_approx = NOT_REFINED;
+                if (shade<DBG>(P, L, h, found) && goes_on(P, L)) {
+                    trav_begin(v, g, P.tmax, stk, stride, P.stack_cap, TN);
+                } else {
+                    end_photon<DBG>(P, L);
+                    steps += uint32_t(L.bounce);
+                    v.cur = TRAV_IDLE;
+                }
+            }
+        }
+        const uint64_t idle = __ballot(v.cur == TRAV_IDLE);
+        const int nidle = __popcll(idle);
+        if (drained) {
+            if (nidle == 64) break;
+            continue;
+        }
+        if (nidle > 0 && (nidle >= P.refill_threshold || nidle == 64)) {
+            // The wave's idle lanes take the next photons: the first time those of the lanes'
+            // numbers in the grid, then photons the wave has claimed with an add on the queue
+            // counter (which counts on from the first ones), 64 at a time while the queue holds
+            // many, else just what the lanes need. The adds of all waves meet at one address:
+            // with one per refill (177,000 in the calorimeter event) they bound that event,
+            // 3.03 against 2.35 ms.
+            const unsigned long long nfirst = (unsigned long long)gridDim.x * blockDim.x;
+            unsigned long long i = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
+            if (first) {
+                first = false;
+                drained = !REFILL || nfirst >= (unsigned long long)P.num_photon;
+            } else {
+                const int rank = int(__builtin_amdgcn_mbcnt_hi(uint32_t(idle >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(idle), 0u)));
+                const int more = nidle - pooled;
+                i = pool + (unsigned long long)rank;
+                if (more > 0) {
+                    const bool many = pool + 2ull * nfirst < (unsigned long long)P.num_photon;
+                    const int take = many ? max(more, 64) : more;
+                    unsigned long long base = 0;
+                    if (lane == 0) base = atomicAdd(P.counters + 1, (unsigned long long)take);
+                    base = __shfl(base, 0, 64) + nfirst;
+                    if (rank >= pooled) i = base + (unsigned long long)(rank - pooled);
+                    pool = base + (unsigned long long)more;
+                    pooled = take - more;
+                } else {
+                    pool += (unsigned long long)nidle;
+                    pooled -= nidle;
+                }
+                drained = pool >= (unsigned long long)P.num_photon;
+            }
+            if (v.cur == TRAV_IDLE && i < (unsigned long long)P.num_photon) {
+                const long long pi = REFILL && P.perm ? (long long)P.perm[i] : (long long)i;
+                if (start_photon<DBG>(P, L, pi)) {
+                    if (goes_on(P, L)) { trav_begin(v, g, P.tmax, stk, stride, P.stack_cap, TN); t_approx = NOT_REFINED; }
+                    else end_photon<DBG>(P, L);
+                } else {
+                    P.hitflag[pi] = 0;
+                }
+            }
+        }
+    }
+    flush_counters(P, steps, cnt.visits, cnt.tests, err, COUNT, cnt.csgb, cnt.ivis);
+}
+
 // ------------------------------------------------------------------ plain form
+// one lane per photon, no refill
 template <bool FP64, bool COUNT, bool DBG, bool LIST, int TM>
 __global__ void __launch_bounds__(256, OXR_PLAIN_WAVES) k_simulate(Params P) {
     extern __shared__ int4 smem4[];
@@ -269,29 +391,16 @@ __global__ void __launch_bounds__(256, OXR_PLAIN_WAVES) k_simulate(Params P) {
     stage_top(P, top, P.ntop);
     stage_csg<TM>(P);
     __syncthreads();
-    long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    unsigned long long steps = 0, visits = 0, tests = 0, csgb = 0, ivis = 0;
-    uint32_t err = 0;
-    if (idx < P.num_photon) {
-        Lane L;
-        if (start_photon<DBG>(P, L, idx)) {
-            uint32_t v = 0, t = 0, cb = 0, iv = 0;
-            while (step_photon<FP64, COUNT, DBG, LIST, TM>(P, L, stk, blockDim.x, top, P.ntop, v, t, err, cb, iv)) {}
-            end_photon<DBG>(P, L);
-            steps = (unsigned long long)L.bounce; visits = v; tests = t; csgb = cb; ivis = iv;
-        } else {
-            P.hitflag[idx] = 0;
-        }
-    }
-    flush_counters(P, steps, visits, tests, err, COUNT, csgb, ivis);
+    run_wave<FP64, COUNT, DBG, LIST, TM, false>(P, stk, blockDim.x, top);
 }
 
 // ------------------------------------------------------------------ persistent form
-// Lanes hold one photon each and run one bounce step per loop turn. When at least
-// refill_threshold lanes of a wave are idle (or all are), the wave claims that many
-// photon indices with one atomicAdd on counters[1] and the idle lanes generate them;
-// with P.perm the k-th claim is photon P.perm[k] (a sorted order), else photon k.
-// Every wave leaves the loop once the counter has passed num_photon and its lanes are idle.
+// A fixed grid whose lanes take photons from a queue: the first by their number in the grid
+// (an add on the queue counter by every wave at once takes tens of microseconds), later
+// ones when at least refill_threshold lanes of a wave are idle (or all are), claimed with one
+// atomicAdd on counters[1]; with P.perm the k-th claim is photon P.perm[k] (a sorted
+// order), else photon k. Every wave leaves the loop once the queue has passed num_photon
+// and its lanes are idle.
 template <bool FP64, bool DBG, bool LIST, int TM>
 __global__ void __launch_bounds__(256, OXR_PERSIST_WAVES) k_simulate_persist(Params P) {
     extern __shared__ int4 smem4[];
@@ -300,44 +409,7 @@ __global__ void __launch_bounds__(256, OXR_PERSIST_WAVES) k_simulate_persist(Par
     stage_top(P, top, P.ntop);
     stage_csg<TM>(P);
     __syncthreads();
-    const int lane = threadIdx.x & 63;
-    Lane L;
-    bool active = false;
-    bool drained = false;
-    unsigned long long steps = 0;
-    uint32_t v = 0, t = 0, err = 0, cb = 0, iv = 0;
-    for (;;) {
-        uint64_t idle = __ballot(!active);
-        int nidle = __popcll(idle);
-        if (!drained && nidle > 0 && (nidle >= P.refill_threshold || nidle == 64)) {
-            int leader = __ffsll((long long)idle) - 1;
-            unsigned long long base = 0;
-            if (lane == leader) base = atomicAdd(P.counters + 1, (unsigned long long)nidle);
-            base = __shfl(base, leader, 64);
-            if (base + (unsigned long long)nidle >= (unsigned long long)P.num_photon) drained = true;
-            if (!active) {
-                unsigned rank = __builtin_amdgcn_mbcnt_hi(uint32_t(idle >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(idle), 0u));
-                unsigned long long my = base + rank;
-                if (my < (unsigned long long)P.num_photon) {
-                    const long long pi = P.perm ? (long long)P.perm[my] : (long long)my;
-                    if (start_photon<DBG>(P, L, pi)) active = true;
-                    else P.hitflag[pi] = 0;
-                }
-            }
-        }
-        if (__ballot(active) == 0ull) {
-            if (drained) break;
-            continue;
-        }
-        if (active) {
-            if (!step_photon<FP64, false, DBG, LIST, TM>(P, L, stk, blockDim.x, top, P.ntop, v, t, err, cb, iv)) {
-                end_photon<DBG>(P, L);
-                steps += (unsigned long long)L.bounce;
-                active = false;
-            }
-        }
-    }
-    flush_counters(P, steps, 0, 0, err, false);
+    run_wave<FP64, false, DBG, LIST, TM, true>(P, stk, blockDim.x, top);
 }
 
 } // namespace oxd

@@ -4,15 +4,17 @@
 //
 // Layout in HBM:
 //   tlas[]  BNode 64 B: both child boxes + child refs; BFS order so the top levels are
-//           the first nodes and a workgroup can stage them in LDS.
-//   blas[]  BNode 64 B per-solid trees over prim AABBs, concatenated.
-//   inst[]  InstD 64 B: world-to-object columns + (solid, iindex|identity, flags, blas root).
+//           the first nodes and a workgroup can stage them in LDS. The two-level form's array
+//           holds the instance tree, then every solid's tree over its prim AABBs.
+//   inst[]  InstD 64 B: world-to-object columns + (solid, iindex|identity, flags, root of the
+//           solid's tree).
 //   prim[]  int2 (nodeOffset, globalPrimIdx<<16|boundary).
-// A child ref >= 0 is an internal node, < 0 is a leaf item ~ref (one instance per TLAS
-// leaf, one prim per BLAS leaf). The traversal stack lives in LDS, one column per lane.
-//   flat[]  int2 (instance, local prim) per leaf when the geometry is flattened: one BVH
-//           over every placed prim's world box, no BLAS level. trace<..., FLAT=true>
-//           walks that tree; FLAT=false walks the two-level one.
+//   flat[]  int4 per leaf when the geometry is flattened: one BVH over every placed prim's
+//           world box, no second level. trace<..., FLAT=true> walks that tree.
+// A child ref is a node (>= 0), a prim leaf ~k (k: the prim's place in prim[], or the leaf's
+// in flat[]; at most 2^30 of them) or an instance leaf 0x80000000 + instance (two-level
+// form), so one unsigned comparison tells what a lane has to do next. The traversal stack
+// lives in LDS, one column per lane, its first entry the end mark.
 #pragma once
 #include "oxr_device.h"
 
@@ -45,24 +47,19 @@ OXD bool visible(const InstD& in, unsigned vizmask) { return ((unsigned(in.info.
 struct SolidD { int primOffset, numPrim, blasRoot, pad; };
 
 struct Geom {
-    const float4* node;
+    const float4* node;    // two float4 per CSG node (load_node)
     const float4* plan;
-    const float4* itra;
+    const float4* itra;    // three float4 per inverse CSG transform, its rows (intersect_leaf)
     const int2* prim;
     const BNode* tlas;
-    const BNode* blas;
     const InstD* inst;
-    const int2* flat;      // flattened leaves (instance, local prim), or null for two levels
+    const int4* flat;      // flattened leaves {instance, prim's place, its node offset, InstD flags}, or null
     int tlas_root;
     int num_inst;
     unsigned vizmask;      // ray visibility mask against InstD flag bits 8-15
-    // radial bounds, two float4 per node {centre, (r_in0, r_out0, r_in1, r_out1)} of the
-    // top tree (instance tree or flattened tree) and of the per-solid trees
-    const float4* rad_top;
-    const float4* rad_blas;
+    // radial bounds, two float4 per node of tlas {centre, (r_in0, r_out0, r_in1, r_out1)}
+    const float4* rad;
 };
-
-constexpr int SENTINEL = int(0x80000000u);
 
 struct Hit {
     float t;
@@ -104,206 +101,254 @@ OXD void to_object(const InstD& in, f3 pos, f3 mom, f3& o, f3& d) {
 }
 
 // Closest hit in (tmin, tmax]; ties in t go to the smaller (instance, local prim) key.
-// SHALLOW: every CSG tree of the geometry has height <= 2 (register-resident CSG stacks).
-// RADIAL: besides its box, each child must pass its radial bound: its surfaces lie between
-// r_in and r_out from the node's centre c, so along a ray from o (direction length |d|) they
-// are no nearer than max(r_in - |o - c|, |o - c| - r_out) / |d|; a child whose bound lies
-// beyond the best hit is skipped, and the bound orders the children and fills the distance
-// stack. Concentric shells, whose boxes all hold the ray origin, are culled this way.
-// stk points at this lane's LDS stack column (element k at stk[k*stride]). With TN,
-// a second column of cap floats follows the stack (at stk + stride*cap) holding each
-// pushed node's box entry distance, and a popped node whose entry lies beyond the best
-// hit so far is dropped without loading it: the same cull the box test applies, so the
-// hit found is the same.
-// During traversal only (t, instance, local prim, object-frame normal) of the best hit
-// stay live; its world normal, local position and identity words are formed afterwards
-// from the instance record, with the same arithmetic as at instance entry.
-template <bool FP64, bool COUNT, bool LIST, bool TN = false, bool FLAT = false, bool SHALLOW = false, bool RADIAL = false,
-          bool SIMPLE = false>
-OXD bool trace(const Geom& g, f3 pos, f3 mom, float tmin, float tmax, Hit& hit,
-               int* stk, int stride, int cap, const BNode* top, int ntop,
-               uint32_t& visits, uint32_t& tests, uint32_t& err, uint32_t& csgb, uint32_t& ivis) {
-    float best = tmax;
-    int best_inst = 0, best_item = 0;
-    f3 bn = mk(0.f, 0.f, 0.f);
-    bool found = false;
-    int sp = 0;
-    int cur = g.tlas_root;
-    bool at_top = true;
-    f3 o = pos, d = mom, inv = safe_inv(mom), noi = neg_oi(pos, inv);
-    const float ilen_world = RADIAL ? __builtin_amdgcn_rsqf(dot(mom, mom)) : 1.f;
-    float ilen = ilen_world;
+//
+// A traversal is a resumable state (Trav) moved on by two steps: trav_node visits one BVH
+// node (in the two-level form also enters or leaves an instance), trav_leaf tests one prim.
+// The simulate kernels hold 64 of these in a wave and choose which step runs by how many
+// lanes wait for it; trace() runs one traversal to its end. The order of a lane's own steps
+// is the same in both.
+//
+// Template flags: SHALLOW: every CSG tree of the geometry has height <= 2 (register-resident
+// CSG stacks). RADIAL: besides its box, each child must pass its radial bound: its surfaces
+// lie between r_in and r_out from the node's centre c, so along a ray from o (direction
+// length |d|) they are no nearer than max(r_in - |o - c|, |o - c| - r_out) / |d|; a child
+// whose bound lies beyond the best hit is skipped, and the bound orders the children and
+// fills the distance stack. Concentric shells, whose boxes all hold the ray origin, are
+// culled this way. TN: a second column of cap floats follows the stack (at stk + stride*cap)
+// holding each pushed node's box entry distance, and a popped node whose entry lies beyond
+// the best hit so far is dropped without loading it: the same cull the box test applies, so
+// the hit found is the same.
+//
+// Only (t, instance, local prim, object-frame normal) of the best hit and the stack position
+// live between steps: the ray in the current frame and its reciprocals are formed again
+// where a run of steps begins (ray_of, from the photon and the instance record), and the
+// best hit's world normal, local position and identity words after the end (trav_hit), all
+// with the same arithmetic.
+//
+// What a lane waits for, as ranges of the unsigned ref: [0, TRAV_WAIT_END) a node step,
+// from PRIM_LEAVES on a leaf step, and between the two a lane whose traversal has ended or
+// that holds no photon.
+constexpr uint32_t INST_LEAVES = 0x80000000u;
+constexpr uint32_t TRAV_BACK = 0xbffffff0u;       // leave the instance's tree
+constexpr uint32_t TRAV_WAIT_END = 0xbffffff1u;
+constexpr uint32_t TRAV_DONE = 0xbffffff8u;       // the traversal has ended (best_inst < 0: a miss)
+constexpr uint32_t TRAV_IDLE = 0xbffffff9u;       // the lane holds no photon
+constexpr uint32_t PRIM_LEAVES = 0xc0000000u;
+constexpr int INST_IDENT = 1 << 30;               // Trav::inst: the instance's transform is the identity
+struct Trav {
+    float best;
+    uint32_t cur;
+    int sp;
+    int inst;                   // two-level form: the instance being walked, -1 in the instance tree
+    int best_inst, best_item;   // (instance, prim's place), or (flat leaf, 0): leaves are numbered in that order
+    f3 bn;
+};
+OXD bool at_node(const Trav& v) { return v.cur < TRAV_WAIT_END; }
+OXD bool at_leaf(const Trav& v) { return v.cur >= PRIM_LEAVES; }
+OXD void trav_begin(Trav& v, const Geom& g, float tmax, int* stk, int stride, int cap, bool tn) {
+    v.best = tmax;
+    v.cur = uint32_t(g.tlas_root);
+    stk[0] = int(TRAV_DONE);
+    if (tn) reinterpret_cast<float*>(stk)[stride * cap] = -INFINITY;
+    v.sp = 1;
+    v.inst = -1;
+    v.best_inst = -1;
+    v.best_item = 0;
+    v.bn = mk(0.f, 0.f, 0.f);
+}
+
+// the ray in the frame of the current tree, and what the slab tests need of it
+struct RayF { f3 o, inv, noi; float ilen; };
+template <bool RADIAL>
+OXD void ray_frame(RayF& r, f3 o, f3 d) {
+    r.o = o;
+    r.inv = safe_inv(d);
+    r.noi = neg_oi(o, r.inv);
+    r.ilen = RADIAL ? __builtin_amdgcn_rsqf(dot(d, d)) : 1.f;
+}
+template <bool FLAT, bool RADIAL>
+OXD void ray_of(RayF& r, const Geom& g, const Trav& v, f3 pos, f3 mom) {
+    f3 o = pos, d = mom;
+    if (!FLAT && v.inst >= 0 && !(v.inst & INST_IDENT)) to_object(g.inst[v.inst], pos, mom, o, d);
+    ray_frame<RADIAL>(r, o, d);
+}
+
+// the next stack entry worth visiting; the first one is the end mark
+template <bool TN>
+OXD void trav_pop(Trav& v, const int* stk, int stride, int cap) {
+    v.sp--;
+    if (TN) {
+        const float* stkt = reinterpret_cast<const float*>(stk + stride * cap);
+        while (stkt[v.sp * stride] > v.best) v.sp--;
+    }
+    v.cur = uint32_t(stk[v.sp * stride]);
+}
+
+struct TraceCount { uint32_t visits, tests, csgb, ivis; };
+
+template <bool COUNT, bool TN, bool FLAT, bool RADIAL>
+OXD void trav_node(Trav& v, const Geom& g, RayF& r, f3 pos, f3 mom, int* stk, int stride, int cap, const BNode* top, int ntop,
+                   uint32_t& err, TraceCount& cnt) {
     float* stkt = reinterpret_cast<float*>(stk + stride * cap);
-    // pop the next entry worth visiting; false when the stack is empty
-    auto pop = [&]() -> bool {
-        while (sp > 0) {
-            sp--;
-            if (!TN || stkt[sp * stride] <= best) { cur = stk[sp * stride]; return true; }
+    if (FLAT || v.cur < INST_LEAVES) {
+        const int cur = int(v.cur);
+        BNode nd;
+        if (cur < ntop) nd = lds_node(top, cur);
+        else nd = g.tlas[cur];
+        if (COUNT) cnt.visits++;
+        float tn0, tn1;
+        bool h0 = box_hit(nd.a.x, nd.a.y, nd.a.z, nd.a.w, nd.b.x, nd.b.y, r.noi, r.inv, v.best, tn0);
+        bool h1 = box_hit(nd.b.z, nd.b.w, nd.c.x, nd.c.y, nd.c.z, nd.c.w, r.noi, r.inv, v.best, tn1);
+        if (RADIAL) {
+            const float4 rc = g.rad[2 * cur], rr = g.rad[2 * cur + 1];
+            const float dx = r.o.x - rc.x, dy = r.o.y - rc.y, dz = r.o.z - rc.z;
+            const float dist = __builtin_amdgcn_sqrtf(dx * dx + dy * dy + dz * dz);
+            const float lb0 = fmaxf(rr.x - dist, dist - rr.y) * r.ilen;
+            const float lb1 = fmaxf(rr.z - dist, dist - rr.w) * r.ilen;
+            h0 = h0 && lb0 <= v.best;
+            h1 = h1 && lb1 <= v.best;
+            tn0 = fmaxf(tn0, lb0);
+            tn1 = fmaxf(tn1, lb1);
         }
-        return false;
-    };
-    int inst = 0;
-    int primOffset = 0;
-    for (;;) {
-        if (cur >= 0) {
-            BNode nd;
-            if (at_top && cur < ntop) nd = lds_node(top, cur);
-            else nd = at_top ? g.tlas[cur] : g.blas[cur];
-            if (COUNT) visits++;
-            float tn0, tn1;
-            bool h0 = box_hit(nd.a.x, nd.a.y, nd.a.z, nd.a.w, nd.b.x, nd.b.y, noi, inv, best, tn0);
-            bool h1 = box_hit(nd.b.z, nd.b.w, nd.c.x, nd.c.y, nd.c.z, nd.c.w, noi, inv, best, tn1);
-            if (RADIAL) {
-                const float4* rb = at_top ? g.rad_top : g.rad_blas;
-                const float4 rc = rb[2 * cur], rr = rb[2 * cur + 1];
-                const float dx = o.x - rc.x, dy = o.y - rc.y, dz = o.z - rc.z;
-                const float dist = __builtin_amdgcn_sqrtf(dx * dx + dy * dy + dz * dz);
-                const float lb0 = fmaxf(rr.x - dist, dist - rr.y) * ilen;
-                const float lb1 = fmaxf(rr.z - dist, dist - rr.w) * ilen;
-                h0 = h0 && lb0 <= best;
-                h1 = h1 && lb1 <= best;
-                tn0 = fmaxf(tn0, lb0);
-                tn1 = fmaxf(tn1, lb1);
-            }
+        if (h0 || h1) {
+            const bool first0 = h0 && !(h1 && tn1 < tn0);   // the nearer child, child 0 in a tie
+            v.cur = uint32_t(first0 ? nd.ch.x : nd.ch.y);
             if (h0 && h1) {
-                bool first0 = tn0 <= tn1;
-                int nearc = first0 ? nd.ch.x : nd.ch.y;
-                int farc = first0 ? nd.ch.y : nd.ch.x;
-                if (sp < cap) {
-                    stk[sp * stride] = farc;
-                    if (TN) stkt[sp * stride] = first0 ? tn1 : tn0;
-                    sp++;
+                if (v.sp < cap) {
+                    stk[v.sp * stride] = first0 ? nd.ch.y : nd.ch.x;
+                    if (TN) stkt[v.sp * stride] = first0 ? tn1 : tn0;
+                    v.sp++;
                 } else {
                     err |= 1u;
                 }
-                cur = nearc;
-            } else if (h0) {
-                cur = nd.ch.x;
-            } else if (h1) {
-                cur = nd.ch.y;
-            } else if (!pop()) {
-                break;
             }
-            continue;
+        } else {
+            trav_pop<TN>(v, stk, stride, cap);
         }
-        if (cur == SENTINEL) {
-            at_top = true;
-            o = pos; d = mom; inv = safe_inv(mom); noi = neg_oi(pos, inv);
-            ilen = ilen_world;
-            if (!pop()) break;
-            continue;
-        }
-        int item = ~cur;
-        if (FLAT) {
-            // flattened leaf: one placed prim, tested in its instance's frame; the same
-            // (instance, local prim) key and arithmetic as the two-level path
-            const int2 fi = g.flat[item];
-            const InstD in = g.inst[fi.x];
-            if (COUNT) ivis++;
-            if (!visible(in, g.vizmask)) {
-                if (!pop()) break;
-                continue;
-            }
-            f3 lo = pos, ld = mom;
-            if ((in.info.z & 1) == 0) to_object(in, pos, mom, lo, ld);
-            int nodeOffset = g.prim[in.info.x + fi.y].x;
-            if (COUNT) {
-                tests++;
-                unsigned tc0 = __float_as_uint(g.node[4 * nodeOffset + 3].z);
-                unsigned nn = tc0 >= CSG_LEAF ? 1u : __float_as_uint(g.node[4 * nodeOffset].x);
-                for (unsigned k = 0; k < nn; k++) {
-                    float4 q3 = g.node[4 * (nodeOffset + int(k)) + 3];
-                    csgb += 64u;
-                    if (__float_as_uint(q3.z) >= CSG_LEAF && (__float_as_uint(q3.w) & 0x7fffffffu) != 0u) csgb += 64u;
-                }
-            }
-            Is is;
-            if (intersect_prim<FP64, LIST, SHALLOW, SIMPLE>(is, g.node, nodeOffset, g.plan, g.itra, tmin, lo, ld)) {
-                float t = is.w;
-                bool closer = t >= tmin && (t < best || (found && t == best && (fi.x < best_inst || (fi.x == best_inst && fi.y < best_item))));
-                if (closer) {
-                    found = true;
-                    best = t; best_inst = fi.x; best_item = fi.y;
-                    bn = mk(is.x, is.y, is.z);
-                }
-            }
-            if (!pop()) break;
-            continue;
-        }
-        if (at_top) {
-            const InstD in = g.inst[item];
-            if (COUNT) ivis++;
-            if (!visible(in, g.vizmask)) {
-                if (!pop()) break;
-                continue;
-            }
-            inst = item;
-            primOffset = in.info.x;
-            if ((in.info.z & 1) == 0) {
-                to_object(in, pos, mom, o, d);
-                inv = safe_inv(d);
-                noi = neg_oi(o, inv);
-                if (RADIAL) ilen = __builtin_amdgcn_rsqf(dot(d, d));
-            }
-            if (sp < cap) {
-                stk[sp * stride] = SENTINEL;
-                if (TN) stkt[sp * stride] = -INFINITY;
-                sp++;
-            } else {
-                err |= 1u;
-            }
-            at_top = false;
-            cur = in.info.w;
-            continue;
-        }
-        // prim leaf: item is the local prim index within the instance's solid
-        int nodeOffset = g.prim[primOffset + item].x;
-        if (COUNT) {
-            tests++;
-            unsigned tc0 = __float_as_uint(g.node[4 * nodeOffset + 3].z);
-            unsigned nn = tc0 >= CSG_LEAF ? 1u : __float_as_uint(g.node[4 * nodeOffset].x);
-            for (unsigned k = 0; k < nn; k++) {
-                float4 q3 = g.node[4 * (nodeOffset + int(k)) + 3];
-                csgb += 64u;
-                if (__float_as_uint(q3.z) >= CSG_LEAF && (__float_as_uint(q3.w) & 0x7fffffffu) != 0u) csgb += 64u;
-            }
-        }
-        Is is;
-        if (intersect_prim<FP64, LIST, SHALLOW, SIMPLE>(is, g.node, nodeOffset, g.plan, g.itra, tmin, o, d)) {
-            // a reported distance outside the ray interval is ignored, as by
-            // optixReportIntersection (CSGOptiX/CSGOptiX7.cu:912): a convex polyhedron
-            // wholly behind the ray reports valid with the zeroed isect
-            float t = is.w;
-            bool closer = t >= tmin && (t < best || (found && t == best && (inst < best_inst || (inst == best_inst && item < best_item))));
-            if (closer) {
-                found = true;
-                best = t; best_inst = inst; best_item = item;
-                bn = mk(is.x, is.y, is.z);
-            }
-        }
-        if (!pop()) break;
+        return;
     }
-    if (!found) {
+    if constexpr (!FLAT) {
+        if (v.cur == TRAV_BACK) {      // the instance's tree is done: back to the world frame
+            v.inst = -1;
+            ray_frame<RADIAL>(r, pos, mom);
+            trav_pop<TN>(v, stk, stride, cap);
+            return;
+        }
+        const int item = int(v.cur - INST_LEAVES);
+        const InstD in = g.inst[item];
+        if (COUNT) cnt.ivis++;
+        if (!visible(in, g.vizmask)) {
+            trav_pop<TN>(v, stk, stride, cap);
+            return;
+        }
+        const bool ident = (in.info.z & 1) != 0;
+        v.inst = item | (ident ? INST_IDENT : 0);
+        if (!ident) {
+            f3 o, d;
+            to_object(in, pos, mom, o, d);
+            ray_frame<RADIAL>(r, o, d);
+        }
+        if (v.sp < cap) {
+            stk[v.sp * stride] = int(TRAV_BACK);
+            if (TN) stkt[v.sp * stride] = -INFINITY;
+            v.sp++;
+        } else {
+            err |= 1u;
+        }
+        v.cur = uint32_t(in.info.w);
+    }
+}
+
+template <bool FP64, bool COUNT, bool LIST, bool TN, bool FLAT, bool SHALLOW, bool SIMPLE>
+OXD void trav_leaf(Trav& v, const Geom& g, f3 pos, f3 mom, float tmin, const int* stk, int stride, int cap, TraceCount& cnt) {
+    const int leaf = int(~v.cur);
+    f3 o = pos, d = mom;
+    int nodeOffset;
+    if (FLAT) {
+        const int4 fi = g.flat[leaf];
+        if (COUNT) cnt.ivis++;
+        if (((unsigned(fi.w) >> 8) & g.vizmask) == 0u) {
+            trav_pop<TN>(v, stk, stride, cap);
+            return;
+        }
+        if ((fi.w & 1) == 0) to_object(g.inst[fi.x], pos, mom, o, d);
+        nodeOffset = fi.z;
+    } else {
+        if (!(v.inst & INST_IDENT)) to_object(g.inst[v.inst], pos, mom, o, d);
+        nodeOffset = g.prim[leaf].x;
+    }
+    if (COUNT) {
+        cnt.tests++;
+        const unsigned nn = node_type(g.node, nodeOffset) >= CSG_LEAF ? 1u : node_word0(g.node, nodeOffset);
+        for (unsigned k = 0; k < nn; k++) {   // 64 B per CSGNode and per transform it carries
+            const float4 q1 = g.node[2 * (nodeOffset + int(k)) + 1];
+            cnt.csgb += 64u;
+            if (__float_as_uint(q1.z) >= CSG_LEAF && (__float_as_uint(q1.w) & 0x7fffffffu) != 0u) cnt.csgb += 64u;
+        }
+    }
+    Is is;
+    if (intersect_prim<FP64, LIST, SHALLOW, SIMPLE>(is, g.node, nodeOffset, g.plan, g.itra, tmin, o, d)) {
+        // a reported distance outside the ray interval is ignored, as by
+        // optixReportIntersection (CSGOptiX/CSGOptiX7.cu:912): a convex polyhedron
+        // wholly behind the ray reports valid with the zeroed isect
+        const float t = is.w;
+        // ties go to the smaller (instance, prim)
+        const int ki = FLAT ? leaf : (v.inst & ~INST_IDENT), kp = FLAT ? 0 : leaf;
+        const bool before = v.best_inst >= 0 && t == v.best && (ki < v.best_inst || (ki == v.best_inst && kp < v.best_item));
+        if (t >= tmin && (t < v.best || before)) {
+            v.best = t; v.best_inst = ki; v.best_item = kp;
+            v.bn = mk(is.x, is.y, is.z);
+        }
+    }
+    trav_pop<TN>(v, stk, stride, cap);
+}
+
+// the ended traversal's hit; false for a miss
+template <bool FLAT>
+OXD bool trav_hit(const Trav& v, const Geom& g, f3 pos, f3 mom, Hit& hit) {
+    if (v.best_inst < 0) {
         hit.t = 0.f; hit.n = mk(0.f, 0.f, 0.f); hit.lpos = mk(0.f, 0.f, 0.f);
         hit.ii_id = 0xffffffffu; hit.gpbd = 0xffffffffu;
         return false;
     }
-    const InstD in = g.inst[best_inst];
+    int bi = v.best_inst, bp = v.best_item;
+    if (FLAT) {
+        const int4 fi = g.flat[bi];
+        bi = fi.x; bp = fi.y;
+    }
+    const InstD in = g.inst[bi];
     f3 bo = pos, bd = mom;
     bool ident = (in.info.z & 1) != 0;
     if (!ident) to_object(in, pos, mom, bo, bd);
-    hit.t = best;
-    hit.lpos = mk(bo.x + best * bd.x, bo.y + best * bd.y, bo.z + best * bd.z);
+    hit.t = v.best;
+    hit.lpos = mk(bo.x + v.best * bd.x, bo.y + v.best * bd.y, bo.z + v.best * bd.z);
     hit.ii_id = uint32_t(in.info.y);
-    hit.gpbd = uint32_t(g.prim[in.info.x + best_item].y);
+    hit.gpbd = uint32_t(g.prim[bp].y);
     if (!ident) {
-        hit.n = mk(in.c0.x * bn.x + in.c1.x * bn.y + in.c2.x * bn.z,
-                   in.c0.y * bn.x + in.c1.y * bn.y + in.c2.y * bn.z,
-                   in.c0.z * bn.x + in.c1.z * bn.y + in.c2.z * bn.z);
+        hit.n = mk(in.c0.x * v.bn.x + in.c1.x * v.bn.y + in.c2.x * v.bn.z,
+                   in.c0.y * v.bn.x + in.c1.y * v.bn.y + in.c2.y * v.bn.z,
+                   in.c0.z * v.bn.x + in.c1.z * v.bn.y + in.c2.z * v.bn.z);
     } else {
-        hit.n = bn;
+        hit.n = v.bn;
     }
     return true;
+}
+
+// one ray to its end (the query kernels)
+template <bool FP64, bool LIST, bool FLAT>
+OXD bool trace(const Geom& g, f3 pos, f3 mom, float tmin, float tmax, Hit& hit, int* stk, int stride, int cap,
+               const BNode* top, int ntop) {
+    Trav v;
+    RayF r;
+    TraceCount cnt;
+    uint32_t err = 0;
+    trav_begin(v, g, tmax, stk, stride, cap, false);
+    ray_frame<false>(r, pos, mom);
+    while (v.cur != TRAV_DONE) {
+        if (at_leaf(v)) trav_leaf<FP64, false, LIST, false, FLAT, false, false>(v, g, pos, mom, tmin, stk, stride, cap, cnt);
+        else trav_node<false, false, FLAT, false>(v, g, r, pos, mom, stk, stride, cap, top, ntop, err, cnt);
+    }
+    return trav_hit<FLAT>(v, g, pos, mom, hit);
 }
 
 } // namespace oxd
