@@ -355,7 +355,9 @@ hipError_t simulate_persist(hipStream_t s, const Params& P0, int block, int grid
     const bool simple = !debug && P.simple_leaves && !fp64 && !list;
     if (!simple) P.csg_node4 = P.csg_itra4 = P.csg_prim = 0;
     size_t sm = simulate_smem(P, block);
-    dim3 g(grid), b(block);
+    // no more workgroups than the photons fill: idle ones would stage the tree and add to the
+    // counters for nothing (ten photons: 58 us with 768 workgroups, 35 with one)
+    dim3 g((unsigned)std::min<long long>(grid, (P.num_photon + block - 1) / block)), b(block);
     const int tm = trav_mode(P) | (!debug && P.shallow_csg && !list ? 4 : 0);
     if (simple) return P.csg_node4 > 0 ? launch_simulate_simple<48>(s, P, g, b, sm, true, tm)
                                        : launch_simulate_simple<16>(s, P, g, b, sm, true, tm);

@@ -264,8 +264,9 @@ OXD void flush_counters(const Params& P, unsigned long long steps, unsigned long
 // bounce waited for every lane's trace and a prim was tested as soon as one lane reached it,
 // 18-37% of the lanes of an issued instruction were active.
 //   * Nodes run while NODE_LEAST/64 of the wave's photons are at one: a visit costs a tenth to
-//     a fiftieth of a prim test or a bounce and brings lanes on to those. 3 and 10 of 64 cost the
-//     instanced-CSG event 3% more, 12 gained 2% on thin shells and lost 5% there.
+//     a fiftieth of a prim test or a bounce and brings lanes on to those (instanced CSG: 6 of 64
+//     7.7 ms, 3 and 12 8.0, 20 9.3). With radial bounds a visit costs a third more and is most of the
+//     time, so it wants more lanes: NODE_LEAST_RADIAL (thin shells: 6 15.9 ms, 12 15.1, 20 15.6).
 //   * Prims are tested before bounces are computed unless LEAF_WEIGHT times as many lanes wait
 //     for a bounce, the dearer step. With 2 instead of 16 the instanced-CSG event takes 8.5 ms
 //     and thin shells 17.5; 32 is the same as 16; choosing by the steps' measured clocks was
@@ -273,7 +274,11 @@ OXD void flush_counters(const Params& P, unsigned long long steps, unsigned long
 // Kernel times on MI355X, bounce-by-bounce loop -> this one: instanced CSG (10M photons)
 // 9.5 -> 7.8 ms, thin shells (500k) 20.9 -> 16.1 ms, with FP64 roots (150k) 11.8 -> 9.5 ms,
 // pfRICH (300k) 6.5 -> 6.1 ms, calorimeter (2.07M) 2.9 -> 2.4 ms (claims by the chunk, below).
-constexpr int NODE_LEAST = 6, LEAF_WEIGHT = 16;
+// The plain form has no photons to refill idle lanes with, and in a small launch a wave alone on
+// its SIMD pays every turn in full: it runs each step to the last lane (calorimeter, 62k
+// photons: 696 against 780 us).
+constexpr int NODE_LEAST = 6, NODE_LEAST_RADIAL = 12, LEAF_WEIGHT = 16;
+constexpr int NODE_LEAST_PLAIN = 1, LEAF_WEIGHT_PLAIN = 64;
 
 template <bool FP64, bool COUNT, bool DBG, bool LIST, int TM, bool REFILL>
 OXD void run_wave(const Params& P, int* stk, int stride, const BNode* top) {
@@ -295,7 +300,7 @@ OXD void run_wave(const Params& P, int* stk, int stride, const BNode* top) {
         int nnode = __popcll(__ballot(at_node(v)));
         const int nleaf = __popcll(__ballot(at_leaf(v)));
         const int nend = __popcll(__ballot(v.cur == TRAV_DONE));
-        const int least = max(1, ((nnode + nleaf + nend) * NODE_LEAST) >> 6);   // lanes that keep the nodes running
+        const int least = max(1, ((nnode + nleaf + nend) * (!REFILL ? NODE_LEAST_PLAIN : RADIAL ? NODE_LEAST_RADIAL : NODE_LEAST)) >> 6);   // lanes that keep the nodes running
         if (nnode >= least) {
             RayF r;
             const f3 org = P.refine ? ray_origin(L.p.pos, L.p.mom, t_approx) : L.p.pos;
@@ -306,7 +311,7 @@ OXD void run_wave(const Params& P, int* stk, int stride, const BNode* top) {
             } while (nnode >= least);
             continue;
         }
-        if (nleaf > 0 && nleaf * LEAF_WEIGHT >= nend) {
+        if (nleaf > 0 && nleaf * (REFILL ? LEAF_WEIGHT : LEAF_WEIGHT_PLAIN) >= nend) {
             if (at_leaf(v))
                 trav_leaf<FP64, COUNT, LIST, TN, FLAT, SHALLOW, SIMPLE>(v, g, P.refine ? ray_origin(L.p.pos, L.p.mom, t_approx) : L.p.pos,
                                                                        L.p.mom, photon_tmin(P, L), stk, stride, P.stack_cap, cnt);

@@ -138,7 +138,7 @@ constexpr int INST_IDENT = 1 << 30;               // Trav::inst: the instance's 
 struct Trav {
     float best;
     uint32_t cur;
-    int sp;
+    int sp;                     // the free stack entry's offset: entry k of a lane lies at k*stride
     int inst;                   // two-level form: the instance being walked, -1 in the instance tree
     int best_inst, best_item;   // (instance, prim's place), or (flat leaf, 0): leaves are numbered in that order
     f3 bn;
@@ -150,7 +150,7 @@ OXD void trav_begin(Trav& v, const Geom& g, float tmax, int* stk, int stride, in
     v.cur = uint32_t(g.tlas_root);
     stk[0] = int(TRAV_DONE);
     if (tn) reinterpret_cast<float*>(stk)[stride * cap] = -INFINITY;
-    v.sp = 1;
+    v.sp = stride;
     v.inst = -1;
     v.best_inst = -1;
     v.best_item = 0;
@@ -176,12 +176,12 @@ OXD void ray_of(RayF& r, const Geom& g, const Trav& v, f3 pos, f3 mom) {
 // the next stack entry worth visiting; the first one is the end mark
 template <bool TN>
 OXD void trav_pop(Trav& v, const int* stk, int stride, int cap) {
-    v.sp--;
+    v.sp -= stride;
     if (TN) {
         const float* stkt = reinterpret_cast<const float*>(stk + stride * cap);
-        while (stkt[v.sp * stride] > v.best) v.sp--;
+        while (stkt[v.sp] > v.best) v.sp -= stride;
     }
-    v.cur = uint32_t(stk[v.sp * stride]);
+    v.cur = uint32_t(stk[v.sp]);
 }
 
 struct TraceCount { uint32_t visits, tests, csgb, ivis; };
@@ -214,10 +214,10 @@ OXD void trav_node(Trav& v, const Geom& g, RayF& r, f3 pos, f3 mom, int* stk, in
             const bool first0 = h0 && !(h1 && tn1 < tn0);   // the nearer child, child 0 in a tie
             v.cur = uint32_t(first0 ? nd.ch.x : nd.ch.y);
             if (h0 && h1) {
-                if (v.sp < cap) {
-                    stk[v.sp * stride] = first0 ? nd.ch.y : nd.ch.x;
-                    if (TN) stkt[v.sp * stride] = first0 ? tn1 : tn0;
-                    v.sp++;
+                if (v.sp < stride * cap) {
+                    stk[v.sp] = first0 ? nd.ch.y : nd.ch.x;
+                    if (TN) stkt[v.sp] = first0 ? tn1 : tn0;
+                    v.sp += stride;
                 } else {
                     err |= 1u;
                 }
@@ -248,10 +248,10 @@ OXD void trav_node(Trav& v, const Geom& g, RayF& r, f3 pos, f3 mom, int* stk, in
             to_object(in, pos, mom, o, d);
             ray_frame<RADIAL>(r, o, d);
         }
-        if (v.sp < cap) {
-            stk[v.sp * stride] = int(TRAV_BACK);
-            if (TN) stkt[v.sp * stride] = -INFINITY;
-            v.sp++;
+        if (v.sp < stride * cap) {
+            stk[v.sp] = int(TRAV_BACK);
+            if (TN) stkt[v.sp] = -INFINITY;
+            v.sp += stride;
         } else {
             err |= 1u;
         }
