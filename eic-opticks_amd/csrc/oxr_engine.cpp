@@ -193,12 +193,12 @@ int upload_gensteps(Engine& e, EventBuffers& b, hipStream_t s, const float* gs, 
     if (rc) return rc;
     OXR_HIP(b.gs.reserve(size_t(std::max<int64_t>(num_gs, 1)) * 6));
     OXR_HIP(b.gs_off.reserve(size_t(num_gs) + 1));
+    // staged, so the caller's array and off are free again while the copies run
     if (num_gs > 0) {
-        OXR_HIP(hipMemcpyAsync(b.gs.p, gs, size_t(num_gs) * 96, hipMemcpyHostToDevice, s));
-        OXR_HIP(hipMemcpyAsync(b.gs_off.p, off.data(), (size_t(num_gs) + 1) * sizeof(long long), hipMemcpyHostToDevice, s));
+        OXR_HIP(e.stage.h2d(s, b.gs.p, gs, size_t(num_gs) * 96));
+        OXR_HIP(e.stage.h2d(s, b.gs_off.p, off.data(), (size_t(num_gs) + 1) * sizeof(long long)));
         OXR_HIP(oxl::fill_seed(s, b.gs_off.p, int(num_gs), b.seed.p, n));
     }
-    OXR_HIP(hipStreamSynchronize(s));
     *num_photon = n;
     return OXR_OK;
 }
@@ -212,7 +212,9 @@ int run_launch(Engine& e, EventBuffers& b, hipStream_t s, int64_t n, int64_t slo
     P.pre = pre; P.npre = npre; P.input = input;
     size_t smem = oxl::simulate_smem(P, block);
     if (smem > 64 * 1024) return fail(OXR_EINVAL, "LDS budget exceeded: lower block_size or lds_top_nodes");
-    OXR_HIP(hipMemsetAsync(b.counters.p, 0, 8 * sizeof(unsigned long long), s));
+    // the last launch's selection left the counters zero; a launch that failed may not have
+    if (!e.counters_zero) OXR_HIP(hipMemsetAsync(b.counters.p, 0, 8 * sizeof(unsigned long long), s));
+    e.counters_zero = false;
     // record slots past a photon's last point stay zero, as the reference's zeroed record array
     if (P.record && n > 0) OXR_HIP(hipMemsetAsync(P.record, 0, size_t(n) * size_t(e.cfg.max_record) * 64, s));
     if (P.rec && n > 0) OXR_HIP(hipMemsetAsync(P.rec, 0, size_t(n) * size_t(e.cfg.max_rec) * 16, s));
@@ -240,13 +242,17 @@ int run_launch(Engine& e, EventBuffers& b, hipStream_t s, int64_t n, int64_t slo
         OXR_HIP(oxl::simulate_plain(s, P, block, e.cfg.fp64_roots != 0, count, e.has_list));
     }
     OXR_HIP(hipEventRecord(e.e1, s));
-    OXR_HIP(oxl::compact(s, b.hitflag.p, b.photon.p, n, b.counts.p, b.offs.p, b.hit.p, n));
+    OXR_HIP(oxl::compact(s, b.hitflag.p, b.photon.p, n, b.counts.p, b.offs.p, b.hit.p, n, b.counters.p, e.pub));
     OXR_HIP(hipEventRecord(e.e2, s));
+    OXR_HIP(hipStreamSynchronize(s));
+    e.stage.idle();
     unsigned long long ctr[8] = {0};
     long long nhit = 0;
-    OXR_HIP(hipMemcpyAsync(ctr, b.counters.p, sizeof(ctr), hipMemcpyDeviceToHost, s));
-    if (n > 0) OXR_HIP(hipMemcpyAsync(&nhit, b.offs.p + oxl::compact_blocks(n), sizeof(long long), hipMemcpyDeviceToHost, s));
-    OXR_HIP(hipStreamSynchronize(s));
+    if (n > 0) {   // nothing was launched for none, and the counters are as they were
+        std::memcpy(ctr, e.pub->counters, sizeof(ctr));
+        nhit = e.pub->num_hit;
+    }
+    e.counters_zero = true;
     if (ctr[4] != 0) return fail(OXR_EINVAL, "traversal stack overflow in BVH (geometry deeper than the stack)");
     float k_ms = 0.f, c_ms = 0.f;
     OXR_HIP(hipEventElapsedTime(&k_ms, e.e0, e.e1));
@@ -542,6 +548,9 @@ int oxr_engine_create(const oxr_geometry* g, const oxr_physics* ph, const oxr_co
     if ((he = hipEventCreate(&e->e1)) != hipSuccess) return bail(hip_fail(he, "hipEventCreate"));
     if ((he = hipEventCreate(&e->e2)) != hipSuccess) return bail(hip_fail(he, "hipEventCreate"));
     if ((he = hipEventCreate(&e->eg)) != hipSuccess) return bail(hip_fail(he, "hipEventCreate"));
+    void* pub = nullptr;
+    if ((he = hipHostMalloc(&pub, sizeof(oxd::LaunchResult), hipHostMallocDefault)) != hipSuccess) return bail(hip_fail(he, "hipHostMalloc"));
+    e->pub = static_cast<oxd::LaunchResult*>(pub);
 
     std::vector<int2> primtab;
     int rc = validate_and_prims(*e, g, ph, primtab);
@@ -804,7 +813,9 @@ void oxr_engine_destroy(oxr_engine* eh) {
     if (e->e1) (void)hipEventDestroy(e->e1);
     if (e->e2) (void)hipEventDestroy(e->e2);
     if (e->eg) (void)hipEventDestroy(e->eg);
-    if (e->h_stage) (void)hipHostFree(e->h_stage);
+    e->stage.release();
+    e->ws.release();
+    if (e->pub) (void)hipHostFree(e->pub);
     if (e->stream) (void)hipStreamDestroy(e->stream);
     delete e;
 }
@@ -898,7 +909,8 @@ int oxr_event_set_input_photons(oxr_engine* eh, const float* photons, int64_t n)
     std::lock_guard<std::mutex> lk(e->mu);
     if (n == 0) { e->have_input = false; e->input_n = 0; return OXR_OK; }
     OXR_HIP(e->ev.input.reserve(size_t(n) * 4));
-    OXR_HIP(hipMemcpy(e->ev.input.p, photons, size_t(n) * 64, hipMemcpyHostToDevice));
+    int rc = e->h2d(e->ev.input.p, photons, size_t(n) * 64);
+    if (rc) return rc;
     e->have_input = true;
     e->input_n = n;
     return OXR_OK;
@@ -911,7 +923,8 @@ int oxr_event_set_precooked(oxr_engine* eh, const float* u, int64_t n_photon, in
     if (!u || n_photon == 0) { e->have_pre = false; e->npre = 0; return OXR_OK; }
     if (n_photon < 0 || n_per < 1) return fail(OXR_EINVAL, "precooked shape");
     OXR_HIP(e->ev.pre.reserve(size_t(n_photon) * size_t(n_per)));
-    OXR_HIP(hipMemcpy(e->ev.pre.p, u, size_t(n_photon) * size_t(n_per) * 4, hipMemcpyHostToDevice));
+    int rc = e->h2d(e->ev.pre.p, u, size_t(n_photon) * size_t(n_per) * 4);
+    if (rc) return rc;
     e->have_pre = true;
     e->npre = n_per;
     e->pre_rows = n_photon;
@@ -971,6 +984,8 @@ int oxr_simulate_launch_counting(oxr_engine* eh, oxr_launch_stats* st) {
     return simulate_launch_locked(*e, OXR_FORM_PLAIN, true, st);
 }
 
+static int copy_hits(Engine& e, void* dst, int64_t n);
+
 int oxr_event_get(oxr_engine* eh, int32_t what, void* dst, int64_t cap, int64_t* count) {
     Engine* e = reinterpret_cast<Engine*>(eh);
     if (!e || !count) return fail(OXR_EINVAL, "null argument");
@@ -1017,32 +1032,26 @@ int oxr_event_get(oxr_engine* eh, int32_t what, void* dst, int64_t cap, int64_t*
     int64_t m = std::min(n, std::max<int64_t>(cap, 0));
     if (m > 0) {
         if (!dst) return fail(OXR_EINVAL, "null destination");
-        int rc = e->d2h(dst, src, size_t(m) * item);
+        int rc = what == OXR_GET_HIT ? copy_hits(*e, dst, m) : e->d2h(dst, src, size_t(m) * item);
         if (rc) return rc;
     }
     return m < n ? fail(OXR_ECAPACITY, "destination smaller than count") : OXR_OK;
 }
 
-// Device-to-host copy through the engine's pinned buffer, in chunks of at most 8 MB on the
-// engine stream (after the work that produced src): a copy straight into pageable memory
-// goes through the runtime's own staging at a few GB/s.
+// Copies on the engine stream, after the work that produced src and before the work that
+// reads dst.
 int Engine::d2h(void* dst, const void* src, size_t bytes) {
-    constexpr size_t kStage = size_t(8) << 20;
-    if (bytes == 0) return OXR_OK;
-    const size_t want = std::min(bytes, kStage);
-    if (h_stage_bytes < want) {
-        if (h_stage) (void)hipHostFree(h_stage);
-        h_stage = nullptr;
-        h_stage_bytes = 0;
-        OXR_HIP(hipHostMalloc(&h_stage, want, hipHostMallocDefault));
-        h_stage_bytes = want;
-    }
-    for (size_t off = 0; off < bytes; off += h_stage_bytes) {
-        const size_t k = std::min(h_stage_bytes, bytes - off);
-        OXR_HIP(hipMemcpyAsync(h_stage, static_cast<const char*>(src) + off, k, hipMemcpyDeviceToHost, stream));
-        OXR_HIP(hipStreamSynchronize(stream));
-        std::memcpy(static_cast<char*>(dst) + off, h_stage, k);
-    }
+    OXR_HIP(stage.d2h(stream, dst, src, bytes));
+    return OXR_OK;
+}
+int Engine::h2d(void* dst, const void* src, size_t bytes) {
+    OXR_HIP(stage.h2d(stream, dst, src, bytes));
+    return OXR_OK;
+}
+// the first n hits of the last launch: from what it published when it published that many
+static int copy_hits(Engine& e, void* dst, int64_t n) {
+    if (n > oxd::LaunchResult::HITS) return e.d2h(dst, e.ev.hit.p, size_t(n) * 64);
+    std::memcpy(dst, e.pub->hit, size_t(n) * 64);
     return OXR_OK;
 }
 
@@ -1070,7 +1079,8 @@ int oxr_event_get_merged(oxr_engine* eh, int32_t what, float time_window, void* 
     const void* in = lite ? static_cast<const void*>(e->ev.lite.p) : static_cast<const void*>(e->ev.photon.p);
     OXR_HIP(e->ev.merged.reserve(words * size_t(std::max<int64_t>(e->num_photon, 1))));
     long long nout = 0;
-    OXR_HIP(oxl::merge(e->stream, lite, in, e->num_photon, e->cfg.hitmask, true, time_window, e->ev.merged.p, &nout));
+    OXR_HIP(oxl::merge(e->stream, lite, in, e->num_photon, e->cfg.hitmask, true, time_window, e->ev.merged.p, &nout, e->ws));
+    e->ws.trim();
     return copy_out(*e, e->ev.merged.p, nout, words * 4, dst, cap, count);
 }
 
@@ -1089,10 +1099,12 @@ int oxr_merge_hits(oxr_engine* eh, int32_t what, float time_window, const void* 
     hipError_t he;
     if ((he = din.reserve(words * size_t(n))) != hipSuccess) return done(hip_fail(he, "merge input"));
     if ((he = dout.reserve(words * size_t(n))) != hipSuccess) return done(hip_fail(he, "merge output"));
-    if ((he = hipMemcpy(din.p, in, words * 4 * size_t(n), hipMemcpyHostToDevice)) != hipSuccess) return done(hip_fail(he, "merge upload"));
+    int rc = e->h2d(din.p, in, words * 4 * size_t(n));
+    if (rc) return done(rc);
     long long nout = 0;
-    if ((he = oxl::merge(e->stream, lite, din.p, n, 0u, false, time_window, dout.p, &nout)) != hipSuccess)
+    if ((he = oxl::merge(e->stream, lite, din.p, n, 0u, false, time_window, dout.p, &nout, e->ws)) != hipSuccess)
         return done(hip_fail(he, "merge"));
+    e->ws.trim();
     return done(copy_out(*e, dout.p, nout, words * 4, dst, cap, count));
 }
 
@@ -1127,7 +1139,7 @@ int oxr_simulate(oxr_engine* eh, const float* gs, int64_t num_gs, int32_t event_
         int64_t room = std::max<int64_t>(0, hit_cap - total_hit);
         int64_t take = std::min(room, s.num_hit);
         if (take > 0 && hits) {
-            int rcc = e->d2h(static_cast<char*>(hits) + size_t(total_hit) * 64, e->ev.hit.p, size_t(take) * 64);
+            int rcc = copy_hits(*e, static_cast<char*>(hits) + size_t(total_hit) * 64, take);
             if (rcc) return rcc;
         }
         if (take < s.num_hit) overflow = true;
@@ -1149,20 +1161,20 @@ int oxr_trace_rays(oxr_engine* eh, const float* rays, int64_t n, float* prd) {
     if (!e || n < 0 || (n > 0 && (!rays || !prd))) return fail(OXR_EINVAL, "bad argument");
     if (n == 0) return OXR_OK;
     std::lock_guard<std::mutex> lk(e->mu);
-    DBuf<float4> dr, dp;
-    auto cleanup = [&]() { dr.release(); dp.release(); };
-    hipError_t x;
-    if ((x = dr.reserve(size_t(n) * 2)) != hipSuccess) { cleanup(); return hip_fail(x, "hipMalloc rays"); }
-    if ((x = dp.reserve(size_t(n) * 2)) != hipSuccess) { cleanup(); return hip_fail(x, "hipMalloc prd"); }
-    if ((x = hipMemcpy(dr.p, rays, size_t(n) * 32, hipMemcpyHostToDevice)) != hipSuccess) { cleanup(); return hip_fail(x, "copy rays"); }
+    // device buffers kept in the engine's work space, copies staged on its stream: allocating
+    // two buffers, two copies from pageable memory and freeing took most of a call
+    DBuf<char>&dr = e->ws.slot[0], &dp = e->ws.slot[1];
+    OXR_HIP(dr.reserve(size_t(n) * 32));
+    OXR_HIP(dp.reserve(size_t(n) * 32));
+    int rc = e->h2d(dr.p, rays, size_t(n) * 32);
+    if (rc) return rc;
     EventBuffers dummy;
     oxd::Params P = e->params(dummy, 0, 0, 0, 256);
-    if ((x = oxl::trace_rays(e->stream, P, dr.p, n, dp.p, e->cfg.fp64_roots != 0, e->has_list)) != hipSuccess) { cleanup(); return hip_fail(x, "trace launch"); }
-    if ((x = hipStreamSynchronize(e->stream)) != hipSuccess) { cleanup(); return hip_fail(x, "trace sync"); }
-    x = hipMemcpy(prd, dp.p, size_t(n) * 32, hipMemcpyDeviceToHost);
-    cleanup();
-    if (x != hipSuccess) return hip_fail(x, "copy prd");
-    return OXR_OK;
+    OXR_HIP(oxl::trace_rays(e->stream, P, reinterpret_cast<const float4*>(dr.p), n, reinterpret_cast<float4*>(dp.p),
+                            e->cfg.fp64_roots != 0, e->has_list));
+    rc = e->d2h(prd, dp.p, size_t(n) * 32);
+    e->ws.trim();
+    return rc;
 }
 
 int oxr_simtrace(oxr_engine* eh, const float* gs, int64_t num_gs, float* simtrace, int64_t capacity, int64_t* num_out) {
@@ -1186,28 +1198,20 @@ int oxr_simtrace(oxr_engine* eh, const float* gs, int64_t num_gs, float* simtrac
     if (!simtrace) return fail(OXR_EINVAL, "null simtrace buffer");
     if (num_gs > 0x7fffffffLL) return fail(OXR_EINVAL, "too many gensteps");
     std::lock_guard<std::mutex> lk(e->mu);
-    DBuf<float4> dg, dout;
-    DBuf<long long> doff;
-    auto cleanup = [&]() { dg.release(); dout.release(); doff.release(); };
-    hipError_t x;
-    if ((x = dg.reserve(size_t(num_gs) * 6)) != hipSuccess || (x = doff.reserve(size_t(num_gs) + 1)) != hipSuccess ||
-        (x = dout.reserve(size_t(n) * 4)) != hipSuccess) {
-        cleanup(); return hip_fail(x, "hipMalloc simtrace");
-    }
-    if ((x = hipMemcpy(dg.p, gs, size_t(num_gs) * 96, hipMemcpyHostToDevice)) != hipSuccess ||
-        (x = hipMemcpy(doff.p, off.data(), off.size() * sizeof(long long), hipMemcpyHostToDevice)) != hipSuccess) {
-        cleanup(); return hip_fail(x, "copy FRAME gensteps");
-    }
+    DBuf<char>&dg = e->ws.slot[0], &doff = e->ws.slot[1], &dout = e->ws.slot[2];
+    OXR_HIP(dg.reserve(size_t(num_gs) * 96));
+    OXR_HIP(doff.reserve(off.size() * sizeof(long long)));
+    OXR_HIP(dout.reserve(size_t(n) * 64));
+    int rc = e->h2d(dg.p, gs, size_t(num_gs) * 96);
+    if (!rc) rc = e->h2d(doff.p, off.data(), off.size() * sizeof(long long));
+    if (rc) return rc;
     EventBuffers dummy;
     oxd::Params P = e->params(dummy, 0, 0, 0, 256);
-    if ((x = oxl::simtrace(e->stream, P, dg.p, doff.p, int(num_gs), n, dout.p, e->cfg.fp64_roots != 0, e->has_list)) != hipSuccess) {
-        cleanup(); return hip_fail(x, "simtrace launch");
-    }
-    if ((x = hipStreamSynchronize(e->stream)) != hipSuccess) { cleanup(); return hip_fail(x, "simtrace sync"); }
-    x = hipMemcpy(simtrace, dout.p, size_t(n) * 64, hipMemcpyDeviceToHost);
-    cleanup();
-    if (x != hipSuccess) return hip_fail(x, "copy simtrace");
-    return OXR_OK;
+    OXR_HIP(oxl::simtrace(e->stream, P, reinterpret_cast<const float4*>(dg.p), reinterpret_cast<const long long*>(doff.p), int(num_gs),
+                          n, reinterpret_cast<float4*>(dout.p), e->cfg.fp64_roots != 0, e->has_list));
+    rc = e->d2h(simtrace, dout.p, size_t(n) * 64);
+    e->ws.trim();
+    return rc;
 }
 
 int oxr_intersect_prim(oxr_engine* eh, int32_t prim_index, const float* rays, int64_t n, float* isect, int32_t* valid) {
@@ -1218,21 +1222,18 @@ int oxr_intersect_prim(oxr_engine* eh, int32_t prim_index, const float* rays, in
     std::lock_guard<std::mutex> lk(e->mu);
     int2 pr;
     OXR_HIP(hipMemcpy(&pr, e->prim.p + prim_index, sizeof(int2), hipMemcpyDeviceToHost));
-    DBuf<float4> dr, di;
-    DBuf<int> dv;
-    auto cleanup = [&]() { dr.release(); di.release(); dv.release(); };
-    hipError_t x;
-    if ((x = dr.reserve(size_t(n) * 2)) != hipSuccess || (x = di.reserve(size_t(n))) != hipSuccess || (x = dv.reserve(size_t(n))) != hipSuccess) {
-        cleanup(); return hip_fail(x, "hipMalloc isect");
-    }
-    if ((x = hipMemcpy(dr.p, rays, size_t(n) * 32, hipMemcpyHostToDevice)) != hipSuccess) { cleanup(); return hip_fail(x, "copy rays"); }
-    if ((x = oxl::intersect_prim(e->stream, e->geom(), pr.x, dr.p, n, di.p, dv.p, e->cfg.fp64_roots != 0, e->has_list)) != hipSuccess) { cleanup(); return hip_fail(x, "isect launch"); }
-    if ((x = hipStreamSynchronize(e->stream)) != hipSuccess) { cleanup(); return hip_fail(x, "isect sync"); }
-    if ((x = hipMemcpy(isect, di.p, size_t(n) * 16, hipMemcpyDeviceToHost)) != hipSuccess) { cleanup(); return hip_fail(x, "copy isect"); }
-    x = hipMemcpy(valid, dv.p, size_t(n) * 4, hipMemcpyDeviceToHost);
-    cleanup();
-    if (x != hipSuccess) return hip_fail(x, "copy valid");
-    return OXR_OK;
+    DBuf<char>&dr = e->ws.slot[0], &di = e->ws.slot[1], &dv = e->ws.slot[2];
+    OXR_HIP(dr.reserve(size_t(n) * 32));
+    OXR_HIP(di.reserve(size_t(n) * 16));
+    OXR_HIP(dv.reserve(size_t(n) * 4));
+    int rc = e->h2d(dr.p, rays, size_t(n) * 32);
+    if (rc) return rc;
+    OXR_HIP(oxl::intersect_prim(e->stream, e->geom(), pr.x, reinterpret_cast<const float4*>(dr.p), n, reinterpret_cast<float4*>(di.p),
+                                reinterpret_cast<int*>(dv.p), e->cfg.fp64_roots != 0, e->has_list));
+    rc = e->d2h(isect, di.p, size_t(n) * 16);
+    if (!rc) rc = e->d2h(valid, dv.p, size_t(n) * 4);
+    e->ws.trim();
+    return rc;
 }
 
 int oxr_autotune(oxr_engine* eh, int32_t repeat, double* results, int32_t max_results, int32_t* num_results) {

@@ -5,6 +5,7 @@
 #include <string>
 #include <vector>
 #include <mutex>
+#include "oxr_copy.h"
 #include "../../include/oxr.h"
 #include "oxr_kernels.h"
 
@@ -33,6 +34,23 @@ struct DBuf {
     }
     void release() { if (p) (void)hipFree(p); p = nullptr; n = 0; }
 };
+
+} // namespace oxh
+namespace oxl {
+// Device buffers that a call (a merge, a query) uses and the engine keeps for the next:
+// allocating and freeing them in every call cost a merge of 34k hits 60 of its 400 us and a
+// query of 250k rays, with its pageable copies, 340 of 910.
+struct Workspace {
+    static constexpr int N = 15;
+    oxh::DBuf<char> slot[N];
+    int used = 0;
+    size_t bytes() const { size_t b = 0; for (const auto& x : slot) b += x.n; return b; }
+    void release() { for (auto& x : slot) x.release(); }
+    // what stays allocated between calls is bounded
+    void trim() { if (bytes() > (size_t(512) << 20)) release(); }
+};
+} // namespace oxl
+namespace oxh {
 
 // One event slice's device buffers (the QEvt role).
 struct EventBuffers {
@@ -114,10 +132,14 @@ struct Engine {
     bool launched = false;
     bool hitlite_ready = false;
     hipEvent_t e0 = nullptr, e1 = nullptr, e2 = nullptr, eg = nullptr;
-    // pinned staging for gathers (grown on demand up to 8 MB); see d2h
-    void* h_stage = nullptr;
-    size_t h_stage_bytes = 0;
+    // Host <-> device copies through pinned staging (oxr_copy.h), on the engine stream. d2h ends
+    // with the data in dst; h2d returns when src may be reused, its copy in stream order.
+    Stager stage;
     int d2h(void* dst, const void* src, size_t bytes);
+    int h2d(void* dst, const void* src, size_t bytes);
+    oxl::Workspace ws;                  // merges and queries
+    oxd::LaunchResult* pub = nullptr;   // pinned: what the last launch left for the host
+    bool counters_zero = false;         // ev.counters is zero (the last launch's selection left it so)
     std::mutex mu;   // serialises C-ABI calls on one engine
 
     oxd::Geom geom() const;

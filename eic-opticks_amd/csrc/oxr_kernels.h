@@ -73,6 +73,16 @@ struct Params {
     int nseg;
 };
 
+// What the host reads of a finished launch, in pinned host memory: the counters, the hit
+// count and the first hits (64 B each).
+struct LaunchResult {
+    static constexpr int HITS = 1024;
+    unsigned long long counters[8];
+    long long num_hit;
+    long long pad[7];
+    float4 hit[4 * HITS];
+};
+
 } // namespace oxd
 
 namespace oxl {
@@ -135,8 +145,11 @@ bool production_kernels(const oxd::Params& P);
 // receives the sorted photon indices (inside val).
 hipError_t order_photons(hipStream_t s, const oxd::Params& P, int key_bits, unsigned long long* key, unsigned* val,
                          void* tmp, size_t* tmp_bytes, const unsigned** perm);
+// ordered hit selection; with pub the launch counters ctr, the hit count and the first hits
+// are also written there (pinned host memory) and ctr is zeroed
 hipError_t compact(hipStream_t s, const uint8_t* flag, const float4* photon, long long n, int* counts,
-                   long long* offs, float4* hit, long long hit_cap);
+                   long long* offs, float4* hit, long long hit_cap, unsigned long long* ctr = nullptr,
+                   oxd::LaunchResult* pub = nullptr);
 // compact() for the serving form: the chunk offsets (nb+1) and the 8 launch counters are
 // also written to host_offs/host_ctr, and hit rows below hcap to hhit, all pinned host
 // memory; rows from hcap on go to dhit (device, dcap rows) at the same row index
@@ -147,8 +160,10 @@ hipError_t compact_host(hipStream_t s, const uint8_t* flag, const float4* photon
 hipError_t scatter_lite(hipStream_t s, const uint8_t* flag, const uint4* lite, long long n, const long long* offs,
                         uint4* hitlite, long long hit_cap);
 // merge of sphoton (lite=false) or sphotonlite items by (identity, time bucket); see oxr_merge.hip
+// ws: device work space kept by the caller between calls (grown on demand)
+struct Workspace;
 hipError_t merge(hipStream_t s, bool lite, const void* in, long long n, unsigned select_mask, bool select,
-                 float time_window, void* out, long long* num_out);
+                 float time_window, void* out, long long* num_out, Workspace& ws);
 hipError_t trace_rays(hipStream_t s, const oxd::Params& P, const float4* rays, long long n, float4* prd, bool fp64,
                       bool list);
 hipError_t simtrace(hipStream_t s, const oxd::Params& P, const float4* gs, const long long* offsets, int num_gs,

@@ -9,7 +9,7 @@
 //                      (both in oxr_sim.h, instantiated in oxr_sim_*.hip)
 // Production variants (DBG=false) resume photons that k_generate made; the debug
 // variants (seqhis, records, precooked streams, counting) generate in place.
-//   k_count/k_scan/k_scatter  ordered hit compaction (SU::count_if/copy_if, SU.cu:49-166)
+//   k_count/k_select/k_scatter  ordered hit compaction (SU::count_if/copy_if, SU.cu:49-166)
 //   k_trace_rays, k_intersect_prim  geometry queries
 //   k_simtrace                      2-D cross-section rays from FRAME gensteps (CSGOptiX7.cu:536-577)
 #include "oxr_sim.h"
@@ -44,12 +44,18 @@ __global__ void __launch_bounds__(256) k_generate(Params P) {
 // ------------------------------------------------------------------ hit compaction
 constexpr int CHUNK = 4096;   // photons per compaction block (256 lanes x 16)
 
+// one 16-byte load per lane where the flags allow it (each flag byte is 0 or 1)
 __global__ void __launch_bounds__(256) k_count(const uint8_t* __restrict__ flag, long long n, int* __restrict__ counts) {
     long long base = (long long)blockIdx.x * CHUNK;
     int c = 0;
-    for (int k = threadIdx.x; k < CHUNK; k += 256) {
-        long long i = base + k;
-        if (i < n && flag[i]) c++;
+    if (base + CHUNK <= n && (reinterpret_cast<uintptr_t>(flag) & 15u) == 0u) {
+        const uint4 w = reinterpret_cast<const uint4*>(flag + base)[threadIdx.x];
+        c = __popc(w.x) + __popc(w.y) + __popc(w.z) + __popc(w.w);
+    } else {
+        for (int k = threadIdx.x; k < CHUNK; k += 256) {
+            long long i = base + k;
+            if (i < n && flag[i]) c++;
+        }
     }
     c = (int)wave_sum((unsigned long long)c);
     __shared__ int ws[4];
@@ -58,30 +64,67 @@ __global__ void __launch_bounds__(256) k_count(const uint8_t* __restrict__ flag,
     if (threadIdx.x == 0) counts[blockIdx.x] = ws[0] + ws[1] + ws[2] + ws[3];
 }
 
-// single workgroup exclusive scan of the per-block counts; total to out[nb]
-__global__ void __launch_bounds__(1024) k_scan(const int* __restrict__ counts, int nb, long long* __restrict__ out) {
-    __shared__ long long part[1024];
-    long long carry = 0;
-    for (int base = 0; base < nb; base += 1024) {
-        int i = base + threadIdx.x;
-        long long v = i < nb ? counts[i] : 0;
-        part[threadIdx.x] = v;
-        __syncthreads();
-        for (int off = 1; off < 1024; off <<= 1) {
-            long long add = threadIdx.x >= off ? part[threadIdx.x - off] : 0;
-            __syncthreads();
-            part[threadIdx.x] += add;
-            __syncthreads();
-        }
-        if (i < nb) out[i] = carry + part[threadIdx.x] - v;
-        long long tot = part[1023];
-        __syncthreads();
-        carry += tot;
+// The hits in photon order. Each block sums the counts of the blocks before it (at most a few
+// thousand ints from L2) instead of waiting for a scan kernel, and notes its offset for
+// k_scatter. What the host reads after a launch - the launch counters, the hit count and the
+// first hits - is also written straight to pinned host memory (pub), so a launch ends without
+// copy commands; the counters are left zero for the next launch.
+__global__ void __launch_bounds__(256) k_select(const uint8_t* __restrict__ flag, const float4* __restrict__ photon, long long n,
+                                                const int* __restrict__ counts, long long* __restrict__ offs,
+                                                float4* __restrict__ hit, long long hit_cap, unsigned long long* ctr,
+                                                LaunchResult* pub) {
+    __shared__ unsigned long long part[4];
+    __shared__ int ws[4];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    unsigned long long before = 0;
+    for (unsigned b = threadIdx.x; b < blockIdx.x; b += 256) before += (unsigned long long)counts[b];
+    before = wave_sum(before);
+    if (lane == 0) part[w] = before;
+    __syncthreads();
+    long long o = (long long)(part[0] + part[1] + part[2] + part[3]);
+    const bool last = blockIdx.x == gridDim.x - 1;
+    const long long total = last ? o + counts[blockIdx.x] : 0;
+    if (threadIdx.x == 0) {
+        offs[blockIdx.x] = o;
+        if (last) offs[gridDim.x] = total;
     }
-    if (threadIdx.x == 0) out[nb] = carry;
+    if (last && pub) {
+        if (threadIdx.x < 8) {
+            pub->counters[threadIdx.x] = ctr[threadIdx.x];
+            ctr[threadIdx.x] = 0ull;
+        }
+        if (threadIdx.x == 0) pub->num_hit = total;
+    }
+    const long long base = (long long)blockIdx.x * CHUNK;
+    for (int k = 0; k < CHUNK && base + k < n; k += 256) {
+        long long i = base + k + threadIdx.x;
+        bool f = i < n && flag[i];
+        uint64_t m = __ballot(f);
+        unsigned rank = __builtin_amdgcn_mbcnt_hi(uint32_t(m >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(m), 0u));
+        if (lane == 0) ws[w] = __popcll(m);
+        __syncthreads();
+        int ahead = 0;
+        for (int q = 0; q < w; q++) ahead += ws[q];
+        int tot = ws[0] + ws[1] + ws[2] + ws[3];
+        if (f) {
+            const long long dst = o + ahead + rank;
+            const float4* src = photon + 4 * i;
+            const float4 v0 = src[0], v1 = src[1], v2 = src[2], v3 = src[3];
+            if (dst < hit_cap) {
+                float4* d = hit + 4 * dst;
+                d[0] = v0; d[1] = v1; d[2] = v2; d[3] = v3;
+            }
+            if (pub && dst < LaunchResult::HITS) {
+                float4* d = pub->hit + 4 * dst;
+                d[0] = v0; d[1] = v1; d[2] = v2; d[3] = v3;
+            }
+        }
+        o += tot;
+        __syncthreads();
+    }
 }
 
-// W float4 per item: 4 for sphoton, 1 for sphotonlite
+// the same selection of another array by the offsets k_select left; W float4 per item
 template <int W>
 __global__ void __launch_bounds__(256) k_scatter(const uint8_t* __restrict__ flag, const float4* __restrict__ photon,
                                                  long long n, const long long* __restrict__ offs,
@@ -115,8 +158,8 @@ __global__ void __launch_bounds__(256) k_scatter(const uint8_t* __restrict__ fla
 }
 
 // Serving form's compaction: the same ordered selection, published straight to pinned
-// host memory so a finished step needs no copy command. k_scan_host is k_scan in a 256-lane
-// workgroup that also writes the offsets and the step's 8 launch counters to the host.
+// host memory so a finished step needs no copy command. k_scan_host scans the per-block counts in
+// one 256-lane workgroup and also writes the offsets and the step's 8 launch counters to the host.
 // k_scatter_host stages each 256-photon group's hits in LDS and writes them as one
 // contiguous run, so the PCIe writes are whole lines: rows below hcap go to the host
 // block, any beyond it to the device buffer at the same row (the host fetches those).
@@ -433,12 +476,11 @@ hipError_t order_photons(hipStream_t s, const Params& P, int key_bits, unsigned 
 int compact_blocks(long long n) { return int((n + CHUNK - 1) / CHUNK); }
 
 hipError_t compact(hipStream_t s, const uint8_t* flag, const float4* photon, long long n, int* counts,
-                   long long* offs, float4* hit, long long hit_cap) {
+                   long long* offs, float4* hit, long long hit_cap, unsigned long long* ctr, LaunchResult* pub) {
     if (n <= 0) return hipSuccess;
     int nb = compact_blocks(n);
     hipLaunchKernelGGL(k_count, dim3(nb), dim3(256), 0, s, flag, n, counts);
-    hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, counts, nb, offs);
-    hipLaunchKernelGGL(k_scatter<4>, dim3(nb), dim3(256), 0, s, flag, photon, n, offs, hit, hit_cap);
+    hipLaunchKernelGGL(k_select, dim3(nb), dim3(256), 0, s, flag, photon, n, counts, offs, hit, hit_cap, ctr, pub);
     return hipGetLastError();
 }
 

@@ -15,7 +15,7 @@
 // already selected input skips the selection (ALREADY_HITMASK_SELECTED, SPM.hh:23). The fold is a left
 // fold in sorted order; the reduce operations are associative, so this equals any
 // grouping a parallel reduce-by-key would use.
-#include "oxr_kernels.h"
+#include "oxr_engine.h"
 #include <hipcub/hipcub.hpp>
 
 namespace oxd {
@@ -117,23 +117,32 @@ namespace oxl {
 using namespace oxd;
 
 namespace {
+// the next slot of the kept work space: a merge allocated and freed some fourteen buffers
+// per call before (200k photons, 34k hits: see the figures at Workspace)
 struct Tmp {
+    Workspace& ws;
+    int k;
     void* p = nullptr;
-    ~Tmp() { if (p) (void)hipFree(p); }
-    hipError_t get(size_t bytes) { return hipMalloc(&p, bytes ? bytes : 1); }
+    explicit Tmp(Workspace& w) : ws(w), k(w.used++) {}
+    hipError_t get(size_t bytes) {
+        hipError_t e = ws.slot[k].reserve(bytes ? bytes : 1);
+        p = ws.slot[k].p;
+        return e;
+    }
 };
 inline unsigned nblk(long long n) { return unsigned((n + 255) / 256); }
 }
 
 template <bool LITE>
 static hipError_t merge_t(hipStream_t s, const uint32_t* in, long long n, unsigned mask, bool select, float tw,
-                          uint32_t* out, long long* num_out) {
+                          uint32_t* out, long long* num_out, Workspace& ws) {
     *num_out = 0;
+    ws.used = 0;
     if (n <= 0) return hipSuccess;
     if (n > 0x7fffffffLL) return hipErrorInvalidValue;
     const int N = int(n);
     hipError_t e;
-    Tmp sel, flag, nsel, tmp;
+    Tmp sel(ws), flag(ws), nsel(ws), tmp(ws);
     int m = N;
     const uint32_t* psel = nullptr;
     if (select) {
@@ -157,7 +166,7 @@ static hipError_t merge_t(hipStream_t s, const uint32_t* in, long long n, unsign
         *num_out = m;
         return hipStreamSynchronize(s);
     }
-    Tmp k0, k1, v0, v1, uk, cnt, st, nr, tmp2, tmp3, tmp4;
+    Tmp k0(ws), k1(ws), v0(ws), v1(ws), uk(ws), cnt(ws), st(ws), nr(ws), tmp2(ws), tmp3(ws), tmp4(ws);
     if ((e = k0.get(size_t(m) * 8)) != hipSuccess || (e = k1.get(size_t(m) * 8)) != hipSuccess ||
         (e = v0.get(size_t(m) * 4)) != hipSuccess || (e = v1.get(size_t(m) * 4)) != hipSuccess ||
         (e = uk.get(size_t(m) * 8)) != hipSuccess || (e = cnt.get(size_t(m) * 4)) != hipSuccess ||
@@ -188,9 +197,9 @@ static hipError_t merge_t(hipStream_t s, const uint32_t* in, long long n, unsign
 }
 
 hipError_t merge(hipStream_t s, bool lite, const void* in, long long n, unsigned select_mask, bool select,
-                 float time_window, void* out, long long* num_out) {
-    if (lite) return merge_t<true>(s, (const uint32_t*)in, n, select_mask, select, time_window, (uint32_t*)out, num_out);
-    return merge_t<false>(s, (const uint32_t*)in, n, select_mask, select, time_window, (uint32_t*)out, num_out);
+                 float time_window, void* out, long long* num_out, Workspace& ws) {
+    if (lite) return merge_t<true>(s, (const uint32_t*)in, n, select_mask, select, time_window, (uint32_t*)out, num_out, ws);
+    return merge_t<false>(s, (const uint32_t*)in, n, select_mask, select, time_window, (uint32_t*)out, num_out, ws);
 }
 
 } // namespace oxl

@@ -146,6 +146,8 @@ struct Server {
     oxr_server_config cfg{};
     std::thread th;
     std::mutex mu;
+    std::mutex copy_mu;              // who holds it may use the helper threads
+    CopyPool copies;
     std::condition_variable cv_work, cv_done;
     std::deque<std::unique_ptr<Req>> incoming;
     std::vector<std::unique_ptr<Req>> active;
@@ -617,37 +619,23 @@ int oxr_server_take_hits(oxr_server* sh, int64_t id, void* dst, int64_t cap, int
         r = std::move(it->second);
         s->finished.erase(it);
     }
-    // the hits reached pinned host memory before the request completed: a host copy,
-    // no device work on the caller's thread; large ones split over a few threads (one
-    // thread copies at about a third of what the memory system delivers)
-    struct Piece { const char* src; char* dst; size_t n; };
-    std::vector<Piece> pieces;
-    char* o = static_cast<char*>(dst);
+    // the hits reached pinned host memory before the request completed: a host copy, no
+    // device work on the caller's thread. Large ones are split over the kept helper threads
+    // (one thread copies at about a third of what the memory system delivers), unless another
+    // caller is using them.
     size_t total = 0;
+    for (auto& h : r->hits) total += size_t(h.n) * 64;
+    std::unique_lock<std::mutex> helpers(s->copy_mu, std::defer_lock);
+    const bool helped = total >= (size_t(1) << 20) && helpers.try_lock();
+    if (helped) s->copies.begin();
+    char* o = static_cast<char*>(dst);
     for (auto& h : r->hits) {
-        pieces.push_back({static_cast<const char*>(h.blk->p) + size_t(h.first) * 64, o, size_t(h.n) * 64});
+        const char* src = static_cast<const char*>(h.blk->p) + size_t(h.first) * 64;
+        if (helped) s->copies.copy(o, src, size_t(h.n) * 64);
+        else std::memcpy(o, src, size_t(h.n) * 64);
         o += size_t(h.n) * 64;
-        total += size_t(h.n) * 64;
     }
-    const size_t SPLIT = size_t(16) << 20;
-    int nt = int(std::min<size_t>(8, total / SPLIT));
-    if (nt <= 1) {
-        for (auto& p : pieces) std::memcpy(p.dst, p.src, p.n);
-    } else {
-        // thread t copies bytes [t*total/nt, (t+1)*total/nt) of the concatenated pieces
-        auto work = [&](int t) {
-            size_t b = total * size_t(t) / size_t(nt), e = total * size_t(t + 1) / size_t(nt), at = 0;
-            for (auto& p : pieces) {
-                size_t lo = std::max(b, at), hi = std::min(e, at + p.n);
-                if (lo < hi) std::memcpy(p.dst + (lo - at), p.src + (lo - at), hi - lo);
-                at += p.n;
-            }
-        };
-        std::vector<std::thread> th;
-        for (int t = 1; t < nt; t++) th.emplace_back(work, t);
-        work(0);
-        for (auto& x : th) x.join();
-    }
+    if (helped) s->copies.end();
     r->hits.clear();
     return OXR_OK;
 }
