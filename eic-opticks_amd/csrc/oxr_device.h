@@ -304,18 +304,21 @@ OXD TexX tex_x(const Tables& t, float nm) {
     X.a = xf - fl;
     X.b = 1.0f - X.a;
     int i0 = int(fl);
-    X.m0 = i0 % nx; if (X.m0 < 0) X.m0 += nx;
+    if (unsigned(i0) >= unsigned(nx)) {   // beyond the table: wrap round (the remainder is 30 instructions)
+        i0 %= nx;
+        if (i0 < 0) i0 += nx;
+    }
+    X.m0 = i0;
     X.m1 = X.m0 + 1; if (X.m1 == nx) X.m1 = 0;
     return X;
 }
-OXD float4 boundary_fetch(const Tables& t, const TexX& X, unsigned line, unsigned k) {
-    const float4* row = t.bnd + size_t(2u * line + k) * t.num_wl;
-    float4 v0 = row[X.m0], v1 = row[X.m1];
+OXD float4 boundary_fetch(const float4* row, const TexX& X) {
+    float4 v0 = row[unsigned(X.m0)], v1 = row[unsigned(X.m1)];
     const float a = X.a, b = X.b;
     return make_float4(b * v0.x + a * v1.x, b * v0.y + a * v1.y, b * v0.z + a * v1.z, b * v0.w + a * v1.w);
 }
 OXD float4 boundary_lookup(const Tables& t, float nm, unsigned line, unsigned k) {
-    return boundary_fetch(t, tex_x(t, nm), line, k);
+    return boundary_fetch(t.bnd + size_t(2u * line + k) * unsigned(t.num_wl), tex_x(t, nm));
 }
 
 OXD float icdf_lookup(const Tables& t, float x, int row) {

@@ -117,16 +117,18 @@ constexpr int MAX_REJECT = 10000;
 
 // qbnd::fill_state (qudarap/qbnd.h:184-214)
 OXD void fill_state(const Tables& t, St& s, unsigned boundary, float wl, float cosTheta) {
-    int line = int(boundary) * 4;
-    int m1 = cosTheta > 0.f ? line + 3 : line + 0;
-    int m2 = cosTheta > 0.f ? line + 0 : line + 3;
-    int su = cosTheta > 0.f ? line + 2 : line + 1;
+    // a boundary's lines: 0 outer material, 1 outer surface, 2 inner surface, 3 inner material,
+    // two rows each; one product for the four rows
+    const bool out = cosTheta > 0.f;
+    const unsigned nw = unsigned(t.num_wl);
+    const float4* first = t.bnd + size_t(boundary * 8u) * nw;
+    const unsigned m1 = out ? 6u * nw : 0u, m2 = out ? 0u : 6u * nw, su = out ? 4u * nw : 2u * nw;
     const TexX X = tex_x(t, wl);   // one wavelength coordinate for the four rows
-    s.m1 = boundary_fetch(t, X, m1, 0);
-    s.m1g2 = boundary_fetch(t, X, m1, 1);
-    s.m2 = boundary_fetch(t, X, m2, 0);
-    s.su = boundary_fetch(t, X, su, 0);
-    s.opt = t.optical[su];
+    s.m1 = boundary_fetch(first + m1, X);
+    s.m1g2 = boundary_fetch(first + (m1 + nw), X);
+    s.m2 = boundary_fetch(first + m2, X);
+    s.su = boundary_fetch(first + su, X);
+    s.opt = t.optical[boundary * 4u + (out ? 2u : 1u)];
 }
 
 // qsim::uniform_sphere (qudarap/qsim.h:177-183)
@@ -360,8 +362,7 @@ OXD int propagate(Ph& p, const Hit& h, f3 normal, Rng& r, const Tables& t, int a
     if (command == BOUNDARY) {
         int ems = int(s.opt.y);
         if (ems == 1) command = propagate_at_boundary(flag, p, s, normal, r, d, aligned);
-        else if (ems == 2) command = propagate_at_surface(flag, p, s, normal, r, d, aligned);
-        else if (lpos_cost(h.lpos) < 0.f) command = propagate_at_surface(flag, p, s, normal, r, d, aligned);
+        else if (ems == 2 || lpos_cost(h.lpos) < 0.f) command = propagate_at_surface(flag, p, s, normal, r, d, aligned);
         else if (ems == 3) { advance(r, 1); keep(r, d.w3, d.w4, d.w5); flag = SURFACE_DETECT; command = BREAK; }
     }
     set_flag(p, flag);
@@ -385,14 +386,22 @@ OXG void gen_torch(Ph& p, const float4* gs, uint64_t photon_id, Rng& r) {
         if (type == 8) { advance(r, 3); keep(r, d.w3, d.w4, d.w5); }
         else { advance(r, 2); keep(r, d.w2, d.w3, d.w4); }
     }
-    float sinPhi, cosPhi;
+    // One call for the angle of types 1, 4, 7 and 8, one for the phase of types 6, 7 and 8:
+    // with the library's fallback inlined at each of five places the refill step was 40 KB
+    // long, and a kernel's first photons wait for these instructions to be fetched.
+    float sinPhi = 0.f, cosPhi = 0.f;
+    if (type == 1 || type == 4 || type == 7 || type == 8) {
+        float frac = type == 8 ? u0 : ax + u1 * (ay - ax);
+        if (type == 4) {
+            float f = float(photon_id) / float(numphoton);
+            frac = ax * (1.f - f) + ay * f;
+        }
+        xsincos(TWOPI * frac, sinPhi, cosPhi);
+    }
     if (type == 1) {
         p.mom = gmom;
         float u_zenith = zx + u0 * (zy - zx);
-        float u_azimuth = ax + u1 * (ay - ax);
         float rr = radius * u_zenith;
-        float phi = TWOPI * u_azimuth;
-        xsincos(phi, sinPhi, cosPhi);
         p.pos = mk(rr * cosPhi, rr * sinPhi, 0.f);
         rotateUz(p.pos, p.mom);
         p.pos = add(p.pos, gpos);
@@ -400,19 +409,12 @@ OXG void gen_torch(Ph& p, const float4* gs, uint64_t photon_id, Rng& r) {
         rotateUz(p.pol, p.mom);
     } else if (type == 7) {
         float u_zenith = zx + u0 * (zy - zx);
-        float u_azimuth = ax + u1 * (ay - ax);
-        float phi = TWOPI * u_azimuth;
-        xsincos(phi, sinPhi, cosPhi);
         float cosTheta = 1.f - 2.f * u_zenith;
         float sinTheta = sqrtf(1.f - cosTheta * cosTheta);
         float flip = copysignf(1.f, radius);
         p.mom = mk(flip * sinTheta * cosPhi, flip * sinTheta * sinPhi, flip * cosTheta);
         float rad = fabsf(radius);
         p.pos = mk(sinTheta * cosPhi * rad, sinTheta * sinPhi * rad, cosTheta * rad);
-        float phase = TWOPI * distance;
-        xsincos(phase, sinPhi, cosPhi);
-        p.pol = mk(cosPhi, sinPhi, 0.f);
-        rotateUz(p.pol, p.mom);
     } else if (type == 6) {
         float u0z, u1a, u, v, b, a;
         int turns = 0;
@@ -430,10 +432,6 @@ OXG void gen_torch(Ph& p, const float4* gs, uint64_t photon_id, Rng& r) {
         float flip = copysignf(1.f, radius);
         p.mom = mk(flip * a * u, flip * a * v, flip * (2.f * b - 1.f));
         p.pos = mk(a * u * rad, a * v * rad, (2.f * b - 1.f) * rad);
-        float phase = TWOPI * distance;
-        xsincos(phase, sinPhi, cosPhi);
-        p.pol = mk(cosPhi, sinPhi, 0.f);
-        rotateUz(p.pol, p.mom);
     } else if (type == 2) {
         p.mom = gmom;
         float frac = float(photon_id) / float(numphoton);
@@ -452,10 +450,6 @@ OXG void gen_torch(Ph& p, const float4* gs, uint64_t photon_id, Rng& r) {
         p.pol = mk(0.f, -1.f, 0.f);
         rotateUz(p.pol, p.mom);
     } else if (type == 4) {
-        float f = float(photon_id) / float(numphoton);
-        float frac = ax * (1.f - f) + ay * f;
-        float phi = TWOPI * frac;
-        xsincos(phi, sinPhi, cosPhi);
         float rr = radius < 0.f ? -radius : radius;
         p.mom = mk(radius < 0.f ? -cosPhi : cosPhi, 0.f, radius < 0.f ? -sinPhi : sinPhi);
         p.pos = mk(rr * cosPhi, 0.f, rr * sinPhi);
@@ -478,14 +472,13 @@ OXG void gen_torch(Ph& p, const float4* gs, uint64_t photon_id, Rng& r) {
         p.pol = mk(0.f, -1.f, 0.f);
         rotateUz(p.pol, p.mom);
     } else if (type == 8) {
-        float phi = TWOPI * u0;
         float cosTheta = 1.f - 2.f * u1;
         float sinTheta = sqrtf(1.f - cosTheta * cosTheta);
-        sincos_bounded(phi, sinPhi, cosPhi);
         p.mom = mk(sinTheta * cosPhi, sinTheta * sinPhi, cosTheta);
         p.pos = gpos;
-        float phase = TWOPI * u2;
-        sincos_bounded(phase, sinPhi, cosPhi);
+    }
+    if (type == 6 || type == 7 || type == 8) {
+        xsincos(TWOPI * (type == 8 ? u2 : distance), sinPhi, cosPhi);
         p.pol = mk(cosPhi, sinPhi, 0.f);
         rotateUz(p.pol, p.mom);
     }
