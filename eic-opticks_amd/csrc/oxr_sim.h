@@ -3,18 +3,17 @@
 // support (LIST) and the traversal mode TM (bit 0: stack entries carry box entry distances;
 // bit 1: the flattened BVH; bit 2: every CSG tree has height <= 2, so the CSG evaluation
 // stacks live in registers, production kernels without list nodes only; bit 3: nodes also
-// cull by their radial bounds, production and counting kernels). k_generate (oxr_kernels.hip) uses the per-photon pieces; the
-// kernels are instantiated by the four oxr_sim_*.hip units, one per (FP64, LIST) pair, which
-// compile in parallel.
+// cull by their radial bounds, production and counting kernels). k_generate
+// (oxr_kernels.hip) uses the per-photon pieces; the kernels are instantiated by the
+// oxr_sim_*.hip units, one per (FP64, LIST) pair and two for simple leaves, which compile in
+// parallel.
 #pragma once
 #include "oxr_kernels.h"
 
-
 // Minimum waves per SIMD the simulate kernels are compiled for (VGPR budget 512/N per
-// lane). The latency-bound traversal wants occupancy more than registers: measured on
-// MI355X (crystal-calorimeter event), 4 waves beat 3 and 5 for both forms; with the
-// simple-leaf kernels 5 waves lost on every event (instanced CSG 11.4 against 8.8 ms), and
-// with the CSG arrays in LDS 3 waves lost too (instanced CSG 9.0 against 7.9 ms).
+// lane). 4 beat 3 and 5 on MI355X: with 5 the spilled registers cost more than the wave
+// brings (instanced CSG 11.0 against 8.5 ms), with 3 the loop waits more for memory (thin
+// shells 20.0 against 17.5 ms; with FP64 roots 3 waves are 2% faster).
 #ifndef OXR_PERSIST_WAVES
 #define OXR_PERSIST_WAVES 4
 #endif
