@@ -1,7 +1,8 @@
 """The hits of a launch are its photons with the mask's bits, in photon order, at the edges of
 what the selection and the copies work in: 4096 photons a workgroup, 1024 hits written straight
-to the host, 1 MB (16384 photons) a copy in one piece, 2 MB without helpers, four slots of 2 MB. One engine takes
-all sizes in turn, so each launch follows one that left other counts behind."""
+to the host, 1 MB (16384 photons) a copy in one piece, 2 MB without helpers, four slots of
+2 MB. One engine takes all sizes in turn, so each launch follows one that left other counts
+behind."""
 import numpy as np
 import pytest
 
