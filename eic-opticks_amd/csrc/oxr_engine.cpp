@@ -40,6 +40,7 @@ oxd::Geom Engine::geom() const {
     g.tlas_root = f ? tlas_root_f : tlas_root; g.num_inst = num_inst;
     g.vizmask = cfg.vizmask;
     g.rad = f ? rad_flat.p : rad_tlas.p;
+    g.far_extent = far_extent; g.far_scale = far_scale;
     return g;
 }
 
@@ -449,10 +450,13 @@ static std::vector<float4> device_nodes(const oxr_geometry* g, std::vector<int2>
 // its rays. reach is the longest distance from a ray's origin to anything in the scene: a
 // quadric's discriminant in single precision is off by at most 16 ulps of its square, so a ray
 // may be reported to hit a sphere or cylinder up to sqrt(r^2 + 2e-6 reach^2) from its axis
-// (twice that bound), and the boxes take that radius.
+// (twice that bound), and the boxes take that radius. A ray from further away than the scene
+// is wide widens the boxes as it meets them (far_pad, oxr_trace.h): stretch is the most that
+// a distance in the world grows by on its way into a leaf's frame and its margin back, the
+// longest column of the leaf's transform times the norm of its inverse.
 // Instanced CSG, 10M photons: 7.7 -> 6.1 ms; 200k photons 540 -> 466 us; the served stream of 24
 // events 9.5 -> 7.9 ms.
-static bool leaf_box(const oxr_geometry* g, int64_t ni, const double A[4][3], double reach, Box& out) {
+static bool leaf_box(const oxr_geometry* g, int64_t ni, const double A[4][3], double reach, Box& out, double& stretch) {
     const float* q = g->node + 16 * ni;
     const uint32_t tc = fbits(q[14]), gt = fbits(q[15]) & 0x7fffffffu;
     if (tc != 101u && tc != 103u && tc != 105u && tc != 110u) return false;
@@ -474,6 +478,8 @@ static bool leaf_box(const oxr_geometry* g, int64_t ni, const double A[4][3], do
     for (int r = 0; r < 3; r++) for (int k = 0; k < 3; k++) norm2 += I[r][k] * I[r][k];
     const double far = reach * std::sqrt(norm2);   // the reach in the leaf's frame
     if (!std::isfinite(far)) return false;
+    for (int k = 0; k < 3; k++)
+        stretch = std::max(stretch, std::sqrt(norm2 * (M[0][k] * M[0][k] + M[1][k] * M[1][k] + M[2][k] * M[2][k])));
     const double flat = 16.0 * 6e-8 * far;         // planes: a few ulps of the distance
     auto map = [&](double x, double y, double z, double* w) {
         for (int k = 0; k < 3; k++) w[k] = x * M[0][k] + y * M[1][k] + z * M[2][k] + M[3][k];
@@ -517,7 +523,7 @@ static bool leaf_box(const oxr_geometry* g, int64_t ni, const double A[4][3], do
 }
 
 // b: the prim's object box turned into the world; cut to the leaves' box where that is known
-static void tighten(const oxr_geometry* g, int64_t prim, const float* inst, double reach, Box& b) {
+static void tighten(const oxr_geometry* g, int64_t prim, const float* inst, double reach, Box& b, double& stretch) {
     int32_t numNode, nodeOffset;
     std::memcpy(&numNode, g->prim + 16 * prim, 4);
     std::memcpy(&nodeOffset, g->prim + 16 * prim + 1, 4);
@@ -532,7 +538,7 @@ static void tighten(const oxr_geometry* g, int64_t prim, const float* inst, doub
         const uint32_t tc = fbits(g->node[16 * (nodeOffset + i) + 14]);
         if (tc == 0u || is_op(tc)) continue;
         Box lb;
-        if (!leaf_box(g, nodeOffset + i, A, reach, lb)) return;
+        if (!leaf_box(g, nodeOffset + i, A, reach, lb, stretch)) return;
         all.grow(lb);
     }
     Box cut = b;
@@ -744,6 +750,7 @@ int oxr_engine_create(const oxr_geometry* g, const oxr_physics* ph, const oxr_co
     }
     // the world box of prim p of solid gas placed by q
     const double reach = 2.0 * std::sqrt(3.0) * W;
+    double stretch = 1.0;
     auto placed_box = [&](const float* q, int32_t gas, size_t p) -> oxh::Box {
         const oxh::Box& ob = prim_boxes[size_t(gas)][p];
         oxh::Box wb = oxh::Box::empty();
@@ -753,7 +760,7 @@ int oxr_engine_create(const oxr_geometry* g, const oxr_physics* ph, const oxr_co
             for (int k = 0; k < 3; k++) w[k] = pt[0] * q[k] + pt[1] * q[4 + k] + pt[2] * q[8 + k] + q[12 + k];
             wb.grow_point(w);
         }
-        tighten(g, e->solid_prim_offset[size_t(gas)] + int64_t(p), q, reach, wb);
+        tighten(g, e->solid_prim_offset[size_t(gas)] + int64_t(p), q, reach, wb, stretch);
         return wb;
     };
     // ---- instances and TLAS
@@ -865,6 +872,8 @@ int oxr_engine_create(const oxr_geometry* g, const oxr_physics* ph, const oxr_co
         int32_t gas; std::memcpy(&gas, g->inst + 16 * i + 7, 4);
         insts[size_t(i)].info.w = e->solid_blas_root[size_t(gas)];
     }
+    e->far_extent = float(0.5 * reach);
+    e->far_scale = float(1.5e-3 * stretch);   // sqrt(2e-6) for the quadrics, the rest for the planes (flat)
     tl.nodes.insert(tl.nodes.end(), blas_all.begin(), blas_all.end());
     tl.rad.insert(tl.rad.end(), rad_blas.begin(), rad_blas.end());
     if (e->stack_cap() > 96) return bail(fail(OXR_EINVAL, "BVH too deep for the traversal stack"));

@@ -105,6 +105,7 @@ struct Engine {
     int64_t top_nodes() const { return top_nodes(tune); }
     DBuf<uint4> optical;
     DBuf<float> icdf;
+    float far_extent = 0.f, far_scale = 0.f;   // oxd::far_pad
     int tlas_root = 0;
     int num_inst = 0, num_solid = 0, num_prim = 0, num_node = 0, num_itra = 0;
     int dev_nodes = 0;       // nodes on the device: num_node and the copies of shared trees (device_nodes)

@@ -293,6 +293,9 @@ OXD void run_wave(const Params& P, int* stk, int stride, const BNode* top) {
     TraceCount cnt = {0, 0, 0, 0};
     v.cur = TRAV_IDLE;
     bool first = true, drained = false;
+    // A photon of the wave started outside the scene (far_pad): a bounce takes it to a surface,
+    // inside, or so little beyond that the stored margins, twice the errors' bound, hold it.
+    bool far_wave = false;
     unsigned long long pool = 0;   // photons the wave has claimed and not yet started: [pool, pool + pooled)
     int pooled = 0;
     for (;;) {
@@ -301,13 +304,17 @@ OXD void run_wave(const Params& P, int* stk, int stride, const BNode* top) {
         const int nend = __popcll(__ballot(v.cur == TRAV_DONE));
         const int least = max(1, ((nnode + nleaf + nend) * (!REFILL ? NODE_LEAST_PLAIN : RADIAL ? NODE_LEAST_RADIAL : NODE_LEAST)) >> 6);   // lanes that keep the nodes running
         if (nnode >= least) {
-            RayF r;
             const f3 org = P.refine ? ray_origin(L.p.pos, L.p.mom, t_approx) : L.p.pos;
-            if (at_node(v)) ray_of<FLAT, RADIAL>(r, g, v, org, L.p.mom);
-            do {
-                if (at_node(v)) trav_node<COUNT, TN, FLAT, RADIAL>(v, g, r, org, L.p.mom, stk, stride, P.stack_cap, top, P.ntop, err, cnt);
-                nnode = __popcll(__ballot(at_node(v)));
-            } while (nnode >= least);
+            auto visit = [&](auto r) __attribute__((always_inline)) {
+                if (at_node(v)) ray_of<FLAT, RADIAL>(r, g, v, org, L.p.mom);
+                do {
+                    if (at_node(v)) trav_node<COUNT, TN, FLAT, RADIAL>(v, g, r, org, L.p.mom, stk, stride, P.stack_cap, top, P.ntop, err, cnt);
+                    nnode = __popcll(__ballot(at_node(v)));
+                } while (nnode >= least);
+            };
+            // in a loop of its own: one for both takes three registers more and 1-4% on every event
+            if (__builtin_expect(far_wave, 0)) visit(RayF<true>());
+            else visit(RayF<false>());
             continue;
         }
         if (nleaf > 0 && nleaf * (REFILL ? LEAF_WEIGHT : LEAF_WEIGHT_PLAIN) >= nend) {
@@ -336,6 +343,7 @@ OXD void run_wave(const Params& P, int* stk, int stride, const BNode* top) {
         }
         const uint64_t idle = __ballot(v.cur == TRAV_IDLE);
         const int nidle = __popcll(idle);
+        if (far_wave) far_wave = __ballot(v.cur != TRAV_IDLE && far_away(g, L.p.pos)) != 0ull;
         if (drained) {
             if (nidle == 64) break;
             continue;
@@ -380,6 +388,7 @@ OXD void run_wave(const Params& P, int* stk, int stride, const BNode* top) {
                     P.hitflag[pi] = 0;
                 }
             }
+            far_wave = __ballot(v.cur != TRAV_IDLE && far_away(g, L.p.pos)) != 0ull;
         }
     }
     flush_counters(P, steps, cnt.visits, cnt.tests, err, COUNT, cnt.csgb, cnt.ivis);

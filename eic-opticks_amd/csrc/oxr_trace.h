@@ -59,6 +59,8 @@ struct Geom {
     unsigned vizmask;      // ray visibility mask against InstD flag bits 8-15
     // radial bounds, two float4 per node of tlas {centre, (r_in0, r_out0, r_in1, r_out1)}
     const float4* rad;
+    // far_pad's: half the reach that the world boxes hold, and the pad per distance beyond it
+    float far_extent, far_scale;
 };
 
 struct Hit {
@@ -79,11 +81,23 @@ OXD f3 safe_inv(f3 d) {
               __builtin_amdgcn_rcpf(fabsf(d.z) > e ? d.z : copysignf(e, d.z)));
 }
 OXD f3 neg_oi(f3 o, f3 inv) { return mk(-(o.x * inv.x), -(o.y * inv.y), -(o.z * inv.z)); }
-// slab test of one child box (noi = -origin*inv)
-OXD bool box_hit(float lx, float ly, float lz, float hx, float hy, float hz, f3 noi, f3 inv, float tbest, float& tn) {
-    float tx0 = fmaf(lx, inv.x, noi.x), tx1 = fmaf(hx, inv.x, noi.x);
-    float ty0 = fmaf(ly, inv.y, noi.y), ty1 = fmaf(hy, inv.y, noi.y);
-    float tz0 = fmaf(lz, inv.z, noi.z), tz1 = fmaf(hz, inv.z, noi.z);
+// The world boxes of quadrics hold what their single-precision tests may report from origins
+// within the scene (tighten, oxr_engine.cpp). The error of a test grows with the origin's
+// distance D: from outside, a box has to reach sqrt(2e-6 (D^2 - reach^2)) further, times the
+// worst stretch of a leaf's transform, than the margin it was stored with. Nothing is added
+// for an origin within the scene.
+OXD bool far_away(const Geom& g, f3 pos) { return dot(pos, pos) > g.far_extent * g.far_extent; }
+OXD float far_pad(const Geom& g, f3 pos) {
+    const float dist = __builtin_amdgcn_sqrtf(dot(pos, pos)) + g.far_extent;
+    const float over = fmaf(dist, dist, -4.f * g.far_extent * g.far_extent);
+    return over > 0.f ? g.far_scale * __builtin_amdgcn_sqrtf(over) : 0.f;
+}
+// slab test of one child box (noi_lo, noi_hi: -origin*inv for its low and high planes, which
+// differ by what the box is widened by)
+OXD bool box_hit(float lx, float ly, float lz, float hx, float hy, float hz, f3 noi_lo, f3 noi_hi, f3 inv, float tbest, float& tn) {
+    float tx0 = fmaf(lx, inv.x, noi_lo.x), tx1 = fmaf(hx, inv.x, noi_hi.x);
+    float ty0 = fmaf(ly, inv.y, noi_lo.y), ty1 = fmaf(hy, inv.y, noi_hi.y);
+    float tz0 = fmaf(lz, inv.z, noi_lo.z), tz1 = fmaf(hz, inv.z, noi_hi.z);
     float n = fmaxf(fmaxf(fminf(tx0, tx1), fminf(ty0, ty1)), fminf(tz0, tz1));
     float f = fminf(fminf(fmaxf(tx0, tx1), fmaxf(ty0, ty1)), fmaxf(tz0, tz1));
     tn = n;
@@ -158,19 +172,42 @@ OXD void trav_begin(Trav& v, const Geom& g, float tmax, int* stk, int stride, in
 }
 
 // the ray in the frame of the current tree, and what the slab tests need of it
-struct RayF { f3 o, inv, noi; float ilen; };
-template <bool RADIAL>
-OXD void ray_frame(RayF& r, f3 o, f3 d) {
+// WIDE: the world boxes are widened for origins outside the scene (far_pad); the high planes
+// then have their own product, and a radial bound lies off, sqrt(3) of the pad, nearer
+template <bool WIDE> struct RayF {
+    f3 o, inv, noi;
+    float ilen;
+    OXD f3 noi_high() const { return noi; }
+    OXD float bound(float x) const { return x * ilen; }
+    OXD void widen(float) {}
+};
+template <> struct RayF<true> {
+    f3 o, inv, noi, noi_hi;
+    float ilen, off;
+    OXD f3 noi_high() const { return noi_hi; }
+    OXD float bound(float x) const { return fmaf(x, ilen, -off); }
+    OXD void widen(float pad) {
+        noi_hi = mk(fmaf(pad, inv.x, noi.x), fmaf(pad, inv.y, noi.y), fmaf(pad, inv.z, noi.z));
+        noi = mk(fmaf(-pad, inv.x, noi.x), fmaf(-pad, inv.y, noi.y), fmaf(-pad, inv.z, noi.z));
+        off = 1.7321f * pad * ilen;
+    }
+};
+template <bool RADIAL, bool WIDE>
+OXD void ray_frame(RayF<WIDE>& r, f3 o, f3 d, float pad) {
     r.o = o;
     r.inv = safe_inv(d);
     r.noi = neg_oi(o, r.inv);
     r.ilen = RADIAL ? __builtin_amdgcn_rsqf(dot(d, d)) : 1.f;
+    r.widen(pad);
 }
-template <bool FLAT, bool RADIAL>
-OXD void ray_of(RayF& r, const Geom& g, const Trav& v, f3 pos, f3 mom) {
+template <bool RADIAL, bool WIDE>
+OXD void ray_world(RayF<WIDE>& r, const Geom& g, f3 pos, f3 mom) { ray_frame<RADIAL>(r, pos, mom, WIDE ? far_pad(g, pos) : 0.f); }
+template <bool FLAT, bool RADIAL, bool WIDE>
+OXD void ray_of(RayF<WIDE>& r, const Geom& g, const Trav& v, f3 pos, f3 mom) {
     f3 o = pos, d = mom;
-    if (!FLAT && v.inst >= 0 && !(v.inst & INST_IDENT)) to_object(g.inst[v.inst], pos, mom, o, d);
-    ray_frame<RADIAL>(r, o, d);
+    const bool world = FLAT || v.inst < 0 || (v.inst & INST_IDENT) != 0;
+    if (!world) to_object(g.inst[v.inst], pos, mom, o, d);
+    ray_frame<RADIAL>(r, o, d, WIDE && world ? far_pad(g, pos) : 0.f);
 }
 
 // the next stack entry worth visiting; the first one is the end mark
@@ -186,8 +223,8 @@ OXD void trav_pop(Trav& v, const int* stk, int stride, int cap) {
 
 struct TraceCount { uint32_t visits, tests, csgb, ivis; };
 
-template <bool COUNT, bool TN, bool FLAT, bool RADIAL>
-OXD void trav_node(Trav& v, const Geom& g, RayF& r, f3 pos, f3 mom, int* stk, int stride, int cap, const BNode* top, int ntop,
+template <bool COUNT, bool TN, bool FLAT, bool RADIAL, bool WIDE>
+OXD void trav_node(Trav& v, const Geom& g, RayF<WIDE>& r, f3 pos, f3 mom, int* stk, int stride, int cap, const BNode* top, int ntop,
                    uint32_t& err, TraceCount& cnt) {
     float* stkt = reinterpret_cast<float*>(stk + stride * cap);
     if (FLAT || v.cur < INST_LEAVES) {
@@ -201,13 +238,13 @@ OXD void trav_node(Trav& v, const Geom& g, RayF& r, f3 pos, f3 mom, int* stk, in
         else nd = g.tlas[cur];
         if (COUNT) cnt.visits++;
         float tn0, tn1;
-        bool h0 = box_hit(nd.a.x, nd.a.y, nd.a.z, nd.a.w, nd.b.x, nd.b.y, r.noi, r.inv, v.best, tn0);
-        bool h1 = box_hit(nd.b.z, nd.b.w, nd.c.x, nd.c.y, nd.c.z, nd.c.w, r.noi, r.inv, v.best, tn1);
+        bool h0 = box_hit(nd.a.x, nd.a.y, nd.a.z, nd.a.w, nd.b.x, nd.b.y, r.noi, r.noi_high(), r.inv, v.best, tn0);
+        bool h1 = box_hit(nd.b.z, nd.b.w, nd.c.x, nd.c.y, nd.c.z, nd.c.w, r.noi, r.noi_high(), r.inv, v.best, tn1);
         if (RADIAL) {
             const float dx = r.o.x - rc.x, dy = r.o.y - rc.y, dz = r.o.z - rc.z;
             const float dist = __builtin_amdgcn_sqrtf(dx * dx + dy * dy + dz * dz);
-            const float lb0 = fmaxf(rr.x - dist, dist - rr.y) * r.ilen;
-            const float lb1 = fmaxf(rr.z - dist, dist - rr.w) * r.ilen;
+            const float lb0 = r.bound(fmaxf(rr.x - dist, dist - rr.y));
+            const float lb1 = r.bound(fmaxf(rr.z - dist, dist - rr.w));
             h0 = h0 && lb0 <= v.best;
             h1 = h1 && lb1 <= v.best;
             tn0 = fmaxf(tn0, lb0);
@@ -233,7 +270,7 @@ OXD void trav_node(Trav& v, const Geom& g, RayF& r, f3 pos, f3 mom, int* stk, in
     if constexpr (!FLAT) {
         if (v.cur == TRAV_BACK) {      // the instance's tree is done: back to the world frame
             v.inst = -1;
-            ray_frame<RADIAL>(r, pos, mom);
+            ray_world<RADIAL>(r, g, pos, mom);
             trav_pop<TN>(v, stk, stride, cap);
             return;
         }
@@ -249,7 +286,7 @@ OXD void trav_node(Trav& v, const Geom& g, RayF& r, f3 pos, f3 mom, int* stk, in
         if (!ident) {
             f3 o, d;
             to_object(in, pos, mom, o, d);
-            ray_frame<RADIAL>(r, o, d);
+            ray_frame<RADIAL>(r, o, d, 0.f);
         }
         if (v.sp < stride * cap) {
             stk[v.sp] = int(TRAV_BACK);
@@ -342,11 +379,11 @@ template <bool FP64, bool LIST, bool FLAT>
 OXD bool trace(const Geom& g, f3 pos, f3 mom, float tmin, float tmax, Hit& hit, int* stk, int stride, int cap,
                const BNode* top, int ntop) {
     Trav v;
-    RayF r;
+    RayF<true> r;
     TraceCount cnt;
     uint32_t err = 0;
     trav_begin(v, g, tmax, stk, stride, cap, false);
-    ray_frame<false>(r, pos, mom);
+    ray_world<false>(r, g, pos, mom);
     while (v.cur != TRAV_DONE) {
         if (at_leaf(v)) trav_leaf<FP64, false, LIST, false, FLAT, false, false>(v, g, pos, mom, tmin, stk, stride, cap, cnt);
         else trav_node<false, false, FLAT, false>(v, g, r, pos, mom, stk, stride, cap, top, ntop, err, cnt);
