@@ -9,6 +9,7 @@
 // parallel.
 #pragma once
 #include "oxr_kernels.h"
+#include "oxr_steps.h"
 
 // Minimum waves per SIMD the simulate kernels are compiled for (VGPR budget 512/N per
 // lane). 4 beat 3 and 5 on MI355X: with 5 the spilled registers cost more than the wave
@@ -336,7 +337,7 @@ OXD void run_wave(const Params& P, int* stk, int stride, const BNode* top) {
                     trav_begin(v, g, P.tmax, stk, stride, P.stack_cap, TN);
                 } else {
                     end_photon<DBG>(P, L);
-                    steps += uint32_t(L.bounce);
+                    add_steps(steps, L.bounce, [&](uint32_t n) { atomicAdd(P.counters + 0, (unsigned long long)n); });
                     v.cur = TRAV_IDLE;
                 }
             }
