@@ -5,84 +5,6 @@
 
 namespace oxh {
 
-CopyPool::~CopyPool() {
-    {
-        std::lock_guard<std::mutex> lk(mu_);
-        stop_ = true;
-    }
-    cv_.notify_all();
-    for (auto& t : threads_) t.join();
-}
-
-void CopyPool::begin() {
-    if (!started_) {
-        started_ = true;
-        try {
-            for (int k = 0; k < HELPERS; k++) threads_.emplace_back([this] { run(); });
-        } catch (...) {   // no thread to be had: the caller copies alone (or with those that started)
-        }
-    }
-    {
-        std::lock_guard<std::mutex> lk(mu_);
-        busy_ = true;
-    }
-    cv_.notify_all();
-}
-
-void CopyPool::end() { busy_ = false; }
-
-void CopyPool::run() {
-    unsigned seen = 0;
-    for (;;) {
-        {
-            std::unique_lock<std::mutex> lk(mu_);
-            cv_.wait(lk, [&] { return stop_ || busy_; });
-            if (stop_) return;
-        }
-        while (busy_ && !stop_) {
-            if (job_.load() == seen) {
-                __builtin_ia32_pause();
-                continue;
-            }
-            inside_.fetch_add(1);
-            seen = job_.load();
-            take_parts();
-            inside_.fetch_sub(1);
-        }
-    }
-}
-
-// parts are claimed one by one, so a helper that wakes late finds none left
-void CopyPool::take_parts() {
-    for (;;) {
-        const int k = next_.fetch_add(1), parts = parts_.load();
-        if (k >= parts) return;
-        const size_t step = (bytes_ / size_t(parts)) & ~size_t(63);
-        const size_t at = step * size_t(k), n = k == parts - 1 ? bytes_ - at : step;
-        std::memcpy(dst_ + at, src_ + at, n);
-        left_.fetch_sub(1);
-    }
-}
-
-void CopyPool::copy(char* dst, const char* src, size_t bytes) {
-    if (!busy_ || threads_.empty() || bytes < (size_t(256) << 10)) {
-        std::memcpy(dst, src, bytes);
-        return;
-    }
-    // The fields are rewritten only when no helper reads them: all parts of the last job are
-    // taken, and a helper that comes in meanwhile finds none until next_ starts again below.
-    next_.store(1 << 20);
-    while (inside_.load() != 0) {}
-    dst_ = dst; src_ = src; bytes_ = bytes;
-    const int parts = 2 * (int(threads_.size()) + 1);
-    parts_.store(parts);
-    left_.store(parts);
-    next_.store(0);
-    job_.fetch_add(1);
-    take_parts();
-    while (left_.load() > 0) {}
-}
-
 hipError_t Stager::ready(size_t bytes) {
     hipError_t e;
     for (int k = 0; k < SLOTS; k++)

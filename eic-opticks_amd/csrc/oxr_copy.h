@@ -8,41 +8,9 @@
 // helpers, whose waking costs more than they bring (512 KB: 121 us with them, 76 without).
 #pragma once
 #include <hip/hip_runtime.h>
-#include <atomic>
-#include <condition_variable>
-#include <mutex>
-#include <thread>
-#include <vector>
+#include "oxr_pool.h"
 
 namespace oxh {
-
-// Helper threads for host copies, started by the first large one and joined with the owner.
-// One copy() at a time (the engine's lock).
-class CopyPool {
-public:
-    ~CopyPool();
-    // memcpy split over the helpers and the caller
-    void copy(char* dst, const char* src, size_t bytes);
-    // helpers spin for work between begin and end instead of sleeping
-    void begin();
-    void end();
-private:
-    static constexpr int HELPERS = 5;
-    void run();
-    void take_parts();
-    std::vector<std::thread> threads_;
-    bool started_ = false;
-    std::mutex mu_;
-    std::condition_variable cv_;
-    std::atomic<bool> busy_{false}, stop_{false};
-    std::atomic<unsigned> job_{0};
-    std::atomic<int> next_{0}, left_{0};
-    char* dst_ = nullptr;
-    const char* src_ = nullptr;
-    size_t bytes_ = 0;
-    std::atomic<int> parts_{0};
-    std::atomic<int> inside_{0};   // helpers between reading job_ and leaving take_parts
-};
 
 // The pinned ring of one engine; all its copies run on the engine's stream.
 struct Stager {

@@ -146,8 +146,7 @@ struct Server {
     oxr_server_config cfg{};
     std::thread th;
     std::mutex mu;
-    std::mutex copy_mu;              // who holds it may use the helper threads
-    CopyPool copies;
+    CopyPool copies;                 // take_hits, its callers together
     std::condition_variable cv_work, cv_done;
     std::deque<std::unique_ptr<Req>> incoming;
     std::vector<std::unique_ptr<Req>> active;
@@ -621,12 +620,10 @@ int oxr_server_take_hits(oxr_server* sh, int64_t id, void* dst, int64_t cap, int
     }
     // the hits reached pinned host memory before the request completed: a host copy, no
     // device work on the caller's thread. Large ones are split over the kept helper threads
-    // (one thread copies at about a third of what the memory system delivers), unless another
-    // caller is using them.
+    // (one thread copies at about a third of what the memory system delivers).
     size_t total = 0;
     for (auto& h : r->hits) total += size_t(h.n) * 64;
-    std::unique_lock<std::mutex> helpers(s->copy_mu, std::defer_lock);
-    const bool helped = total >= (size_t(1) << 20) && helpers.try_lock();
+    const bool helped = total >= (size_t(1) << 20);
     if (helped) s->copies.begin();
     char* o = static_cast<char*>(dst);
     for (auto& h : r->hits) {

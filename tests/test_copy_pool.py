@@ -1,0 +1,63 @@
+"""The helper threads of host copies (eic-opticks_amd/csrc/oxr_pool.cpp), on the CPU: several
+callers copy through one pool at once, buffers of sizes about its limits and parts, and every
+byte arrives and none beside them; a pool is made and joined many times over."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, 'eic-opticks_amd', 'csrc')
+
+PROGRAM = r'''
+#include "oxr_pool.h"
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+using namespace oxh;
+
+static const size_t SIZES[] = {1, 63, (256u << 10) - 1, 256u << 10, (256u << 10) + 1, 777777, (1u << 20) + 13, (2u << 20), (5u << 20) + 1};
+
+// one caller: its own windows about its own copies, the pattern its number and the turn's
+static int caller(CopyPool& pool, int id, int turns) {
+    std::vector<char> src((5u << 20) + 64), dst(src.size() + 64);
+    for (int t = 0; t < turns; t++) {
+        const size_t n = SIZES[size_t(t * 7 + id) % (sizeof(SIZES) / sizeof(SIZES[0]))], off = size_t(t % 3);
+        for (size_t i = 0; i < n + off; i++) src[i] = char((i * 2654435761u >> 8) + size_t(id * 31 + t));
+        std::memset(dst.data(), 0x5a, n + 64);
+        if (t % 2 == 0) pool.begin();
+        pool.copy(dst.data() + 8, src.data() + off, n);
+        if (t % 2 == 0) pool.end();
+        if (std::memcmp(dst.data() + 8, src.data() + off, n) != 0) return 1;
+        for (int k = 0; k < 8; k++) if (dst[size_t(k)] != 0x5a || dst[n + 8 + size_t(k)] != 0x5a) return 1;
+    }
+    return 0;
+}
+
+int main(int, char** a) {
+    const int callers = std::atoi(a[1]), turns = std::atoi(a[2]), pools = std::atoi(a[3]);
+    std::atomic<int> bad{0};
+    for (int p = 0; p < pools; p++) {
+        CopyPool pool;
+        std::vector<std::thread> th;
+        for (int c = 0; c < callers; c++) th.emplace_back([&, c] { bad += caller(pool, c, turns); });
+        for (auto& t : th) t.join();
+    }
+    return bad ? 1 : 0;
+}
+'''
+
+
+@pytest.fixture(scope='module')
+def program(tmp_path_factory):
+    d = tmp_path_factory.mktemp('pool')
+    (d / 'pool.cpp').write_text(PROGRAM)
+    subprocess.check_call(['g++', '-O2', '-std=c++17', '-I', CSRC, str(d / 'pool.cpp'), os.path.join(CSRC, 'oxr_pool.cpp'),
+                           '-o', str(d / 'pool'), '-lpthread'])
+    return str(d / 'pool')
+
+
+@pytest.mark.parametrize('callers,turns,pools', [(1, 40, 3), (2, 60, 2), (4, 60, 2), (7, 30, 1), (2, 2, 60)])
+def test_callers_together(program, callers, turns, pools):
+    subprocess.run([program, str(callers), str(turns), str(pools)], check=True, timeout=120)
