@@ -1,6 +1,8 @@
 """The helper threads of host copies (eic-opticks_amd/csrc/oxr_pool.cpp), on the CPU: several
 callers copy through one pool at once, buffers of sizes about its limits and parts, and every
-byte arrives and none beside them; a pool is made and joined many times over."""
+byte arrives and none beside them; a pool is made and joined many times over; and it has no
+more threads than the processors it may run on, down to none beside the caller, and they do
+not take processor time while a window stays open without a copy."""
 import os
 import subprocess
 
@@ -11,10 +13,13 @@ CSRC = os.path.join(ROOT, 'eic-opticks_amd', 'csrc')
 
 PROGRAM = r'''
 #include "oxr_pool.h"
+#include <chrono>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <ctime>
+#include <dirent.h>
 using namespace oxh;
 
 static const size_t SIZES[] = {1, 63, (256u << 10) - 1, 256u << 10, (256u << 10) + 1, 777777, (1u << 20) + 13, (2u << 20), (5u << 20) + 1};
@@ -35,7 +40,36 @@ static int caller(CopyPool& pool, int id, int turns) {
     return 0;
 }
 
-int main(int, char** a) {
+static int threads_now() {
+    int n = 0;
+    if (DIR* d = opendir("/proc/self/task")) {
+        while (dirent* e = readdir(d)) n += e->d_name[0] != '.';
+        closedir(d);
+    }
+    return n;
+}
+
+int main(int argc, char** a) {
+    if (argc == 3) {   // processor time of an open window of so many ms, copies before and after
+        CopyPool pool;
+        pool.begin();
+        int bad = caller(pool, 0, 40);
+        const std::clock_t c = std::clock();
+        std::this_thread::sleep_for(std::chrono::milliseconds(std::atoi(a[2])));
+        std::printf("%ld\n", long(1000.0 * double(std::clock() - c) / CLOCKS_PER_SEC));
+        bad += caller(pool, 0, 40);
+        pool.end();
+        return bad;
+    }
+    if (argc == 2) {   // the threads of a pool at work
+        CopyPool pool;
+        pool.begin();
+        const int n = threads_now();
+        const int bad = caller(pool, 0, 40);
+        pool.end();
+        std::printf("%d\n", n);
+        return bad;
+    }
     const int callers = std::atoi(a[1]), turns = std::atoi(a[2]), pools = std::atoi(a[3]);
     std::atomic<int> bad{0};
     for (int p = 0; p < pools; p++) {
@@ -61,3 +95,16 @@ def program(tmp_path_factory):
 @pytest.mark.parametrize('callers,turns,pools', [(1, 40, 3), (2, 60, 2), (4, 60, 2), (7, 30, 1), (2, 2, 60)])
 def test_callers_together(program, callers, turns, pools):
     subprocess.run([program, str(callers), str(turns), str(pools)], check=True, timeout=120)
+
+
+@pytest.mark.parametrize('cpus', [1, 2, 3, 64])
+def test_threads_fit_the_processors(program, cpus):
+    here = sorted(os.sched_getaffinity(0))[:cpus]
+    r = subprocess.run([program, 'threads'], check=True, timeout=120, stdout=subprocess.PIPE,
+                       preexec_fn=lambda: os.sched_setaffinity(0, here))
+    assert int(r.stdout) == min(6, len(here))
+
+
+def test_waiting_takes_no_processor_time(program):
+    r = subprocess.run([program, 'window', '400'], check=True, timeout=120, stdout=subprocess.PIPE)
+    assert int(r.stdout) < 40   # ms; five helpers that spin throughout take up to 2000
