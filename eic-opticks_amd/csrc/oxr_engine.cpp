@@ -144,20 +144,20 @@ oxd::Params Engine::params(EventBuffers& b, int64_t n, int64_t slot_off, int32_t
 
 int ensure_event_capacity(Engine& e, EventBuffers& b, int64_t n) {
     size_t N = size_t(std::max<int64_t>(n, 1));
-    OXR_HIP(b.seed.reserve(N));
-    OXR_HIP(b.photon.reserve(4 * N));
-    if (e.cfg.seq_enabled) OXR_HIP(b.seq.reserve(2 * N));
-    if (e.cfg.max_record > 0) OXR_HIP(b.record.reserve(4 * N * size_t(e.cfg.max_record)));
-    if (e.cfg.max_rec > 0) OXR_HIP(b.rec.reserve(N * size_t(e.cfg.max_rec)));
-    if (e.cfg.max_prd > 0) OXR_HIP(b.prd.reserve(2 * N * size_t(e.cfg.max_prd)));
-    if (e.cfg.photonlite) OXR_HIP(b.lite.reserve(N));
-    OXR_HIP(b.hitflag.reserve(N));
-    OXR_HIP(b.rstate.reserve(N));
-    OXR_HIP(b.hit.reserve(4 * N));
+    OXR_HIP(e.ws.reserve(b.seed, N));
+    OXR_HIP(e.ws.reserve(b.photon, 4 * N));
+    if (e.cfg.seq_enabled) OXR_HIP(e.ws.reserve(b.seq, 2 * N));
+    if (e.cfg.max_record > 0) OXR_HIP(e.ws.reserve(b.record, 4 * N * size_t(e.cfg.max_record)));
+    if (e.cfg.max_rec > 0) OXR_HIP(e.ws.reserve(b.rec, N * size_t(e.cfg.max_rec)));
+    if (e.cfg.max_prd > 0) OXR_HIP(e.ws.reserve(b.prd, 2 * N * size_t(e.cfg.max_prd)));
+    if (e.cfg.photonlite) OXR_HIP(e.ws.reserve(b.lite, N));
+    OXR_HIP(e.ws.reserve(b.hitflag, N));
+    OXR_HIP(e.ws.reserve(b.rstate, N));
+    OXR_HIP(e.ws.reserve(b.hit, 4 * N));
     int nb = oxl::compact_blocks(int64_t(N));
-    OXR_HIP(b.counts.reserve(size_t(nb)));
-    OXR_HIP(b.offs.reserve(size_t(nb) + 1));
-    OXR_HIP(b.counters.reserve(8));
+    OXR_HIP(e.ws.reserve(b.counts, size_t(nb)));
+    OXR_HIP(e.ws.reserve(b.offs, size_t(nb) + 1));
+    OXR_HIP(e.ws.reserve(b.counters, 8));
     return OXR_OK;
 }
 
@@ -192,8 +192,8 @@ int upload_gensteps(Engine& e, EventBuffers& b, hipStream_t s, const float* gs, 
     }
     int rc = ensure_event_capacity(e, b, n);
     if (rc) return rc;
-    OXR_HIP(b.gs.reserve(size_t(std::max<int64_t>(num_gs, 1)) * 6));
-    OXR_HIP(b.gs_off.reserve(size_t(num_gs) + 1));
+    OXR_HIP(e.ws.reserve(b.gs, size_t(std::max<int64_t>(num_gs, 1)) * 6));
+    OXR_HIP(e.ws.reserve(b.gs_off, size_t(num_gs) + 1));
     // staged, so the caller's array and off are free again while the copies run
     if (num_gs > 0) {
         OXR_HIP(e.stage.h2d(s, b.gs.p, gs, size_t(num_gs) * 96));
@@ -231,11 +231,11 @@ int run_launch(Engine& e, EventBuffers& b, hipStream_t s, int64_t n, int64_t slo
             // under as many genstep-index bits as the event needs
             int bits = 16;
             while (bits < 64 && (int64_t(1) << (bits - 16)) < e.num_gs) bits++;
-            OXR_HIP(b.okey.reserve(2 * size_t(n)));
-            OXR_HIP(b.oval.reserve(2 * size_t(n)));
+            OXR_HIP(e.ws.reserve(b.okey, 2 * size_t(n)));
+            OXR_HIP(e.ws.reserve(b.oval, 2 * size_t(n)));
             size_t tb = 0;
             OXR_HIP(oxl::order_photons(s, P, bits, b.okey.p, b.oval.p, nullptr, &tb, nullptr));
-            OXR_HIP(b.otmp.reserve(std::max<size_t>(tb, 1)));
+            OXR_HIP(e.ws.reserve(b.otmp, std::max<size_t>(tb, 1)));
             OXR_HIP(oxl::order_photons(s, P, bits, b.okey.p, b.oval.p, b.otmp.p, &tb, &P.perm));
         }
         OXR_HIP(oxl::simulate_persist(s, P, block, grid, e.cfg.fp64_roots != 0, e.has_list));
@@ -936,7 +936,7 @@ void oxr_engine_destroy(oxr_engine* eh) {
     if (e->e2) (void)hipEventDestroy(e->e2);
     if (e->eg) (void)hipEventDestroy(e->eg);
     e->stage.release();
-    e->ws.release();
+    e->ws.give_back();
     if (e->pub) (void)hipHostFree(e->pub);
     if (e->stream) (void)hipStreamDestroy(e->stream);
     delete e;
@@ -1030,7 +1030,7 @@ int oxr_event_set_input_photons(oxr_engine* eh, const float* photons, int64_t n)
     if (!e || n < 0 || (n > 0 && !photons)) return fail(OXR_EINVAL, "bad input photons");
     std::lock_guard<std::mutex> lk(e->mu);
     if (n == 0) { e->have_input = false; e->input_n = 0; return OXR_OK; }
-    OXR_HIP(e->ev.input.reserve(size_t(n) * 4));
+    OXR_HIP(e->ws.reserve(e->ev.input, size_t(n) * 4));
     int rc = e->h2d(e->ev.input.p, photons, size_t(n) * 64);
     if (rc) return rc;
     e->have_input = true;
@@ -1044,7 +1044,7 @@ int oxr_event_set_precooked(oxr_engine* eh, const float* u, int64_t n_photon, in
     std::lock_guard<std::mutex> lk(e->mu);
     if (!u || n_photon == 0) { e->have_pre = false; e->npre = 0; return OXR_OK; }
     if (n_photon < 0 || n_per < 1) return fail(OXR_EINVAL, "precooked shape");
-    OXR_HIP(e->ev.pre.reserve(size_t(n_photon) * size_t(n_per)));
+    OXR_HIP(e->ws.reserve(e->ev.pre, size_t(n_photon) * size_t(n_per)));
     int rc = e->h2d(e->ev.pre.p, u, size_t(n_photon) * size_t(n_per) * 4);
     if (rc) return rc;
     e->have_pre = true;
@@ -1140,7 +1140,7 @@ int oxr_event_get(oxr_engine* eh, int32_t what, void* dst, int64_t cap, int64_t*
             if (e->launched && !e->hitlite_ready) {
                 // same selection and order as the sphoton hits (sphotonlite_selector,
                 // sphotonlite.h:159-165): reuse the launch's compaction offsets
-                OXR_HIP(e->ev.hitlite.reserve(size_t(std::max<int64_t>(e->num_hit, 1))));
+                OXR_HIP(e->ws.reserve(e->ev.hitlite, size_t(std::max<int64_t>(e->num_hit, 1))));
                 OXR_HIP(oxl::scatter_lite(e->stream, e->ev.hitflag.p, e->ev.lite.p, e->num_photon, e->ev.offs.p,
                                           e->ev.hitlite.p, e->num_hit));
                 OXR_HIP(hipStreamSynchronize(e->stream));
@@ -1199,10 +1199,11 @@ int oxr_event_get_merged(oxr_engine* eh, int32_t what, float time_window, void* 
     if (lite && !e->cfg.photonlite) return fail(OXR_ESTATE, "photonlite is off");
     size_t words = lite ? 4 : 16;
     const void* in = lite ? static_cast<const void*>(e->ev.lite.p) : static_cast<const void*>(e->ev.photon.p);
-    OXR_HIP(e->ev.merged.reserve(words * size_t(std::max<int64_t>(e->num_photon, 1))));
+    OXR_HIP(e->ws.reserve(e->ev.merged, words * size_t(std::max<int64_t>(e->num_photon, 1))));
     long long nout = 0;
+    oxl::WorkCall work(e->ws);
     OXR_HIP(oxl::merge(e->stream, lite, in, e->num_photon, e->cfg.hitmask, true, time_window, e->ev.merged.p, &nout, e->ws));
-    e->ws.trim();
+    work.keep();
     return copy_out(*e, e->ev.merged.p, nout, words * 4, dst, cap, count);
 }
 
@@ -1219,14 +1220,15 @@ int oxr_merge_hits(oxr_engine* eh, int32_t what, float time_window, const void* 
     DBuf<uint32_t> din, dout;
     auto done = [&](int rc) { din.release(); dout.release(); return rc; };
     hipError_t he;
-    if ((he = din.reserve(words * size_t(n))) != hipSuccess) return done(hip_fail(he, "merge input"));
-    if ((he = dout.reserve(words * size_t(n))) != hipSuccess) return done(hip_fail(he, "merge output"));
+    if ((he = e->ws.reserve(din, words * size_t(n))) != hipSuccess) return done(hip_fail(he, "merge input"));
+    if ((he = e->ws.reserve(dout, words * size_t(n))) != hipSuccess) return done(hip_fail(he, "merge output"));
     int rc = e->h2d(din.p, in, words * 4 * size_t(n));
     if (rc) return done(rc);
     long long nout = 0;
+    oxl::WorkCall work(e->ws);
     if ((he = oxl::merge(e->stream, lite, din.p, n, 0u, false, time_window, dout.p, &nout, e->ws)) != hipSuccess)
         return done(hip_fail(he, "merge"));
-    e->ws.trim();
+    work.keep();
     return done(copy_out(*e, dout.p, nout, words * 4, dst, cap, count));
 }
 
@@ -1285,9 +1287,10 @@ int oxr_trace_rays(oxr_engine* eh, const float* rays, int64_t n, float* prd) {
     std::lock_guard<std::mutex> lk(e->mu);
     // device buffers kept in the engine's work space, copies staged on its stream: allocating
     // two buffers, two copies from pageable memory and freeing took most of a call
+    oxl::WorkCall work(e->ws);
     DBuf<char>&dr = e->ws.slot[0], &dp = e->ws.slot[1];
-    OXR_HIP(dr.reserve(size_t(n) * 32));
-    OXR_HIP(dp.reserve(size_t(n) * 32));
+    OXR_HIP(e->ws.get(0, size_t(n) * 32));
+    OXR_HIP(e->ws.get(1, size_t(n) * 32));
     int rc = e->h2d(dr.p, rays, size_t(n) * 32);
     if (rc) return rc;
     EventBuffers dummy;
@@ -1295,7 +1298,7 @@ int oxr_trace_rays(oxr_engine* eh, const float* rays, int64_t n, float* prd) {
     OXR_HIP(oxl::trace_rays(e->stream, P, reinterpret_cast<const float4*>(dr.p), n, reinterpret_cast<float4*>(dp.p),
                             e->cfg.fp64_roots != 0, e->has_list));
     rc = e->d2h(prd, dp.p, size_t(n) * 32);
-    e->ws.trim();
+    if (!rc) work.keep();
     return rc;
 }
 
@@ -1320,10 +1323,11 @@ int oxr_simtrace(oxr_engine* eh, const float* gs, int64_t num_gs, float* simtrac
     if (!simtrace) return fail(OXR_EINVAL, "null simtrace buffer");
     if (num_gs > 0x7fffffffLL) return fail(OXR_EINVAL, "too many gensteps");
     std::lock_guard<std::mutex> lk(e->mu);
+    oxl::WorkCall work(e->ws);
     DBuf<char>&dg = e->ws.slot[0], &doff = e->ws.slot[1], &dout = e->ws.slot[2];
-    OXR_HIP(dg.reserve(size_t(num_gs) * 96));
-    OXR_HIP(doff.reserve(off.size() * sizeof(long long)));
-    OXR_HIP(dout.reserve(size_t(n) * 64));
+    OXR_HIP(e->ws.get(0, size_t(num_gs) * 96));
+    OXR_HIP(e->ws.get(1, off.size() * sizeof(long long)));
+    OXR_HIP(e->ws.get(2, size_t(n) * 64));
     int rc = e->h2d(dg.p, gs, size_t(num_gs) * 96);
     if (!rc) rc = e->h2d(doff.p, off.data(), off.size() * sizeof(long long));
     if (rc) return rc;
@@ -1332,7 +1336,7 @@ int oxr_simtrace(oxr_engine* eh, const float* gs, int64_t num_gs, float* simtrac
     OXR_HIP(oxl::simtrace(e->stream, P, reinterpret_cast<const float4*>(dg.p), reinterpret_cast<const long long*>(doff.p), int(num_gs),
                           n, reinterpret_cast<float4*>(dout.p), e->cfg.fp64_roots != 0, e->has_list));
     rc = e->d2h(simtrace, dout.p, size_t(n) * 64);
-    e->ws.trim();
+    if (!rc) work.keep();
     return rc;
 }
 
@@ -1344,17 +1348,18 @@ int oxr_intersect_prim(oxr_engine* eh, int32_t prim_index, const float* rays, in
     std::lock_guard<std::mutex> lk(e->mu);
     int2 pr;
     OXR_HIP(hipMemcpy(&pr, e->prim.p + prim_index, sizeof(int2), hipMemcpyDeviceToHost));
+    oxl::WorkCall work(e->ws);
     DBuf<char>&dr = e->ws.slot[0], &di = e->ws.slot[1], &dv = e->ws.slot[2];
-    OXR_HIP(dr.reserve(size_t(n) * 32));
-    OXR_HIP(di.reserve(size_t(n) * 16));
-    OXR_HIP(dv.reserve(size_t(n) * 4));
+    OXR_HIP(e->ws.get(0, size_t(n) * 32));
+    OXR_HIP(e->ws.get(1, size_t(n) * 16));
+    OXR_HIP(e->ws.get(2, size_t(n) * 4));
     int rc = e->h2d(dr.p, rays, size_t(n) * 32);
     if (rc) return rc;
     OXR_HIP(oxl::intersect_prim(e->stream, e->geom(), pr.x, reinterpret_cast<const float4*>(dr.p), n, reinterpret_cast<float4*>(di.p),
                                 reinterpret_cast<int*>(dv.p), e->cfg.fp64_roots != 0, e->has_list));
     rc = e->d2h(isect, di.p, size_t(n) * 16);
     if (!rc) rc = e->d2h(valid, dv.p, size_t(n) * 4);
-    e->ws.trim();
+    if (!rc) work.keep();
     return rc;
 }
 

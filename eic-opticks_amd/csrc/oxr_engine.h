@@ -6,6 +6,7 @@
 #include <vector>
 #include <mutex>
 #include "oxr_copy.h"
+#include "oxr_dbuf.h"
 #include "../../include/oxr.h"
 #include "oxr_kernels.h"
 
@@ -20,37 +21,6 @@ int hip_fail(hipError_t e, const char* what);
         hipError_t _e = (call);                                              \
         if (_e != hipSuccess) return ::oxh::hip_fail(_e, #call);             \
     } while (0)
-
-template <typename T>
-struct DBuf {
-    T* p = nullptr;
-    size_t n = 0;     // capacity in elements
-    hipError_t reserve(size_t want) {
-        if (want <= n) return hipSuccess;
-        if (p) { hipError_t e = hipFree(p); if (e != hipSuccess) return e; p = nullptr; n = 0; }
-        hipError_t e = hipMalloc(reinterpret_cast<void**>(&p), want * sizeof(T));
-        if (e == hipSuccess) n = want;
-        return e;
-    }
-    void release() { if (p) (void)hipFree(p); p = nullptr; n = 0; }
-};
-
-} // namespace oxh
-namespace oxl {
-// Device buffers that a call (a merge, a query) uses and the engine keeps for the next:
-// allocating and freeing them in every call cost a merge of 34k hits 60 of its 400 us and a
-// query of 250k rays, with its pageable copies, 340 of 910.
-struct Workspace {
-    static constexpr int N = 15;
-    oxh::DBuf<char> slot[N];
-    int used = 0;
-    size_t bytes() const { size_t b = 0; for (const auto& x : slot) b += x.n; return b; }
-    void release() { for (auto& x : slot) x.release(); }
-    // what stays allocated between calls is bounded
-    void trim() { if (bytes() > (size_t(512) << 20)) release(); }
-};
-} // namespace oxl
-namespace oxh {
 
 // One event slice's device buffers (the QEvt role).
 struct EventBuffers {
@@ -138,7 +108,7 @@ struct Engine {
     Stager stage;
     int d2h(void* dst, const void* src, size_t bytes);
     int h2d(void* dst, const void* src, size_t bytes);
-    oxl::Workspace ws;                  // merges and queries
+    oxl::Workspace ws;                  // merges and queries (callers hold mu)
     oxd::LaunchResult* pub = nullptr;   // pinned: what the last launch left for the host
     bool counters_zero = false;         // ev.counters is zero (the last launch's selection left it so)
     std::mutex mu;   // serialises C-ABI calls on one engine

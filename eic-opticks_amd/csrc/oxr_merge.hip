@@ -125,7 +125,7 @@ struct Tmp {
     void* p = nullptr;
     explicit Tmp(Workspace& w) : ws(w), k(w.used++) {}
     hipError_t get(size_t bytes) {
-        hipError_t e = ws.slot[k].reserve(bytes ? bytes : 1);
+        hipError_t e = ws.get(k, bytes ? bytes : 1);
         p = ws.slot[k].p;
         return e;
     }
@@ -137,7 +137,6 @@ template <bool LITE>
 static hipError_t merge_t(hipStream_t s, const uint32_t* in, long long n, unsigned mask, bool select, float tw,
                           uint32_t* out, long long* num_out, Workspace& ws) {
     *num_out = 0;
-    ws.used = 0;
     if (n <= 0) return hipSuccess;
     if (n > 0x7fffffffLL) return hipErrorInvalidValue;
     const int N = int(n);

@@ -241,7 +241,10 @@ const char* oxr_last_error(void);
 /* ---- engine lifecycle --------------------------------------------------
  * Replaces CSGOptiX::Create(CSGFoundry*) (CSGOptiX/CSGOptiX.cc:367-399) together with
  * QSim::UploadComponents (qudarap/QSim.cc:118-250) and SBT::createGeom
- * (CSGOptiX/SBT.cc:247-259): copies geometry and tables to HBM and builds the BVHs. */
+ * (CSGOptiX/SBT.cc:247-259): copies geometry and tables to HBM and builds the BVHs.
+ * Besides these and the event's buffers an engine keeps what merges and queries work in, at
+ * most 512 MB of device memory, from call to call; it gives them up when its event buffers
+ * need the memory, and after a call that failed. */
 int  oxr_engine_create(const oxr_geometry* geo, const oxr_physics* phys,
                        const oxr_config* cfg, oxr_engine** out);
 void oxr_engine_destroy(oxr_engine* e);
