@@ -2,6 +2,7 @@
 // per-event genstep upload and seeding, launches, hit compaction, gathers, queries and
 // the autotuner. The serving loop lives in oxr_server.cpp.
 #include "oxr_engine.h"
+#include "oxr_boxes.h"
 #include "oxr_bvh.h"
 #include <algorithm>
 #include <chrono>
@@ -279,27 +280,6 @@ int run_launch(Engine& e, EventBuffers& b, hipStream_t s, int64_t n, int64_t slo
     return OXR_OK;
 }
 
-// inverse of the instance transform in double (row convention, identity column ignored)
-static void invert_instance(const float* q, double W[4][3]) {
-    double a[3][3], t[3];
-    for (int r = 0; r < 3; r++) for (int k = 0; k < 3; k++) a[r][k] = q[4 * r + k];
-    for (int k = 0; k < 3; k++) t[k] = q[12 + k];
-    double det = a[0][0] * (a[1][1] * a[2][2] - a[1][2] * a[2][1]) - a[0][1] * (a[1][0] * a[2][2] - a[1][2] * a[2][0]) +
-                 a[0][2] * (a[1][0] * a[2][1] - a[1][1] * a[2][0]);
-    double inv[3][3];
-    inv[0][0] = (a[1][1] * a[2][2] - a[1][2] * a[2][1]) / det;
-    inv[0][1] = (a[0][2] * a[2][1] - a[0][1] * a[2][2]) / det;
-    inv[0][2] = (a[0][1] * a[1][2] - a[0][2] * a[1][1]) / det;
-    inv[1][0] = (a[1][2] * a[2][0] - a[1][0] * a[2][2]) / det;
-    inv[1][1] = (a[0][0] * a[2][2] - a[0][2] * a[2][0]) / det;
-    inv[1][2] = (a[0][2] * a[1][0] - a[0][0] * a[1][2]) / det;
-    inv[2][0] = (a[1][0] * a[2][1] - a[1][1] * a[2][0]) / det;
-    inv[2][1] = (a[0][1] * a[2][0] - a[0][0] * a[2][1]) / det;
-    inv[2][2] = (a[0][0] * a[1][1] - a[0][1] * a[1][0]) / det;
-    for (int i = 0; i < 3; i++) for (int k = 0; k < 3; k++) W[i][k] = inv[i][k];
-    for (int k = 0; k < 3; k++) W[3][k] = -(t[0] * inv[0][k] + t[1] * inv[1][k] + t[2] * inv[2][k]);
-}
-
 static bool supported_leaf(uint32_t tc) {
     return tc == 101 || tc == 103 || tc == 105 || tc == 108 || tc == 110 || tc == 112 || tc == 117 || tc == 121 ||
            tc == 125;
@@ -440,114 +420,6 @@ static std::vector<float4> device_nodes(const oxr_geometry* g, std::vector<int2>
         }
     }
     return out;
-}
-
-// The world box of one placed prim from its leaves' own shapes, when they are all spheres,
-// zspheres, cylinders or boxes: the union of the leaves' boxes, complemented ones too, so
-// every surface point a test can report lies in it. The corners of the prim's object box
-// turned into the world reach up to 1.7 times as far (a photomultiplier's bulb and neck, turned
-// 45 degrees: 2.2 times the area), and each such box costs node visits and prim tests along
-// its rays. reach is the longest distance from a ray's origin to anything in the scene: a
-// quadric's discriminant in single precision is off by at most 16 ulps of its square, so a ray
-// may be reported to hit a sphere or cylinder up to sqrt(r^2 + 2e-6 reach^2) from its axis
-// (twice that bound), and the boxes take that radius. A ray from further away than the scene
-// is wide widens the boxes as it meets them (far_pad, oxr_trace.h): stretch is the most that
-// a distance in the world grows by on its way into a leaf's frame and its margin back, the
-// longest column of the leaf's transform times the norm of its inverse.
-// Instanced CSG, 10M photons: 7.7 -> 6.1 ms; 200k photons 540 -> 466 us; the served stream of 24
-// events 9.5 -> 7.9 ms.
-static bool leaf_box(const oxr_geometry* g, int64_t ni, const double A[4][3], double reach, Box& out, double& stretch) {
-    const float* q = g->node + 16 * ni;
-    const uint32_t tc = fbits(q[14]), gt = fbits(q[15]) & 0x7fffffffu;
-    if (tc != 101u && tc != 103u && tc != 105u && tc != 110u) return false;
-    double M[4][3];   // leaf to world, row convention
-    if (gt > 0u) {
-        double L[4][3];   // leaf to object
-        invert_instance(g->itra + 16 * (int64_t(gt) - 1), L);
-        for (int r = 0; r < 4; r++) for (int k = 0; k < 3; k++) {
-            M[r][k] = L[r][0] * A[0][k] + L[r][1] * A[1][k] + L[r][2] * A[2][k] + (r == 3 ? A[3][k] : 0.0);
-            if (!std::isfinite(M[r][k])) return false;
-        }
-    } else {
-        for (int r = 0; r < 4; r++) for (int k = 0; k < 3; k++) M[r][k] = A[r][k];
-    }
-    float f[16] = {0};
-    for (int r = 0; r < 4; r++) for (int k = 0; k < 3; k++) f[4 * r + k] = float(M[r][k]);
-    double I[4][3], norm2 = 0.0;
-    invert_instance(f, I);
-    for (int r = 0; r < 3; r++) for (int k = 0; k < 3; k++) norm2 += I[r][k] * I[r][k];
-    const double far = reach * std::sqrt(norm2);   // the reach in the leaf's frame
-    if (!std::isfinite(far)) return false;
-    for (int k = 0; k < 3; k++)
-        stretch = std::max(stretch, std::sqrt(norm2 * (M[0][k] * M[0][k] + M[1][k] * M[1][k] + M[2][k] * M[2][k])));
-    const double flat = 16.0 * 6e-8 * far;         // planes: a few ulps of the distance
-    auto map = [&](double x, double y, double z, double* w) {
-        for (int k = 0; k < 3; k++) w[k] = x * M[0][k] + y * M[1][k] + z * M[2][k] + M[3][k];
-    };
-    auto around = [&](const double* c, double hx, double hy, double hz) {   // the box of a leaf-frame box
-        Box b;
-        for (int k = 0; k < 3; k++) {
-            const double h = std::fabs(M[0][k]) * hx + std::fabs(M[1][k]) * hy + std::fabs(M[2][k]) * hz;
-            b.lo[k] = c[k] - h; b.hi[k] = c[k] + h;
-        }
-        return b;
-    };
-    double c[3];
-    if (tc == 110u) {
-        map(0.0, 0.0, 0.0, c);
-        out = around(c, 0.5 * std::fabs(q[0]) + flat, 0.5 * std::fabs(q[1]) + flat, 0.5 * std::fabs(q[2]) + flat);
-        return true;
-    }
-    const double R = std::sqrt(double(q[3]) * double(q[3]) + 2e-6 * far * far);
-    if (tc == 105u) {
-        const double zc = 0.5 * (double(q[4]) + double(q[5])), hz = 0.5 * std::fabs(double(q[5]) - double(q[4])) + flat;
-        map(0.0, 0.0, zc, c);
-        for (int k = 0; k < 3; k++) {
-            const double h = R * std::sqrt(M[0][k] * M[0][k] + M[1][k] * M[1][k]) + hz * std::fabs(M[2][k]);
-            out.lo[k] = c[k] - h; out.hi[k] = c[k] + h;
-        }
-        return true;
-    }
-    map(q[0], q[1], q[2], c);
-    for (int k = 0; k < 3; k++) {
-        const double h = R * std::sqrt(M[0][k] * M[0][k] + M[1][k] * M[1][k] + M[2][k] * M[2][k]);
-        out.lo[k] = c[k] - h; out.hi[k] = c[k] + h;
-    }
-    if (tc == 103u) {   // and the slab between its planes
-        double zc[3];
-        map(q[0], q[1], double(q[2]) + 0.5 * (double(q[4]) + double(q[5])), zc);
-        const Box slab = around(zc, R, R, 0.5 * std::fabs(double(q[5]) - double(q[4])) + flat);
-        for (int k = 0; k < 3; k++) { out.lo[k] = std::max(out.lo[k], slab.lo[k]); out.hi[k] = std::min(out.hi[k], slab.hi[k]); }
-    }
-    return true;
-}
-
-// b: the prim's object box turned into the world; cut to the leaves' box where that is known
-static void tighten(const oxr_geometry* g, int64_t prim, const float* inst, double reach, Box& b, double& stretch) {
-    int32_t numNode, nodeOffset;
-    std::memcpy(&numNode, g->prim + 16 * prim, 4);
-    std::memcpy(&nodeOffset, g->prim + 16 * prim + 1, 4);
-    double A[4][3];
-    for (int r = 0; r < 4; r++) for (int k = 0; k < 3; k++) A[r][k] = inst[4 * r + k];
-    const uint32_t root = fbits(g->node[16 * int64_t(nodeOffset) + 14]);
-    int64_t n = 1;
-    if (is_op(root)) n = fbits(g->node[16 * int64_t(nodeOffset)]);
-    else if (is_list(root)) return;
-    Box all = Box::empty();
-    for (int64_t i = 0; i < n; i++) {
-        const uint32_t tc = fbits(g->node[16 * (nodeOffset + i) + 14]);
-        if (tc == 0u || is_op(tc)) continue;
-        Box lb;
-        if (!leaf_box(g, nodeOffset + i, A, reach, lb, stretch)) return;
-        all.grow(lb);
-    }
-    Box cut = b;
-    for (int k = 0; k < 3; k++) {
-        cut.lo[k] = std::max(b.lo[k], all.lo[k]);
-        cut.hi[k] = std::min(b.hi[k], all.hi[k]);
-        if (!(cut.lo[k] <= cut.hi[k])) return;   // box and shape disagree: the box stands
-    }
-    b = cut;
 }
 
 } // namespace oxh
@@ -748,21 +620,28 @@ int oxr_engine_create(const oxr_geometry* g, const oxr_physics* ph, const oxr_co
         solid_nodes[size_t(s) + 1] = int32_t(blas_all.size());
         rad_blas.insert(rad_blas.end(), bv.rad.begin(), bv.rad.end());
     }
-    // the world box of prim p of solid gas placed by q
+    // Flattened form, built besides the two levels while the placed prims number at most
+    // kFlatMax and used when the tuning asks (bvh_mode 1): one BVH over every (instance,
+    // prim) with world boxes. A trace then skips the BLAS roots and the return to the top
+    // level, and prims are culled by their own world boxes rather than their instance's. Each
+    // prim is still tested in its instance's frame with the same arithmetic and the
+    // closest-hit key is the same, so the hits are identical.
+    const int64_t kFlatMax = int64_t(1) << 21;
+    int64_t placed = 0;
+    for (int64_t i = 0; i < g->num_inst; i++) {
+        int32_t gas; std::memcpy(&gas, g->inst + 16 * i + 7, 4);
+        placed += e->solid_num_prim[size_t(gas)];
+    }
+    e->has_flat = placed <= kFlatMax;
+    // Instance boxes are cut to the union of their prims' world boxes, which the flattened form
+    // needs anyway. Beyond its size only solids of few prims are cut: the boxes of kCutPrims
+    // prims take about as long as an instance's share of building the tree (0.3 us a prim of five
+    // leaves, 2.7 us). 24,000 instances of 100 prims: created in 380 ms with every box, now in 20.
+    const int kCutPrims = 8;
     const double reach = 2.0 * std::sqrt(3.0) * W;
-    double stretch = 1.0;
-    auto placed_box = [&](const float* q, int32_t gas, size_t p) -> oxh::Box {
-        const oxh::Box& ob = prim_boxes[size_t(gas)][p];
-        oxh::Box wb = oxh::Box::empty();
-        for (int c = 0; c < 8; c++) {
-            double pt[3] = {(c & 1) ? ob.hi[0] : ob.lo[0], (c & 2) ? ob.hi[1] : ob.lo[1], (c & 4) ? ob.hi[2] : ob.lo[2]};
-            double w[3];
-            for (int k = 0; k < 3; k++) w[k] = pt[0] * q[k] + pt[1] * q[4 + k] + pt[2] * q[8 + k] + q[12 + k];
-            wb.grow_point(w);
-        }
-        tighten(g, e->solid_prim_offset[size_t(gas)] + int64_t(p), q, reach, wb, stretch);
-        return wb;
-    };
+    oxh::LeafBoxes leaf_boxes(g, reach);
+    std::vector<oxh::Box> leaf_box;   // of every placed prim, for the flattened form
+    if (e->has_flat) leaf_box.reserve(size_t(placed));
     // ---- instances and TLAS
     std::vector<oxd::InstD> insts(static_cast<size_t>(g->num_inst));
     std::vector<oxh::Box> inst_box(static_cast<size_t>(g->num_inst));
@@ -798,39 +677,27 @@ int oxr_engine_create(const oxr_geometry* g, const oxr_physics* ph, const oxr_co
             for (int k = 0; k < 3; k++) w[k] = p[0] * q[k] + p[1] * q[4 + k] + p[2] * q[8 + k] + q[12 + k];
             wb.grow_point(w);
         }
-        // cut to the union of its prims' boxes
-        Box prims = Box::empty();
-        for (size_t p = 0; p < prim_boxes[size_t(gas)].size(); p++) prims.grow(placed_box(q, gas, p));
-        for (int k = 0; k < 3; k++) { wb.lo[k] = std::max(wb.lo[k], prims.lo[k]); wb.hi[k] = std::min(wb.hi[k], prims.hi[k]); }
+        const std::vector<oxh::Box>& pb = prim_boxes[size_t(gas)];
+        if (e->has_flat || pb.size() <= size_t(kCutPrims)) {
+            Box prims = Box::empty();
+            for (size_t p = 0; p < pb.size(); p++) {
+                const oxh::Box b = leaf_boxes.placed(e->solid_prim_offset[size_t(gas)] + int64_t(p), pb[p], q, W);
+                prims.grow(b);
+                if (e->has_flat) leaf_box.push_back(b);
+            }
+            for (int k = 0; k < 3; k++) { wb.lo[k] = std::max(wb.lo[k], prims.lo[k]); wb.hi[k] = std::min(wb.hi[k], prims.hi[k]); }
+        }
         inst_box[size_t(i)] = wb;
     }
-    // Flattened form, built besides the two levels while the placed prims number at most
-    // kFlatMax and used when the tuning asks (bvh_mode 1): one BVH over every (instance,
-    // prim) with world boxes. A trace then skips the BLAS roots and the return to the top
-    // level, and prims are culled by their own world boxes rather than their instance's;
-    // scenes that mix huge and small boxes (concentric shells around small instances) can
-    // trace slower on it, so the autotuner picks. Each prim is still tested in its
-    // instance's frame with the same arithmetic and the closest-hit key is the same, so the
-    // hits are identical.
-    const int64_t kFlatMax = int64_t(1) << 21;
-    int64_t placed = 0;
-    for (int64_t i = 0; i < g->num_inst; i++) {
-        int32_t gas; std::memcpy(&gas, g->inst + 16 * i + 7, 4);
-        placed += e->solid_num_prim[size_t(gas)];
-    }
-    e->has_flat = placed <= kFlatMax;
     oxh::Bvh tl, tf;
     std::vector<int4> flat_items;   // {instance, prim's place, its node offset, InstD flags}
     if (e->has_flat) {
-        std::vector<oxh::Box> leaf_box;
         std::vector<oxh::RadItem> leaf_rad;
-        leaf_box.reserve(size_t(placed)); flat_items.reserve(size_t(placed)); leaf_rad.reserve(size_t(placed));
+        flat_items.reserve(size_t(placed)); leaf_rad.reserve(size_t(placed));
         for (int64_t i = 0; i < g->num_inst; i++) {
             const float* q = g->inst + 16 * i;
             int32_t gas; std::memcpy(&gas, q + 7, 4);
-            const std::vector<oxh::Box>& pb = prim_boxes[size_t(gas)];
-            for (size_t p = 0; p < pb.size(); p++) {
-                leaf_box.push_back(placed_box(q, gas, p));
+            for (size_t p = 0; p < prim_boxes[size_t(gas)].size(); p++) {
                 const int place = e->solid_prim_offset[size_t(gas)] + int(p);
                 flat_items.push_back(make_int4(int(i), place, primtab[size_t(place)].x, insts[size_t(i)].info.z));
                 // world-frame sphere only for an instance with the identity transform
@@ -873,7 +740,7 @@ int oxr_engine_create(const oxr_geometry* g, const oxr_physics* ph, const oxr_co
         insts[size_t(i)].info.w = e->solid_blas_root[size_t(gas)];
     }
     e->far_extent = float(0.5 * reach);
-    e->far_scale = float(1.5e-3 * stretch);   // sqrt(2e-6) for the quadrics, the rest for the planes (flat)
+    e->far_scale = float(1.5e-3 * leaf_boxes.stretch());   // sqrt(2e-6) for the quadrics, the rest for the planes (flat)
     tl.nodes.insert(tl.nodes.end(), blas_all.begin(), blas_all.end());
     tl.rad.insert(tl.rad.end(), rad_blas.begin(), rad_blas.end());
     if (e->stack_cap() > 96) return bail(fail(OXR_EINVAL, "BVH too deep for the traversal stack"));

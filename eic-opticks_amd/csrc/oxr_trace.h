@@ -82,7 +82,7 @@ OXD f3 safe_inv(f3 d) {
 }
 OXD f3 neg_oi(f3 o, f3 inv) { return mk(-(o.x * inv.x), -(o.y * inv.y), -(o.z * inv.z)); }
 // The world boxes of quadrics hold what their single-precision tests may report from origins
-// within the scene (tighten, oxr_engine.cpp). The error of a test grows with the origin's
+// within the scene (oxr_boxes.h). The error of a test grows with the origin's
 // distance D: from outside, a box has to reach sqrt(2e-6 (D^2 - reach^2)) further, times the
 // worst stretch of a leaf's transform, than the margin it was stored with. Nothing is added
 // for an origin within the scene.
