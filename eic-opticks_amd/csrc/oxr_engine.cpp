@@ -156,7 +156,7 @@ int ensure_event_capacity(Engine& e, EventBuffers& b, int64_t n) {
     OXR_HIP(e.ws.reserve(b.rstate, N));
     OXR_HIP(e.ws.reserve(b.hit, 4 * N));
     int nb = oxl::compact_blocks(int64_t(N));
-    OXR_HIP(e.ws.reserve(b.counts, size_t(nb)));
+    OXR_HIP(e.ws.reserve(b.counts, size_t(oxl::compact_counts(int64_t(N)))));
     OXR_HIP(e.ws.reserve(b.offs, size_t(nb) + 1));
     OXR_HIP(e.ws.reserve(b.counters, 8));
     return OXR_OK;

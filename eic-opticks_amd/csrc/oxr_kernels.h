@@ -135,6 +135,12 @@ OXR_SIMPLE_EXTERN(48)
 // kernel simulate_persist would launch for P (-1 if the runtime cannot tell)
 int persist_occupancy(const oxd::Params& P, int block, bool fp64, bool list);
 int compact_blocks(long long n);
+// Ints that compact's counts take: one per block, and one per 256 of them from this many blocks
+// on (16.8M photons). From there the sums of 256 blocks' counts are made first (k_group): each
+// block's own sum over all before it grows with the square of the launch (us: 4096 blocks 32 both
+// ways, 8192 66 and 59, 32768 405 and 213, 195313 7870 and 1440).
+constexpr int COMPACT_GROUPED_FROM = 4096;
+int compact_counts(long long n);
 // true when P launches the production kernels (no seqhis, records, rec, prd, photonlite
 // or precooked streams)
 bool production_kernels(const oxd::Params& P);

@@ -9,7 +9,7 @@
 //                      (both in oxr_sim.h, instantiated in oxr_sim_*.hip)
 // Production variants (DBG=false) resume photons that k_generate made; the debug
 // variants (seqhis, records, precooked streams, counting) generate in place.
-//   k_count/k_select/k_scatter  ordered hit compaction (SU::count_if/copy_if, SU.cu:49-166)
+//   k_count/k_group/k_select/k_scatter_lite  ordered hit compaction (SU::count_if/copy_if, SU.cu:49-166)
 //   k_trace_rays, k_intersect_prim  geometry queries
 //   k_simtrace                      2-D cross-section rays from FRAME gensteps (CSGOptiX7.cu:536-577)
 #include "oxr_sim.h"
@@ -64,20 +64,33 @@ __global__ void __launch_bounds__(256) k_count(const uint8_t* __restrict__ flag,
     if (threadIdx.x == 0) counts[blockIdx.x] = ws[0] + ws[1] + ws[2] + ws[3];
 }
 
-// The hits in photon order. Each block sums the counts of the blocks before it (at most a few
-// thousand ints from L2) instead of waiting for a scan kernel, and notes its offset for
-// k_scatter. What the host reads after a launch - the launch counters, the hit count and the
+// Sums of the counts of 256 blocks each, for launches of many blocks.
+constexpr int GROUP = 256;
+__global__ void __launch_bounds__(GROUP) k_group(const int* __restrict__ counts, int nb, int* __restrict__ groups) {
+    const int b = blockIdx.x * GROUP + threadIdx.x;
+    const unsigned long long c = wave_sum((unsigned long long)(b < nb ? counts[b] : 0));
+    __shared__ int ws[GROUP / 64];
+    if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = int(c);
+    __syncthreads();
+    if (threadIdx.x == 0) groups[blockIdx.x] = ws[0] + ws[1] + ws[2] + ws[3];
+}
+
+// The hits in photon order. Each block sums the counts of the blocks before it (with groups,
+// of its own group's blocks and the sums of the groups before) instead of waiting for a scan
+// kernel, and notes its offset for k_scatter_lite. What the host reads after a launch - the launch counters, the hit count and the
 // first hits - is also written straight to pinned host memory (pub), so a launch ends without
 // copy commands; the counters are left zero for the next launch.
 __global__ void __launch_bounds__(256) k_select(const uint8_t* __restrict__ flag, const float4* __restrict__ photon, long long n,
-                                                const int* __restrict__ counts, long long* __restrict__ offs,
-                                                float4* __restrict__ hit, long long hit_cap, unsigned long long* ctr,
-                                                LaunchResult* pub) {
+                                                const int* __restrict__ counts, const int* __restrict__ groups,
+                                                long long* __restrict__ offs, float4* __restrict__ hit, long long hit_cap,
+                                                unsigned long long* ctr, LaunchResult* pub) {
     __shared__ unsigned long long part[4];
     __shared__ int ws[4];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     unsigned long long before = 0;
-    for (unsigned b = threadIdx.x; b < blockIdx.x; b += 256) before += (unsigned long long)counts[b];
+    const unsigned group = groups ? blockIdx.x / GROUP : 0u;
+    for (unsigned g = threadIdx.x; g < group; g += 256) before += (unsigned long long)groups[g];
+    for (unsigned b = group * GROUP + threadIdx.x; b < blockIdx.x; b += 256) before += (unsigned long long)counts[b];
     before = wave_sum(before);
     if (lane == 0) part[w] = before;
     __syncthreads();
@@ -124,11 +137,10 @@ __global__ void __launch_bounds__(256) k_select(const uint8_t* __restrict__ flag
     }
 }
 
-// the same selection of another array by the offsets k_select left; W float4 per item
-template <int W>
-__global__ void __launch_bounds__(256) k_scatter(const uint8_t* __restrict__ flag, const float4* __restrict__ photon,
-                                                 long long n, const long long* __restrict__ offs,
-                                                 float4* __restrict__ hit, long long hit_cap) {
+// the same selection of the photonlite items by the offsets k_select left
+__global__ void __launch_bounds__(256) k_scatter_lite(const uint8_t* __restrict__ flag, const uint4* __restrict__ lite,
+                                                      long long n, const long long* __restrict__ offs,
+                                                      uint4* __restrict__ hitlite, long long hit_cap) {
     __shared__ int ws[4];
     long long base = (long long)blockIdx.x * CHUNK;
     long long o = offs[blockIdx.x];
@@ -145,12 +157,7 @@ __global__ void __launch_bounds__(256) k_scatter(const uint8_t* __restrict__ fla
         int tot = ws[0] + ws[1] + ws[2] + ws[3];
         if (f) {
             long long dst = o + before + rank;
-            if (dst < hit_cap) {
-                const float4* s = photon + W * i;
-                float4* d = hit + W * dst;
-#pragma unroll
-                for (int q = 0; q < W; q++) d[q] = s[q];
-            }
+            if (dst < hit_cap) hitlite[dst] = lite[i];
         }
         o += tot;
         __syncthreads();
@@ -474,13 +481,22 @@ hipError_t order_photons(hipStream_t s, const Params& P, int key_bits, unsigned 
 }
 
 int compact_blocks(long long n) { return int((n + CHUNK - 1) / CHUNK); }
+int compact_counts(long long n) {
+    const int nb = compact_blocks(n);
+    return nb > COMPACT_GROUPED_FROM ? nb + (nb + GROUP - 1) / GROUP : nb;
+}
 
 hipError_t compact(hipStream_t s, const uint8_t* flag, const float4* photon, long long n, int* counts,
                    long long* offs, float4* hit, long long hit_cap, unsigned long long* ctr, LaunchResult* pub) {
     if (n <= 0) return hipSuccess;
     int nb = compact_blocks(n);
     hipLaunchKernelGGL(k_count, dim3(nb), dim3(256), 0, s, flag, n, counts);
-    hipLaunchKernelGGL(k_select, dim3(nb), dim3(256), 0, s, flag, photon, n, counts, offs, hit, hit_cap, ctr, pub);
+    int* groups = nullptr;
+    if (nb > COMPACT_GROUPED_FROM) {
+        groups = counts + nb;
+        hipLaunchKernelGGL(k_group, dim3(unsigned((nb + GROUP - 1) / GROUP)), dim3(GROUP), 0, s, counts, nb, groups);
+    }
+    hipLaunchKernelGGL(k_select, dim3(nb), dim3(256), 0, s, flag, photon, n, counts, groups, offs, hit, hit_cap, ctr, pub);
     return hipGetLastError();
 }
 
@@ -499,8 +515,7 @@ hipError_t scatter_lite(hipStream_t s, const uint8_t* flag, const uint4* lite, l
                         uint4* hitlite, long long hit_cap) {
     if (n <= 0) return hipSuccess;
     int nb = compact_blocks(n);
-    hipLaunchKernelGGL(k_scatter<1>, dim3(nb), dim3(256), 0, s, flag, reinterpret_cast<const float4*>(lite), n, offs,
-                       reinterpret_cast<float4*>(hitlite), hit_cap);
+    hipLaunchKernelGGL(k_scatter_lite, dim3(nb), dim3(256), 0, s, flag, lite, n, offs, hitlite, hit_cap);
     return hipGetLastError();
 }
 

@@ -29,6 +29,7 @@ constexpr size_t OFF_GSOFF = align256(OFF_GS + size_t(MAX_GENSTEP) * 96);
 constexpr size_t OFF_SEED = align256(OFF_GSOFF + size_t(MAX_GENSTEP + 1) * sizeof(long long));
 constexpr size_t OFF_RSTATE = align256(OFF_SEED + size_t(MAX_PHOTON) * sizeof(int));
 constexpr size_t OFF_FLAG = align256(OFF_RSTATE + size_t(MAX_PHOTON) * sizeof(ulonglong2));
+static_assert(MAX_BLOCKS <= oxl::COMPACT_GROUPED_FROM, "counts hold one int per block");
 constexpr size_t OFF_COUNTS = align256(OFF_FLAG + size_t(MAX_PHOTON));
 constexpr size_t OFF_OFFS = align256(OFF_COUNTS + size_t(MAX_BLOCKS) * sizeof(int));
 constexpr size_t OFF_CTR = align256(OFF_OFFS + size_t(MAX_BLOCKS + 1) * sizeof(long long));
