@@ -1,7 +1,8 @@
 // oxr_device.h -- device-side vector math, Philox RNG, tables and CSG intersection.
 //
 // Float semantics are deliberate: sources are compiled with -ffp-contract=off and
-// correctly rounded fp32 divide/sqrt, and sin/cos/atan2 are evaluated in fp64 and rounded, so every fp32 result is a function of its inputs alone.
+// correctly rounded fp32 divide/sqrt, and sin/cos/atan2 are evaluated in fp64 and rounded, so
+// every fp32 result is a function of its inputs alone.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -55,7 +56,7 @@ OXD float xlog(float x) {
 // first difference is exact: x and n hi are multiples of 2^-52 and r is below 1), then the
 // Taylor series of sin to r^15 and cos to r^16 on |r| <= pi/4, where the next terms are below
 // half an ulp. Equal to the host libm's (float)sin((double)x), (float)cos((double)x) for every
-// Philox uniform times 2 pi and over |x| <= 8e5 (checked on 2^24 arguments each). The
+// Philox uniform times 2 pi and over |x| <= 8e5 (tests/test_sincos.py). The
 // library's sin and cos reduce twice, carry the code for huge arguments and take three
 // times the instructions.
 OXD void sincos_bounded(float x, float& s, float& c) {

@@ -13,8 +13,8 @@
 
 // Minimum waves per SIMD the simulate kernels are compiled for (VGPR budget 512/N per
 // lane). 4 beat 3 and 5 on MI355X: with 5 the spilled registers cost more than the wave
-// brings (instanced CSG 11.0 against 8.5 ms), with 3 the loop waits more for memory (thin
-// shells 20.0 against 17.5 ms; with FP64 roots 3 waves are 2% faster).
+// brings, with 3 the loop waits more for memory (kernel ms with 4, 3 and 5: instanced CSG 5.95,
+// 6.73, 7.17; calorimeter 2.39, 2.93, 2.76; thin shells, 500k, 11.1, 13.7, 11.5).
 #ifndef OXR_PERSIST_WAVES
 #define OXR_PERSIST_WAVES 4
 #endif
@@ -262,21 +262,22 @@ OXD void flush_counters(const Params& P, unsigned long long steps, unsigned long
 // at the end of its trace with a bounce to compute. A turn of the loop runs one of the three
 // for the lanes that wait for it. The loop is bound by vector issue under divergence: when a
 // bounce waited for every lane's trace and a prim was tested as soon as one lane reached it,
-// 18-37% of the lanes of an issued instruction were active.
+// 18-37% of the lanes of an issued instruction were active, now 38-42%.
 //   * Nodes run while NODE_LEAST/64 of the wave's photons are at one: a visit costs a tenth to
-//     a fiftieth of a prim test or a bounce and brings lanes on to those (instanced CSG: 6 of 64
-//     7.7 ms, 3 and 12 8.0, 20 9.3). With radial bounds a visit costs a third more and is most of the
-//     time, so it wants more lanes: NODE_LEAST_RADIAL (thin shells: 6 15.9 ms, 12 15.1, 20 15.6).
+//     a fiftieth of a prim test or a bounce and brings lanes on to those. With radial bounds a
+//     visit costs a third more and is most of the time, so it wants more lanes
+//     (NODE_LEAST_RADIAL).
 //   * Prims are tested before bounces are computed unless LEAF_WEIGHT times as many lanes wait
-//     for a bounce, the dearer step. With 2 instead of 16 the instanced-CSG event takes 8.5 ms
-//     and thin shells 17.5; 32 is the same as 16; choosing by the steps' measured clocks was
-//     slower on every event but the calorimeter.
-// Kernel times on MI355X, bounce-by-bounce loop -> this one: instanced CSG (10M photons)
-// 9.5 -> 7.8 ms, thin shells (500k) 20.9 -> 16.1 ms, with FP64 roots (150k) 11.8 -> 9.5 ms,
-// pfRICH (300k) 6.5 -> 6.1 ms, calorimeter (2.07M) 2.9 -> 2.4 ms (claims by the chunk, below).
+//     for a bounce, the dearer step. Choosing by the steps' measured clocks was slower on every
+//     event but the calorimeter.
 // The plain form has no photons to refill idle lanes with, and in a small launch a wave alone on
-// its SIMD pays every turn in full: it runs each step to the last lane (calorimeter, 62k
-// photons: 696 against 780 us).
+// its SIMD pays every turn in full: it runs each step to the last lane.
+// Kernel times on MI355X with the settings of tuning_gfx950.json (ms): instanced CSG (10M
+// photons) 5.95, with NODE_LEAST 3 5.88, with 12 6.27; with LEAF_WEIGHT 2 6.52, with 32 5.95.
+// Thin shells (500k) 11.1, with NODE_LEAST_RADIAL 6 12.3, with 20 10.7. Calorimeter (2.07M) 2.39
+// whichever, 2.44 with LEAF_WEIGHT 2; plain form, 62k photons, 0.71, with the persistent form's
+// two values 0.77. The bounce-by-bounce loop took 9.5 (instanced CSG), 20.9 (thin shells) and
+// 2.9 ms (calorimeter) with its own settings.
 constexpr int NODE_LEAST = 6, NODE_LEAST_RADIAL = 12, LEAF_WEIGHT = 16;
 constexpr int NODE_LEAST_PLAIN = 1, LEAF_WEIGHT_PLAIN = 64;
 
@@ -294,8 +295,9 @@ OXD void run_wave(const Params& P, int* stk, int stride, const BNode* top) {
     TraceCount cnt = {0, 0, 0, 0};
     v.cur = TRAV_IDLE;
     bool first = true, drained = false;
-    // A photon of the wave started outside the scene (far_pad): a bounce takes it to a surface,
-    // inside, or so little beyond that the stored margins, twice the errors' bound, hold it.
+    // When the wave last took photons, one it held was outside the scene (far_pad). A bounce takes
+    // it to a surface, inside, or so little beyond that the stored margins, twice the errors'
+    // bound, hold it; looking after every bounce too spills four registers more.
     bool far_wave = false;
     unsigned long long pool = 0;   // photons the wave has claimed and not yet started: [pool, pool + pooled)
     int pooled = 0;
@@ -344,7 +346,6 @@ OXD void run_wave(const Params& P, int* stk, int stride, const BNode* top) {
         }
         const uint64_t idle = __ballot(v.cur == TRAV_IDLE);
         const int nidle = __popcll(idle);
-        if (far_wave) far_wave = __ballot(v.cur != TRAV_IDLE && far_away(g, L.p.pos)) != 0ull;
         if (drained) {
             if (nidle == 64) break;
             continue;

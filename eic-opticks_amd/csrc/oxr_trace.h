@@ -44,7 +44,6 @@ struct InstD { float4 c0, c1, c2; int4 info; };   // info: prim offset, ii_id, f
 // an instance takes part in a trace when its visibility mask shares a bit with the ray's
 // (OptixInstance::visibilityMask against optixTrace's visibilityMask, SBT.cc:538-545)
 OXD bool visible(const InstD& in, unsigned vizmask) { return ((unsigned(in.info.z) >> 8) & vizmask) != 0u; }
-struct SolidD { int primOffset, numPrim, blasRoot, pad; };
 
 struct Geom {
     const float4* node;    // two float4 per CSG node (load_node)
