@@ -28,6 +28,12 @@ void invert_instance(const float* q, double W[4][3]) {
     for (int k = 0; k < 3; k++) W[3][k] = -(t[0] * inv[0][k] + t[1] * inv[1][k] + t[2] * inv[2][k]);
 }
 
+double stretch_of(const float* q, const double inv[4][3]) {
+    double a = 0.0, b = 0.0;
+    for (int r = 0; r < 3; r++) for (int k = 0; k < 3; k++) { a += double(q[4 * r + k]) * q[4 * r + k]; b += inv[r][k] * inv[r][k]; }
+    return std::sqrt(a * b);
+}
+
 LeafBoxes::LeafBoxes(const oxr_geometry* g, double reach) : reach_(reach) {
     first_.push_back(0);
     for (int64_t p = 0; p < g->num_prim; p++) {
@@ -58,7 +64,7 @@ LeafBoxes::LeafBoxes(const oxr_geometry* g, double reach) : reach_(reach) {
     }
 }
 
-bool LeafBoxes::leaf_box(const Leaf& l, const double A[4][3], const double inv[4][3], Box& out) {
+bool LeafBoxes::leaf_box(const Leaf& l, const double A[4][3], const double inv[4][3], Box& out) const {
     double T[4][3];   // leaf to world, row convention
     double norm2 = 0.0;
     if (l.turned) {
@@ -73,16 +79,11 @@ bool LeafBoxes::leaf_box(const Leaf& l, const double A[4][3], const double inv[4
     }
     const double (*M)[3] = l.turned ? T : A;
     const double far = reach_ * std::sqrt(norm2);   // the reach in the leaf's frame
-    double all = far, col2 = 0.0;                   // all: not finite if any term is not
+    double all = far;                               // not finite if any term is not
     for (int r = 0; r < 4; r++) for (int k = 0; k < 3; k++) all += std::fabs(M[r][k]);
     if (!std::isfinite(all)) return false;
     double col[3];                                  // length of M's columns: how far a unit sphere reaches
-    for (int k = 0; k < 3; k++) {
-        const double c2 = M[0][k] * M[0][k] + M[1][k] * M[1][k] + M[2][k] * M[2][k];
-        col2 = std::max(col2, c2);
-        col[k] = std::sqrt(c2);
-    }
-    stretch_ = std::max(stretch_, std::sqrt(norm2 * col2));
+    for (int k = 0; k < 3; k++) col[k] = std::sqrt(M[0][k] * M[0][k] + M[1][k] * M[1][k] + M[2][k] * M[2][k]);
     const double flat = 16.0 * 6e-8 * far;          // planes: a few ulps of the distance
     auto map = [&](double x, double y, double z, double* w) {
         for (int k = 0; k < 3; k++) w[k] = x * M[0][k] + y * M[1][k] + z * M[2][k] + M[3][k];
@@ -120,7 +121,7 @@ bool LeafBoxes::leaf_box(const Leaf& l, const double A[4][3], const double inv[4
     return true;
 }
 
-Box LeafBoxes::placed(int64_t prim, const Box& ob, const float* inst, const double inv[4][3]) {
+Box LeafBoxes::placed(int64_t prim, const Box& ob, const float* inst, const double inv[4][3]) const {
     double A[4][3];
     for (int r = 0; r < 4; r++) for (int k = 0; k < 3; k++) A[r][k] = inst[4 * r + k];
     Box b;   // the object box's, turned

@@ -9,6 +9,9 @@ namespace oxh {
 
 // Inverse of the 4x4 transform q in double (row convention, last column taken as identity).
 void invert_instance(const float* q, double W[4][3]);
+// How much longer a distance in front of q may become behind its inverse and back: the
+// product of both norms, 3 for a rotation.
+double stretch_of(const float* q, const double inv[4][3]);
 
 // The world box of one placed prim from its leaves' own shapes, when they are all spheres,
 // zspheres, cylinders or boxes: the union of the leaves' boxes, complemented ones too, so
@@ -19,9 +22,7 @@ void invert_instance(const float* q, double W[4][3]);
 // quadric's discriminant in single precision is off by at most 16 ulps of its square, so a ray
 // may be reported to hit a sphere or cylinder up to sqrt(r^2 + 2e-6 reach^2) from its axis
 // (twice that bound), and the boxes take that radius. A ray from further away than the scene
-// is wide widens the boxes as it meets them (far_pad, oxr_trace.h): stretch() is the most that
-// a distance in the world grows by on its way into a leaf's frame and its margin back, the
-// longest column of the leaf's transform times the norm of its inverse.
+// is wide widens the boxes as it meets them (far_pad, oxr_trace.h).
 // Instanced CSG, 10M photons: 7.7 -> 6.1 ms; 200k photons 540 -> 466 us; the served stream of 24
 // events 9.5 -> 7.9 ms.
 //
@@ -31,8 +32,7 @@ public:
     LeafBoxes(const oxr_geometry* g, double reach);
     // Prim's object box ob placed by inst (object to world; inv its inverse), cut to its leaves'
     // boxes where their shapes are known.
-    Box placed(int64_t prim, const Box& ob, const float* inst, const double inv[4][3]);
-    double stretch() const { return stretch_; }
+    Box placed(int64_t prim, const Box& ob, const float* inst, const double inv[4][3]) const;
 private:
     struct Leaf {
         uint32_t type;
@@ -42,8 +42,8 @@ private:
         double x, y, z, r;       // centre and radius, or full sides in x, y, z
         double z1, z2;
     };
-    bool leaf_box(const Leaf& l, const double A[4][3], const double inv[4][3], Box& out);
-    double reach_, stretch_ = 1.0;
+    bool leaf_box(const Leaf& l, const double A[4][3], const double inv[4][3], Box& out) const;
+    double reach_;
     std::vector<Leaf> leaves_;
     std::vector<int64_t> first_;   // of each prim in leaves_, and the end; none: shapes not known
 };

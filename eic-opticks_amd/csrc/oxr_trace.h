@@ -58,7 +58,7 @@ struct Geom {
     unsigned vizmask;      // ray visibility mask against InstD flag bits 8-15
     // radial bounds, two float4 per node of tlas {centre, (r_in0, r_out0, r_in1, r_out1)}
     const float4* rad;
-    // far_pad's: half the reach that the world boxes hold, and the pad per distance beyond it
+    // far_pad's: the longest distance of a point of the scene from its origin, and the pad per distance
     float far_extent, far_scale;
 };
 
@@ -80,16 +80,19 @@ OXD f3 safe_inv(f3 d) {
               __builtin_amdgcn_rcpf(fabsf(d.z) > e ? d.z : copysignf(e, d.z)));
 }
 OXD f3 neg_oi(f3 o, f3 inv) { return mk(-(o.x * inv.x), -(o.y * inv.y), -(o.z * inv.z)); }
-// The world boxes of quadrics hold what their single-precision tests may report from origins
-// within the scene (oxr_boxes.h). The error of a test grows with the origin's
-// distance D: from outside, a box has to reach sqrt(2e-6 (D^2 - reach^2)) further, times the
-// worst stretch of a leaf's transform, than the margin it was stored with. Nothing is added
-// for an origin within the scene.
+// A box holds what the single-precision tests of its prims may report from origins within the
+// scene (oxr_boxes.h). The error of a test grows with the origin's distance D: for a ray from
+// outside, a box has to reach sqrt(2e-6) D further, times the worst stretch of a leaf's
+// transform. far_scale holds both; nothing is added for an origin within the scene. In the
+// frame of an instance the pad is as much longer as its transform may stretch it (in_frame).
 OXD bool far_away(const Geom& g, f3 pos) { return dot(pos, pos) > g.far_extent * g.far_extent; }
 OXD float far_pad(const Geom& g, f3 pos) {
-    const float dist = __builtin_amdgcn_sqrtf(dot(pos, pos)) + g.far_extent;
-    const float over = fmaf(dist, dist, -4.f * g.far_extent * g.far_extent);
-    return over > 0.f ? g.far_scale * __builtin_amdgcn_sqrtf(over) : 0.f;
+    return far_away(g, pos) ? g.far_scale * (__builtin_amdgcn_sqrtf(dot(pos, pos)) + g.far_extent) : 0.f;
+}
+OXD float in_frame(const InstD& in, float pad) {
+    const float n2 = in.c0.x * in.c0.x + in.c0.y * in.c0.y + in.c0.z * in.c0.z + in.c1.x * in.c1.x + in.c1.y * in.c1.y +
+                     in.c1.z * in.c1.z + in.c2.x * in.c2.x + in.c2.y * in.c2.y + in.c2.z * in.c2.z;
+    return 1.7321f * pad * __builtin_amdgcn_sqrtf(n2);
 }
 // slab test of one child box (noi_lo, noi_hi: -origin*inv for its low and high planes, which
 // differ by what the box is widened by)
@@ -171,7 +174,7 @@ OXD void trav_begin(Trav& v, const Geom& g, float tmax, int* stk, int stride, in
 }
 
 // the ray in the frame of the current tree, and what the slab tests need of it
-// WIDE: the world boxes are widened for origins outside the scene (far_pad); the high planes
+// WIDE: the boxes are widened for origins outside the scene (far_pad); the high planes
 // then have their own product, and a radial bound lies off, sqrt(3) of the pad, nearer
 template <bool WIDE> struct RayF {
     f3 o, inv, noi;
@@ -201,12 +204,16 @@ OXD void ray_frame(RayF<WIDE>& r, f3 o, f3 d, float pad) {
 }
 template <bool RADIAL, bool WIDE>
 OXD void ray_world(RayF<WIDE>& r, const Geom& g, f3 pos, f3 mom) { ray_frame<RADIAL>(r, pos, mom, WIDE ? far_pad(g, pos) : 0.f); }
+template <bool RADIAL, bool WIDE>
+OXD void ray_inst(RayF<WIDE>& r, const Geom& g, const InstD& in, f3 pos, f3 mom) {
+    f3 o, d;
+    to_object(in, pos, mom, o, d);
+    ray_frame<RADIAL>(r, o, d, WIDE ? in_frame(in, far_pad(g, pos)) : 0.f);
+}
 template <bool FLAT, bool RADIAL, bool WIDE>
 OXD void ray_of(RayF<WIDE>& r, const Geom& g, const Trav& v, f3 pos, f3 mom) {
-    f3 o = pos, d = mom;
-    const bool world = FLAT || v.inst < 0 || (v.inst & INST_IDENT) != 0;
-    if (!world) to_object(g.inst[v.inst], pos, mom, o, d);
-    ray_frame<RADIAL>(r, o, d, WIDE && world ? far_pad(g, pos) : 0.f);
+    if (FLAT || v.inst < 0 || (v.inst & INST_IDENT)) ray_world<RADIAL>(r, g, pos, mom);
+    else ray_inst<RADIAL>(r, g, g.inst[v.inst], pos, mom);
 }
 
 // the next stack entry worth visiting; the first one is the end mark
@@ -282,11 +289,7 @@ OXD void trav_node(Trav& v, const Geom& g, RayF<WIDE>& r, f3 pos, f3 mom, int* s
         }
         const bool ident = (in.info.z & 1) != 0;
         v.inst = item | (ident ? INST_IDENT : 0);
-        if (!ident) {
-            f3 o, d;
-            to_object(in, pos, mom, o, d);
-            ray_frame<RADIAL>(r, o, d, 0.f);
-        }
+        if (!ident) ray_inst<RADIAL>(r, g, in, pos, mom);
         if (v.sp < stride * cap) {
             stk[v.sp] = int(TRAV_BACK);
             if (TN) stkt[v.sp] = -INFINITY;

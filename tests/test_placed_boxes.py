@@ -138,7 +138,6 @@ static int contain(unsigned seed, bool other) {
             if (other && (b.lo[k] > turned.lo[k] + 1e-6 || b.hi[k] < turned.hi[k] - 1e-6)) return 2;
         }
         if (other) continue;
-        if (boxes.stretch() < 1.0) return 3;
         for (size_t n = tree ? 3 : 0; n < geo.node.size() / 16; n++) {
             const float* q = &geo.node[16 * n];
             uint32_t type;
