@@ -339,7 +339,7 @@ OXD void run_wave(const Params& P, int* stk, int stride, const BNode* top) {
                     trav_begin(v, g, P.tmax, stk, stride, P.stack_cap, TN);
                 } else {
                     end_photon<DBG>(P, L);
-                    add_steps(steps, L.bounce, [&](uint32_t n) { atomicAdd(P.counters + 0, (unsigned long long)n); });
+                    add_steps(steps, L.bounce, [&](uint32_t n) __attribute__((always_inline)) { atomicAdd(P.counters + 0, (unsigned long long)n); });
                     v.cur = TRAV_IDLE;
                 }
             }

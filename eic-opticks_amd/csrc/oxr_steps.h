@@ -9,7 +9,7 @@ namespace oxd {
 // once they reach 2^31. A photon's own steps are below 2^31, so the sum never wraps.
 // (constexpr: for the host and the device)
 template <class Hand>
-constexpr void add_steps(uint32_t& steps, int bounces, Hand hand) {
+__attribute__((always_inline)) constexpr void add_steps(uint32_t& steps, int bounces, Hand hand) {
     steps += uint32_t(bounces);
     if (steps >> 31) {
         hand(steps);
